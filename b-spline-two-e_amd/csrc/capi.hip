@@ -425,7 +425,7 @@ static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
     HIP_TRY(ctx, hipStreamWaitEvent(s, rk->windows, 0));
     if (!rk->from_primitives) HIP_TRY(ctx, launch_diag_cells(rk->plan, rk->d, s, true));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], s));
-    HIP_TRY(ctx, launch_tensor_near(rk->plan, rk->d, rk->R, s));
+    HIP_TRY(ctx, launch_tensor_near(rk->plan, rk->d, rk->R, !rk->from_primitives, s));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[4], s));
     HIP_TRY(ctx, hipEventRecord(rk->join, s));
     HIP_TRY(ctx, launch_tensor_far(rk->plan, rk->d, rk->R, m));

@@ -139,7 +139,7 @@ int64_t bs2e_rk_build_static(int64_t k, int64_t n_knots, const double* knots, in
         e = precision == BS2E_PREC_MIXED ? launch_outer_moments_mixed(p, d, s) : launch_outer_moments(p, d, s);
     if (e == hipSuccess) e = launch_pair_windows(p, d, s);
     if (e == hipSuccess) e = launch_diag_cells(p, d, s, true);
-    if (e == hipSuccess) e = launch_tensor_near(p, d, R, s);
+    if (e == hipSuccess) e = launch_tensor_near(p, d, R, true, s);
     if (e == hipSuccess) e = launch_tensor_far(p, d, R, s);
     if (e != hipSuccess)
         return fail(nullptr, BS2E_EDEVICE, std::string("bs2e_rk_build_static: ") + hipGetErrorString(e));

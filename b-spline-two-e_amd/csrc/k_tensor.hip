@@ -18,9 +18,10 @@
 //     windows do not overlap), streamed with non-temporal stores.  Bound by
 //     the FP64 store of R: 8 bytes per integral.
 //   * k3_near: the elements whose pairs share a support interval (a few
-//     percent of each row).  Rows p = (a,c) and (c,a) are identical
-//     (R(a,b,c,d) = R(c,b,a,d)), so one workgroup evaluates row (a,c), a <= c,
-//     and stores it into both rows.  With W_p = [lo, hi], for column q:
+//     percent of each row).  R(a,b,c,d) = R(c,b,a,d) = R(a,d,c,b) = R(b,a,d,c),
+//     so one workgroup per row (a,c), a <= c, evaluates its columns (b,d),
+//     b <= d, that are not before the row and stores each value into all the
+//     equal elements.  With W_p = [lo, hi], for column q:
 //       R = Qtot_p * sum_{w in W_q, w < lo} P_q(w)
 //         + Ptot_p * sum_{w in W_q, w > hi} Q_q(w)
 //         + sum_{w in W_p and W_q} Q_q(w) PP_p(w-1) + P_q(w) QS_p(w+1) + Dsym[w; p, q]
@@ -34,15 +35,20 @@ namespace bs2e {
 
 constexpr int kThreads = 256;
 
+// Rounded-up 32-bit reciprocal of n (0 for n = 1): the upper half of its
+// product with x is x / n exactly for x < 2^32 / n.
+static unsigned recip32(int64_t n) { return n > 1 ? (unsigned)((((uint64_t)1 << 32) + n - 1) / n) : 0; }
+
 // LDS of a near workgroup (row p, window length m):
 //   PPx[i][k], i in [0, m]: 0, PP[0], ..., PP[m-1] (= Ptot)
 //   QSx[i][k], i in [0, m]: QS[0] (= Qtot), ..., QS[m-1], 0
 // so that PP_p(w-1) = PPx[w - lo] and QS_p(w+1) = QSx[w - lo + 1] for w in
-// W_p; the local pair index of p on each interval of W_p; and the row's
-// column segments (one run of consecutive pairs per column spline d).
+// W_p; the local pair index of p on each interval of W_p; the column pairs'
+// runs, one per column spline d, and the column pairs themselves.
 size_t near_lds_bytes(int64_t ks, int64_t K)
 {
-    return sizeof(double) * (size_t)(2 * (ks + 1) * K) + sizeof(int) * (size_t)(kMaxOrder + 2 * kNearMaxSeg + 4);
+    return sizeof(double) * (size_t)(2 * (ks + 1) * K + 2 * (2 * ks - 1) * (2 * ks - 1)) +
+           sizeof(int) * (size_t)(kMaxOrder + 2 * kNearMaxSeg + 4);
 }
 
 __device__ __forceinline__ int pair_at(const int32_t* __restrict__ c_first, int ks, int a, int c)
@@ -51,7 +57,20 @@ __device__ __forceinline__ int pair_at(const int32_t* __restrict__ c_first, int 
     return c_first[c] + (a - lo);
 }
 
-__global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int K, int ks, int U,
+// FOLD: only pairs p = (a, c), a <= c, and q = (b, d), b <= d, q not before p,
+// are evaluated and stored in the up to eight elements that the symmetries of
+// the integral make equal (a <-> c, b <-> d, and the two electrons), so that
+// every diagonal cell is read once; without it (moments from the caller's own
+// containers, which need not be symmetric in a pair's splines) every column of
+// the row, stored into rows (a, c) and (c, a).
+//
+// Bound by the latency of its gathers and the scattered stores of K
+// consecutive multipoles (8 K bytes): one thread per element, the column
+// pairs' indices found once per pair in LDS rather than once per element.
+// Alone, FOLD against every column with a search per element: 2944 pairs x 11
+// multipoles 0.038 -> 0.019 ms, 10128 x 25 0.284 -> 0.181 ms.
+template <bool FOLD>
+__global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int n_iv, int K, int ks, int U, unsigned rK,
                                                     const PairInfo* __restrict__ pairs,
                                                     const int32_t* __restrict__ c_first,
                                                     const int32_t* __restrict__ rows,
@@ -59,20 +78,21 @@ __global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int K,
                                                     const double* __restrict__ PP, const double* __restrict__ QS,
                                                     const double* __restrict__ Dsym, double* __restrict__ R)
 {
-    extern __shared__ double lds[];
-    double* sPPx = lds;                                    // [(ks+1)][K]
-    double* sQSx = lds + (ks + 1) * K;                     // [(ks+1)][K]
-    int* sUp = (int*)(lds + 2 * (ks + 1) * K);             // [kMaxOrder]
-    int* sQ0 = sUp + kMaxOrder;                            // [kNearMaxSeg]: first pair of each segment
-    int* sJ0 = sQ0 + kNearMaxSeg;                          // [kNearMaxSeg + 1]: segment starts in row order
-    int* sNseg = sJ0 + kNearMaxSeg + 1;
+    constexpr int kLanes = kNearMaxSeg;                    // one wavefront scans the runs
+    extern __shared__ __align__(16) double lds[];
+    int4* sCol = (int4*)lds;                               // [(2 ks - 1)^2]: q, (d, b)'s pair or -1, min, max of b, d
+    double* sPPx = lds + 2 * (2 * ks - 1) * (2 * ks - 1);  // [(ks+1)][K]
+    double* sQSx = sPPx + (ks + 1) * K;                    // [(ks+1)][K]
+    int* sUp = (int*)(sQSx + (ks + 1) * K);                // [kMaxOrder]
+    int* sJ0 = sUp + kMaxOrder;                            // [kNearMaxSeg + 1]: first column pair of each spline d
+    int* sB0 = sJ0 + kNearMaxSeg + 1;                      // [kNearMaxSeg]: its first b
     const int tid = threadIdx.x;
     const int p = rows[xcd_block(blockIdx.x, gridDim.x)];   // neighbouring rows gather the same Dsym cells
     const PairInfo pp = pairs[p];
     const int lo = pp.v0, m = pp.m, hi = pp.v0 + pp.m - 1;
     const int pt = (pp.a == pp.c) ? -1 : pair_at(c_first, ks, pp.c, pp.a);   // the identical row (c, a)
     for (int e = tid; e < (ks + 1) * K; e += kThreads) {
-        const int i = e / K, k = e - i * K;
+        const int i = rK ? (int)__umulhi((unsigned)e, rK) : e, k = e - i * K;   // (e < 2^26 / K: an exact quotient)
         const size_t pb = (size_t)p * ks * K + k;
         sPPx[e] = (i == 0) ? 0.0 : PP[pb + (size_t)(i - 1) * K];
         sQSx[e] = (i >= m) ? 0.0 : QS[pb + (size_t)i * K];
@@ -81,56 +101,83 @@ __global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int K,
         const int vz = lo - 1 + tid;
         sUp[tid] = sym_local(pp.a - vz, pp.c - vz, ks);
     }
-    if (tid == 0) {
-        // column pairs (b, d) share an interval with W_p iff
-        // max(b,d) + 2 - k <= hi and min(b,d) + 1 >= lo
-        const int dlo = max(1, lo - 1), dhi = min(n_b, hi + ks - 2);
-        int ns = 0, J = 0;
-        for (int d = dlo; d <= dhi; ++d) {
-            const int b0 = max(1, d - ks + 1);
-            const int blo = max(b0, lo - 1), bhi = min(min(d + ks - 1, n_b), hi + ks - 2);
-            if (blo > bhi) continue;
-            sQ0[ns] = c_first[d] + (blo - b0);
-            sJ0[ns] = J;
-            J += bhi - blo + 1;
-            ++ns;
+    // column pairs (b, d) share an interval with W_p iff max(b,d) + 2 - k <= hi
+    // and min(b,d) + 1 >= lo: one run of b per d
+    const int dlo = max(1, lo - 1), dhi = min(n_b, hi + ks - 2);   // dhi - dlo + 1 <= 2k - 1 <= 39
+    if (tid < kLanes) {
+        const int d = dlo + tid;
+        int b0 = max(max(1, d - ks + 1), lo - 1);
+        int b1 = FOLD ? d : min(min(d + ks - 1, n_b), hi + ks - 2);
+        if (FOLD && d == pp.c) b0 = max(b0, pp.a);         // (pairs are ordered by d, then b)
+        const int len = d > dhi || (FOLD && d < pp.c) ? 0 : max(0, b1 - b0 + 1);
+        int inc = len;
+        for (int off = 1; off < kLanes; off <<= 1) {
+            const int y = __shfl_up(inc, off, kLanes);
+            if (tid >= off) inc += y;
         }
-        sJ0[ns] = J;
-        *sNseg = ns;
+        sJ0[tid] = inc - len;
+        sB0[tid] = b0;
+        if (tid == kLanes - 1) sJ0[kLanes] = inc;
     }
     __syncthreads();
-    const int ns = *sNseg;
-    const int total = sJ0[ns] * K;
+    const int ncol = sJ0[kLanes];
+    for (int j = tid; j < ncol; j += kThreads) {
+        int s = 0;                       // the last run starting at or before j is the one that holds it
+        for (int step = kLanes / 2; step > 0; step >>= 1)
+            if (sJ0[s + step] <= j) s += step;
+        const int d = dlo + s, b = sB0[s] + (j - sJ0[s]);
+        sCol[j] = int4{pair_at(c_first, ks, b, d), FOLD && b != d ? pair_at(c_first, ks, d, b) : -1, min(b, d), max(b, d)};
+    }
+    __syncthreads();
+    const int total = ncol * K;
     const int64_t rowlen = (int64_t)n_pairs * K;
     double* Rp = R + (size_t)p * rowlen;
     double* Rt = R + (size_t)(pt < 0 ? p : pt) * rowlen;
     const unsigned UK = (unsigned)(U * K);   // Dsym has n_iv*U*U*K < 2^31 entries (checked on the host)
     for (int e = tid; e < total; e += kThreads) {
-        const int j = e / K, k = e - j * K;
-        int s = 0;                       // last segment starting at or before j
-        for (int step = kNearMaxSeg / 2; step > 0; step >>= 1)
-            if (s + step < ns && sJ0[s + step] <= j) s += step;
-        const int q = sQ0[s] + (j - sJ0[s]);
-        const PairInfo pq = pairs[q];
-        const int v0q = pq.v0, endq = pq.v0 + pq.m - 1;
+        const int j = rK ? (int)__umulhi((unsigned)e, rK) : e, k = e - j * K;
+        const int4 col = sCol[j];
+        const int q = col.x, qt = col.y, bl = col.z, bh = col.w;
+        const int v0q = max(1, bh + 2 - ks), endq = min(bl + 1, n_iv);   // q's window
         const size_t qb = (size_t)q * ks * K + k;
         double val = 0.0;
         if (v0q < lo) val = sQSx[k] * PP[qb + (size_t)(lo - 1 - v0q) * K];
         if (endq > hi) val += sPPx[m * K + k] * QS[qb + (size_t)(hi + 1 - v0q) * K];
         const int wlo = max(lo, v0q), whi = min(hi, endq);
         double acc = 0.0, dacc = 0.0;
+        const double* qw = Qw + qb + (size_t)(wlo - v0q) * K;
+        const double* pw = Pw + qb + (size_t)(wlo - v0q) * K;
+        const double* sp = sPPx + (wlo - lo) * K + k;
+        const double* sq = sQSx + (wlo - lo + 1) * K + k;
+        int t = bl - (wlo - 1);                              // q's lower local spline on interval w
+        unsigned Dv = (unsigned)(wlo - 1) * U * UK + (unsigned)k;
 #pragma unroll 2
         for (int w = wlo; w <= whi; ++w) {
-            const int jq = w - v0q, jp = w - lo, vz = w - 1;
-            acc += Qw[qb + (size_t)jq * K] * sPPx[jp * K + k] + Pw[qb + (size_t)jq * K] * sQSx[(jp + 1) * K + k];
-            const unsigned uq = (unsigned)sym_local(pq.a - vz, pq.c - vz, ks), up = (unsigned)sUp[jp];
-            const unsigned ulo = up < uq ? up : uq, uhi = up < uq ? uq : up;   // Dsym is read in its upper triangle
-            dacc += Dsym[(unsigned)vz * U * UK + ulo * UK + uhi * (unsigned)K + (unsigned)k];
+            const unsigned uq = (unsigned)(t * ks - ((t * (t - 1)) >> 1) + (bh - bl)), up = (unsigned)sUp[w - lo];
+            const unsigned ulo = min(up, uq), uhi = max(up, uq);   // Dsym is read in its upper triangle
+            dacc += Dsym[Dv + ulo * UK + uhi * (unsigned)K];
+            acc += *qw * *sp + *pw * *sq;
+            qw += K, pw += K, sp += K, sq += K, --t, Dv += U * UK;
         }
         val += acc + dacc;
-        const size_t o = (size_t)q * K + k;
+        const size_t o = (size_t)q * K + k, ot = (size_t)qt * K + k;
         Rp[o] = val;
         if (pt >= 0) Rt[o] = val;
+        if (FOLD) {
+            const size_t op = (size_t)p * K + k, opt = (size_t)pt * K + k;
+            double* const Rq = R + (size_t)q * rowlen;
+            if (qt >= 0) Rp[ot] = val;
+            if (qt >= 0 && pt >= 0) Rt[ot] = val;
+            if (q != p) {
+                Rq[op] = val;
+                if (pt >= 0) Rq[opt] = val;
+                if (qt >= 0) {
+                    double* const Rqt = R + (size_t)qt * rowlen;
+                    Rqt[op] = val;
+                    if (pt >= 0) Rqt[opt] = val;
+                }
+            }
+        }
     }
 }
 
@@ -282,12 +329,13 @@ int64_t count_near_elements(const Plan& p)
     return n;
 }
 
-hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, hipStream_t s)
+hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s)
 {
     if (p.rows.empty()) return hipSuccess;
-    hipLaunchKernelGGL(k3_near, dim3((unsigned)p.rows.size()), dim3(kThreads), near_lds_bytes(p.k_s, p.K), s,
-                       (int)p.n_pairs, (int)p.n_b, (int)p.K, (int)p.k_s, (int)p.U, d.pairs, d.c_first, d.rows, d.Pw,
-                       d.Qw, d.PP, d.QS, d.D, R);
+    const auto kern = symmetric ? k3_near<true> : k3_near<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.rows.size()), dim3(kThreads), near_lds_bytes(p.k_s, p.K), s,
+                       (int)p.n_pairs, (int)p.n_b, (int)p.n_iv, (int)p.K, (int)p.k_s, (int)p.U, recip32(p.K), d.pairs,
+                       d.c_first, d.rows, d.Pw, d.Qw, d.PP, d.QS, d.D, R);
     return hipGetLastError();
 }
 
