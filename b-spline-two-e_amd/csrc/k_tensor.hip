@@ -14,7 +14,7 @@
 // Dsym[v] = D[v] + D[v]^T the symmetrised diagonal cell.
 //
 // Two kernels write disjoint elements, each element exactly once:
-//   * k3_far : a few rows x one column chunk of rank-one products (the pairs'
+//   * k3_far : two rows x one column chunk of rank-one products (the pairs'
 //     windows do not overlap), streamed with non-temporal stores.  Bound by
 //     the FP64 store of R: 8 bytes per integral.
 //   * k3_near: the elements whose pairs share a support interval (a few
@@ -29,6 +29,8 @@
 //     QS_p = Qtot_p left of W_p and 0 right of it); the first two sums are
 //     q's own prefix / suffix sums.  It runs on a second stream, concurrently
 //     with k3_far.
+#include <algorithm>
+
 #include "bs2e_internal.h"
 
 namespace bs2e {
@@ -181,81 +183,159 @@ __global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int n_
     }
 }
 
-// Far workgroups: ROWS rows x one column chunk of rank-one products; the
-// elements whose pairs' windows overlap are left to k3_near.  V = 2: each
-// thread stores two consecutive elements with one 16-byte store (rows of even
-// length, so every row start is 16-byte aligned); V = 1: one element.
+// Far workgroups: ROWS rows x one chunk of 512 ITERS elements of rank-one
+// products, two consecutive elements per thread and 16-byte store; the
+// elements whose pairs' windows overlap are left to k3_near.
+//
+// Bound by the store of R (8 bytes per element).  What the store rate depends
+// on, measured with stores alone over 20.5 GB: one 16-byte store per thread
+// and row reaches 6.5-6.9 TB/s, two or four 5.5-6.5, so a workgroup takes few
+// elements and lives short; and its latency has to stay short too.  Therefore
+//   * no element looks at its pair: pairs are numbered column spline by
+//     column spline, so the chunks right of every window of the workgroup's
+//     rows, and those left of it, are told apart once per workgroup by their
+//     element range, and such a chunk reads one factor table, its multipole
+//     index from the offset in the chunk by a 32-bit multiplication with the
+//     reciprocal of K; only the chunks near the rows' own columns (about
+//     4 (2k - 1)^2 K of a row's n_pairs K elements) test every element;
+//   * SHIFT: where the rows do not start on 128-byte lines (n_pairs K not a
+//     multiple of 16) each row's chunks are shifted to begin on one (by up to
+//     15 elements, into the chunk before), so that no line is written in
+//     parts by two workgroups, which sit on different XCDs; the odd rows of an
+//     odd row length take the same 16-byte stores;
+//   * on the border single elements are stored without the non-temporal hint,
+//     so that the parts of a line meet in L2 (0.143 -> 0.119 ms at 2944 pairs
+//     x 11 multipoles; elsewhere plain stores cost 40 %).
+// x_cols > 0: XCD x takes the x-th eighth of a row's chunks (x_cols of them)
+// row group by row group, so that its L2 keeps that slice of the factors;
+// otherwise the workgroups follow the rows.  The slices pay where the two
+// factor tables take more than half of an XCD's 4 MB L2: whole builds of
+// 10128 x 25 (4.1 MB) 3.27 ms in slices against 3.50 along the rows, of order
+// 9 with 2.8 MB 2.29 against 2.36 and with 2.3 MB 1.50 against 1.64; of
+// 6728 x 17 (1.8 MB) 1.085 against 1.042, 4444 x 17 (1.2 MB) 0.487 against
+// 0.464.
+// k3_far alone, 2 rows x 512 elements, against a test per element and 8-byte
+// stores for odd lengths: 2944 x 11 (lines) 0.145 -> 0.119 ms; 4444 x 17
+// (shifted) 0.519 -> 0.388; 3349 x 9 (odd) 0.257 -> 0.111; 10128 x 25 (lines)
+// 3.18-3.60 -> 3.09.
 typedef double double2_t __attribute__((ext_vector_type(2)));
+typedef double double2u_t __attribute__((ext_vector_type(2), aligned(8)));   // a pair on any element boundary
 
-template <int V, int ROWS, int ITERS>
-__global__ __launch_bounds__(kThreads) void k3_far(int n_pairs, int K, int far_cols, int x_cols,
-                                                   const PairInfo* __restrict__ pairs,
+constexpr int kFarLine = 16;            // elements per 128-byte line
+constexpr int kFarLd = kMaxK + 2;       // a row's factors in LDS, the first one again behind the last
+constexpr unsigned kFarGridY = 32768;   // row groups per grid layer
+constexpr int64_t kFarSliceBytes = (int64_t)2 << 20;   // factor tables beyond which the XCDs take slices
+
+template <int ROWS, int ITERS, bool SHIFT>
+__global__ __launch_bounds__(kThreads) void k3_far(int n_pairs, int n_b, int K, int ks, unsigned rK, unsigned rK1,
+                                                   int far_cols, int x_cols, const PairInfo* __restrict__ pairs,
+                                                   const int32_t* __restrict__ c_first,
                                                    const double* __restrict__ Ptot,
                                                    const double* __restrict__ Qtot, double* __restrict__ R)
 {
-    __shared__ double sA[ROWS * kMaxK];   // Ptot of the rows
-    __shared__ double sB[ROWS * kMaxK];   // Qtot of the rows
-    __shared__ int sLo[ROWS], sHi[ROWS];
-    const int64_t rowlen = (int64_t)n_pairs * K;
+    constexpr int CH = 2 * kThreads * ITERS, NF = SHIFT ? ROWS : 1;
+    __shared__ double sP[ROWS * kFarLd], sQ[ROWS * kFarLd];   // Ptot, Qtot of the rows
     const int tid = threadIdx.x;
-    // XCD x owns the x-th eighth of the column chunks (x_cols of them) and
-    // walks it row group by row group: its L2 keeps that slice of the column
-    // factors while the stores stream past, and the XCDs' stores in flight
-    // spread over eight regions of a row.  Measured in one process against
-    // the row-major order and against chunks x, x + 8, ... per XCD: c5p
-    // 3.45-3.48 ms per build against 3.71-3.76 (k3_far<2,2,2>), c2, c3, c4
-    // within 2 %.
-    const int x = (int)(blockIdx.x % kXcds), j = (int)(blockIdx.x / kXcds);
-    const int ry = j / x_cols, cx = x * x_cols + (j - ry * x_cols);
-    if (cx >= far_cols) return;   // (the last XCD's slice can be short; uniform over the workgroup)
-    const int p0 = ry * ROWS;
+    const int rowlen = n_pairs * K;        // < 2^31 (checked on the host)
+    const int p0 = (int)(blockIdx.z * kFarGridY + blockIdx.y) * ROWS;
+    if (p0 >= n_pairs) return;             // (the last grid layer can be short)
     const int nrows = (n_pairs - p0) < ROWS ? (n_pairs - p0) : ROWS;
-    for (int e = tid; e < nrows * K; e += kThreads) {
-        const int r = e / K, k = e - r * K;
-        sA[r * kMaxK + k] = Ptot[(size_t)(p0 + r) * K + k];
-        sB[r * kMaxK + k] = Qtot[(size_t)(p0 + r) * K + k];
+    const int cx = x_cols ? (int)(blockIdx.x % kXcds) * x_cols + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
+    if (cx >= far_cols) return;            // (the last XCD's slice can be short)
+    const int e0 = cx * CH;
+    const unsigned uK = (unsigned)K;
+    int lo[ROWS], hi[ROWS], shift[ROWS];   // uniform: scalar registers
+    int lo_min = 0x7fffffff, hi_max = 0;
+    double* const Rrow = R + (size_t)p0 * (size_t)rowlen;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const PairInfo pi = pairs[p0 + (r < nrows ? r : 0)];
+        lo[r] = pi.v0;
+        hi[r] = pi.v0 + pi.m - 1;          // last interval of the row's window
+        lo_min = lo[r] < lo_min ? lo[r] : lo_min;
+        hi_max = hi[r] > hi_max ? hi[r] : hi_max;
+        shift[r] = SHIFT ? (int)((uintptr_t)(Rrow + (size_t)r * rowlen) / sizeof(double)) & (kFarLine - 1) : 0;
     }
-    if (tid < nrows) {
-        const PairInfo pi = pairs[p0 + tid];
-        sLo[tid] = pi.v0;
-        sHi[tid] = pi.v0 + pi.m - 1;   // last interval of the row's window
+    // a pair of column c has its window within [c + 2 - k, c + 1]: left of the
+    // rows' windows for c <= lo_min - 2, right of them for c >= hi_max + k - 1
+    const int cl = lo_min - 1 > 1 ? lo_min - 1 : 1, cr = hi_max + ks - 1 < n_b + 1 ? hi_max + ks - 1 : n_b + 1;
+    const int e_left = c_first[cl] * K, e_right = c_first[cr] * K;
+    const bool left = e0 + CH <= e_left, right = e0 - (SHIFT ? kFarLine - 1 : 0) >= e_right;
+    // the chunk's first element is element kb - 16 K of pair qb: an element at
+    // offset o + 16 K from there has pair qb - 16 + o / K and multipole o % K
+    // (rK: the rounded-up reciprocal, 0 for K = 1; its quotient is exact for
+    // o < 2^14, and at most one too large for e0)
+    int qb = rK ? (int)__umulhi((unsigned)e0, rK) : e0;
+    if (qb * K > e0) --qb;
+    const unsigned kb = (unsigned)(e0 - qb * K) + kFarLine * uK;
+    if ((left || right) && nrows == ROWS && e0 + CH <= rowlen && (!SHIFT || e0 > 0)) {
+        // the columns' factors, and the rows' (Ptot of whichever lies left)
+        const double* __restrict__ F = (left ? Ptot : Qtot) + e0;
+        const double* __restrict__ G = (left ? Qtot : Ptot) + (size_t)p0 * K;
+        double2u_t f[NF][ITERS];
+#pragma unroll
+        for (int r = 0; r < NF; ++r)
+#pragma unroll
+            for (int i = 0; i < ITERS; ++i) f[r][i] = *(const double2u_t*)(F - shift[r] + 2 * (i * kThreads + tid));
+        for (int e = tid; e < ROWS * (K + 1); e += kThreads) {
+            const int r = (int)__umulhi((unsigned)e, rK1), k = e - r * (K + 1);
+            sP[r * kFarLd + k] = G[r * K + (k < K ? k : 0)];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITERS; ++i)
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const unsigned o = 2 * (i * kThreads + tid) - shift[r];
+                const unsigned a = kb + o, k = rK ? a - uK * __umulhi(a, rK) : 0;
+                const double* g = sP + r * kFarLd + k;
+                const double2u_t v = f[SHIFT ? r : 0][i];
+                __builtin_nontemporal_store(double2u_t{g[0] * v.x, g[1] * v.y},
+                                            (double2u_t*)(Rrow + (size_t)r * rowlen + e0 + (int)o));
+            }
+        return;
+    }
+    for (int e = tid; e < nrows * (K + 1); e += kThreads) {
+        const int r = (int)__umulhi((unsigned)e, rK1), k = e - r * (K + 1);
+        const size_t g = (size_t)(p0 + r) * K + (k < K ? k : 0);
+        sP[r * kFarLd + k] = Ptot[g];
+        sQ[r * kFarLd + k] = Qtot[g];
     }
     __syncthreads();
-    double* Rrow = R + (size_t)p0 * rowlen;
-    const unsigned uK = (unsigned)K, urow = (unsigned)rowlen;   // rowlen = n_pairs * K < 2^31 (checked on the host)
+#pragma unroll
     for (int i = 0; i < ITERS; ++i) {
-        const unsigned e = (unsigned)V * ((unsigned)cx * kThreads * ITERS + (unsigned)i * kThreads + (unsigned)tid);
-        if (e >= urow) break;
-        const int q0 = (int)(e / uK), k0 = (int)(e - (unsigned)q0 * uK);
-        const PairInfo a0 = pairs[q0];
-        const int v1a = a0.v0 + a0.m - 1;
-        if (V == 1) {
-            const double pt = Ptot[e], qt = Qtot[e];
-            for (int r = 0; r < nrows; ++r) {
-                const bool left = sHi[r] < a0.v0, right = sLo[r] > v1a;
-                if (!left && !right) continue;   // windows overlap: written by k3_near
-                const double val = left ? sA[r * kMaxK + k0] * qt : sB[r * kMaxK + k0] * pt;
-                __builtin_nontemporal_store(val, Rrow + (size_t)r * rowlen + e);
+        int e = 0;
+        unsigned k = 0;
+        double2u_t pt, qt;
+        PairInfo a0, a1;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            if (SHIFT || r == 0) {   // (unshifted rows share their columns)
+                const int o = 2 * (i * kThreads + tid) - shift[r];
+                const unsigned a = kb + o, qo = rK ? __umulhi(a, rK) : a;
+                e = e0 + o;
+                k = a - qo * uK;
+                const int q0 = qb - kFarLine + (int)qo, q1 = k + 1 == uK ? q0 + 1 : q0;
+                // (an element before or behind the row reads a clamped place and is not stored)
+                const int ec = e < 0 ? 0 : e > rowlen - 2 ? rowlen - 2 : e;
+                const double2u_t pv = *(const double2u_t*)(Ptot + ec), qv = *(const double2u_t*)(Qtot + ec);
+                pt = e == ec ? pv : double2u_t{pv.y, pv.x};
+                qt = e == ec ? qv : double2u_t{qv.y, qv.x};
+                a0 = pairs[min(max(q0, 0), n_pairs - 1)];
+                a1 = pairs[min(max(q1, 0), n_pairs - 1)];
             }
-        } else {
-            const int q1 = (k0 + 1 == K) ? q0 + 1 : q0, k1 = (k0 + 1 == K) ? 0 : k0 + 1;
-            const double2_t pt = *(const double2_t*)(Ptot + e), qt = *(const double2_t*)(Qtot + e);
-            const PairInfo a1 = pairs[q1];
-            const int v1b = a1.v0 + a1.m - 1;
-            for (int r = 0; r < nrows; ++r) {
-                const bool l0 = sHi[r] < a0.v0, f0 = l0 || sLo[r] > v1a;
-                const bool l1 = sHi[r] < a1.v0, f1 = l1 || sLo[r] > v1b;
-                double2_t val;
-                val.x = l0 ? sA[r * kMaxK + k0] * qt.x : sB[r * kMaxK + k0] * pt.x;
-                val.y = l1 ? sA[r * kMaxK + k1] * qt.y : sB[r * kMaxK + k1] * pt.y;
-                double* dst = Rrow + (size_t)r * rowlen + e;
-                if (f0 && f1) {
-                    __builtin_nontemporal_store(val, (double2_t*)dst);
-                } else {
-                    if (f0) __builtin_nontemporal_store(val.x, dst);
-                    if (f1) __builtin_nontemporal_store(val.y, dst + 1);
-                }
-            }
+            if (r >= nrows) continue;
+            const bool l0 = hi[r] < a0.v0, l1 = hi[r] < a1.v0;   // the row's window lies left of the column's
+            const bool f0 = e >= 0 && e < rowlen && (l0 || lo[r] > a0.v0 + a0.m - 1);
+            const bool f1 = e + 1 >= 0 && e + 1 < rowlen && (l1 || lo[r] > a1.v0 + a1.m - 1);
+            const double* gp = sP + r * kFarLd + k;
+            const double* gq = sQ + r * kFarLd + k;
+            const double2u_t v = {l0 ? gp[0] * qt.x : gq[0] * pt.x, l1 ? gp[1] * qt.y : gq[1] * pt.y};
+            double* const dst = Rrow + (size_t)r * rowlen + e;
+            // (an element whose windows overlap is left to k3_near)
+            if (f0 && f1) *(double2u_t*)dst = v;
+            else if (f0) dst[0] = v.x;
+            else if (f1) dst[1] = v.y;
         }
     }
 }
@@ -339,49 +419,56 @@ hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, bool
     return hipGetLastError();
 }
 
-// Shapes of the rank-one fill the autotuner chooses from: elements per
-// store (V), rows and element groups per workgroup.
+// Shapes of the rank-one fill the autotuner chooses from: rows and groups of
+// 512 elements per workgroup, and whether the rows' chunks are shifted to
+// lines of memory (the shapes that take rows of odd length).
 struct FarShape {
-    int V, rows, iters;
+    int rows, iters;
+    bool shift;
 };
-static constexpr FarShape kFarShapes[] = {{2, 2, 1}, {2, 2, 2}, {2, 4, 4}, {2, 2, 8}, {2, 1, 4}, {1, 4, 8}, {1, 2, 4}};
+static constexpr FarShape kFarShapes[] = {{2, 1, false}, {2, 2, false}, {4, 1, false}, {1, 2, false},
+                                          {1, 1, false}, {2, 1, true},  {2, 2, true}};
 
 int far_variant_count() { return (int)(sizeof(kFarShapes) / sizeof(kFarShapes[0])); }
 
 bool far_variant_valid(const Plan& p, int v)
 {
-    return v >= 0 && v < far_variant_count() && (kFarShapes[v].V == 1 || (p.n_pairs * p.K) % 2 == 0);
+    return v >= 0 && v < far_variant_count() && (kFarShapes[v].shift || (p.n_pairs * p.K) % 2 == 0);
 }
 
-// 2 rows x 512 elements, one 16-byte store per thread and row: a short
-// workgroup life keeps more stores in flight than longer loops (5.7 TB/s
-// against 5.5 for 2 x 1024 at 0.76 GB); rows of odd length fall back to
-// 8-byte stores.
-int far_variant_default(const Plan& p) { return (p.n_pairs * p.K) % 2 == 0 ? 0 : 5; }
+// 2 rows x 512 elements, shifted unless every row starts on a line (the
+// tensor does): a shifted row reads its own column factors.  Whole builds of
+// 2944 pairs x 11 multipoles (lines) 0.146 ms unshifted against 0.153, of
+// 10128 x 25 (lines) 3.26 against 3.24; of 4444 x 17 0.534 against 0.463.
+int far_variant_default(const Plan& p) { return (p.n_pairs * p.K) % kFarLine == 0 ? 0 : 5; }
 
-template <int V, int ROWS, int ITERS>
+template <int V>
 static void launch_far_shape(const Plan& p, const DevTables& d, double* R, hipStream_t s)
 {
+    constexpr FarShape f = kFarShapes[V];
     const int64_t rowlen = p.n_pairs * p.K;
-    const int64_t per = (int64_t)V * kThreads * ITERS;
-    const int far_cols = (int)((rowlen + per - 1) / per);
-    const int far_rows = (int)((p.n_pairs + ROWS - 1) / ROWS);
-    const int x_cols = (far_cols + kXcds - 1) / kXcds;   // column chunks per XCD
-    hipLaunchKernelGGL((k3_far<V, ROWS, ITERS>), dim3((unsigned)(kXcds * x_cols * far_rows)), dim3(kThreads), 0, s,
-                       (int)p.n_pairs, (int)p.K, far_cols, x_cols, d.pairs, d.Ptot, d.Qtot, R);
+    const int64_t per = 2 * (int64_t)kThreads * f.iters;
+    // (a shifted row's last elements lie up to 15 past its last chunk)
+    const unsigned cols = (unsigned)((rowlen + (f.shift ? kFarLine - 1 : 0) + per - 1) / per);
+    const unsigned rows = (unsigned)((p.n_pairs + f.rows - 1) / f.rows);
+    const unsigned x_cols = 2 * sizeof(double) * rowlen > kFarSliceBytes ? (cols + kXcds - 1) / kXcds : 0;
+    const dim3 grid(x_cols ? kXcds * x_cols : cols, std::min(rows, kFarGridY), (rows + kFarGridY - 1) / kFarGridY);
+    hipLaunchKernelGGL((k3_far<f.rows, f.iters, f.shift>), grid, dim3(kThreads), 0, s, (int)p.n_pairs, (int)p.n_b,
+                       (int)p.K, (int)p.k_s, recip32(p.K), recip32(p.K + 1), (int)cols, (int)x_cols, d.pairs,
+                       d.c_first, d.Ptot, d.Qtot, R);
 }
 
 hipError_t launch_tensor_far(const Plan& p, const DevTables& d, double* R, hipStream_t s)
 {
     const int v = far_variant_valid(p, p.far_variant) ? p.far_variant : far_variant_default(p);
     switch (v) {
-    case 0: launch_far_shape<2, 2, 1>(p, d, R, s); break;
-    case 1: launch_far_shape<2, 2, 2>(p, d, R, s); break;
-    case 2: launch_far_shape<2, 4, 4>(p, d, R, s); break;
-    case 3: launch_far_shape<2, 2, 8>(p, d, R, s); break;
-    case 4: launch_far_shape<2, 1, 4>(p, d, R, s); break;
-    case 5: launch_far_shape<1, 4, 8>(p, d, R, s); break;
-    default: launch_far_shape<1, 2, 4>(p, d, R, s); break;
+    case 0: launch_far_shape<0>(p, d, R, s); break;
+    case 1: launch_far_shape<1>(p, d, R, s); break;
+    case 2: launch_far_shape<2>(p, d, R, s); break;
+    case 3: launch_far_shape<3>(p, d, R, s); break;
+    case 4: launch_far_shape<4>(p, d, R, s); break;
+    case 5: launch_far_shape<5>(p, d, R, s); break;
+    default: launch_far_shape<6>(p, d, R, s); break;
     }
     return hipGetLastError();
 }

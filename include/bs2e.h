@@ -152,7 +152,7 @@ int64_t bs2e_rk_stage_times(bs2e_rk *rk, double *ms, int64_t n);
  * combinable with profiling.  (No reference counterpart.) */
 int64_t bs2e_rk_set_graph(bs2e_rk *rk, int64_t on);
 /* Autotuner: times, on this handle's own tables, each shape of the rank-one
- * fill (elements per store, rows and elements per workgroup) and each
+ * fill (rows and elements per workgroup, rows shifted to lines of memory) and each
  * multipole chunk of the diagonal-cell kernel, and keeps the fastest for
  * this handle and, for the process, for every basis of the same order, GL
  * order, multipole count, pair and interval counts (force != 0 re-times a
@@ -170,7 +170,7 @@ int64_t bs2e_rk_tuning(const bs2e_rk *rk, int64_t *out, int64_t n);
  * rank-one fill is measured against.  (No reference counterpart.) */
 int64_t bs2e_store_ceiling(bs2e_ctx *ctx, void *dst, int64_t n_bytes, int64_t reps, double *gbs);
 /* Pins the rank-one fill shape (0 .. the shapes the autotuner times; those
- * with two elements per store need an even n_pairs * K) and the multipoles
+ * without shifted rows need an even n_pairs * K) and the multipoles
  * per diagonal-cell workgroup (1 .. the largest that fits) for this handle's
  * next builds; BS2E_EINVAL outside those.  All choices compute the same
  * values.  (No reference counterpart.) */
