@@ -269,7 +269,8 @@ int far_variant_default(const Plan& p);
 hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s);
 size_t outer_lds_bytes(int64_t ks, int64_t kgl, int64_t K);
 size_t inner_lds_bytes(int64_t ks, int64_t kgl, int64_t kc);
-int inner_kc(int64_t ks, int64_t kgl, int64_t K);   // multipoles per diagonal-cell workgroup (0: unsupported)
+int inner_kc(int64_t ks, int64_t kgl, int64_t K);   // largest multipole chunk of a diagonal-cell workgroup (0: unsupported)
+int inner_kc_used(const Plan& p);                   // the chunk the next build takes
 hipError_t launch_scatter_4d(const Plan& p, const DevTables& d, const int64_t* d_off4, double* rk, double* rmk,
                              int64_t* iv, int64_t* i, int64_t* j, hipStream_t s);
 hipError_t launch_scatter_6d(const Plan& p, const DevTables& d, const DiagEntry* d_diag, int64_t n_diag, double* rdk,

@@ -798,7 +798,7 @@ int64_t bs2e_rk_tuning(const bs2e_rk* rk, int64_t* out, int64_t n)
     if (!rk || !out) return fail(nullptr, BS2E_EINVAL, "bs2e_rk_tuning: NULL argument");
     const Plan& p = rk->plan;
     const int64_t v[2] = {far_variant_valid(p, p.far_variant) ? p.far_variant : far_variant_default(p),
-                          (p.inner_kc >= 1) ? p.inner_kc : inner_kc(p.k_s, p.k_gl, p.K)};
+                          rk->from_primitives ? inner_kc(p.k_s, p.k_gl, p.K) : inner_kc_used(p)};
     for (int64_t i = 0; i < n && i < 2; ++i) out[i] = v[i];
     return BS2E_OK;
 }

@@ -17,8 +17,8 @@
 //   cells of mat_els.f90:460-483 as the contraction over the outer points
 //     D[v][uo][ui][k] = h_v sum_q (w_q B_a B_c)(r_q) * J'[k][q][ui],
 //     J'[k][q][u]     = s_q / r_q^(k+1) * sum_p w_p rho_qp^k B_b B_d(rho_qp),
-//   with s_q = (r_q - bp_v)/2 and rho_qp = s_q x_p + (r_q + bp_v)/2; each
-//   thread accumulates kc multipoles in registers, staging in LDS.
+//   with s_q = (r_q - bp_v)/2 and rho_qp = s_q x_p + (r_q + bp_v)/2, on the
+//   FP64 matrix cores, a few multipoles at a time staged in LDS.
 // kw_pair_windows: per banded pair p and multipole k, the window moments
 //   Pw/Qw[p][j][k] (j-th interval of p's support window), their prefix (P)
 //   and suffix (Q) sums and totals, gathered from Pl/Ql.
@@ -42,17 +42,13 @@ size_t outer_lds_bytes(int64_t ks, int64_t kgl, int64_t K)
     return sizeof(double) * (size_t)(kgl * ks + kgl + 2 * kgl * K);
 }
 
-// Orders up to kMfOrder (U <= 45 local pairs, three 16-wide tiles) with at
-// most 16 GL points contract the diagonal cells on the FP64 matrix cores
-// (kp_inner_mf); other bases use the vector-ALU kernel kp_inner.
-constexpr int kMfOrder = 9;
-constexpr int kMfMaxKc = 16;  // multipoles per matrix-core workgroup (register accumulators)
-constexpr int kMfSteps = 4;   // 4-point steps of the contraction: the matrix-core path takes k_GL <= 16
-
+// The multipoles that one diagonal-cell workgroup may be given (what a caller
+// can pin): 16, up to order 9 and 16 GL points as many as tables of all of
+// them in LDS would allow, 4 elsewhere.
 size_t inner_lds_bytes(int64_t ks, int64_t kgl, int64_t kc)
 {
     const int64_t U = ks * (ks + 1) / 2;
-    if (ks <= kMfOrder && kgl <= 4 * kMfSteps)   // sBo, sBi, sR, sWB, sX0, sXr, sJ[kc]
+    if (ks <= 9 && kgl <= 16)
         return sizeof(double) * (size_t)(kgl * ks + kgl * kgl * ks + kgl + kgl * U + 2 * kgl * kgl + kc * kgl * U);
     return sizeof(double) *
            (size_t)(kgl * ks + kgl * kgl * ks + kgl + kgl * kgl + kgl * U + kc * kgl * kgl + kc * kgl * U);
@@ -60,14 +56,25 @@ size_t inner_lds_bytes(int64_t ks, int64_t kgl, int64_t kc)
 
 int inner_kc(int64_t ks, int64_t kgl, int64_t K)
 {
-    if (ks <= kMfOrder && kgl <= 4 * kMfSteps) {   // all multipoles of an interval in one workgroup when they fit
-        for (int64_t kc = std::min<int64_t>(K, kMfMaxKc); kc >= 1; --kc)
+    if (ks <= 9 && kgl <= 16) {
+        for (int64_t kc = std::min<int64_t>(K, 16); kc >= 1; --kc)
             if (inner_lds_bytes(ks, kgl, kc) <= kLdsPerWorkgroup) return (int)kc;
         return 0;
     }
     for (int kc : {4, 2, 1})
         if (kc <= K && inner_lds_bytes(ks, kgl, kc) <= kLdsPerWorkgroup) return kc;
     return inner_lds_bytes(ks, kgl, 1) <= kLdsPerWorkgroup ? 1 : 0;
+}
+
+// LDS of a diagonal-cell workgroup that holds the inner moments of KC
+// multipoles at a time: the splines at the outer and inner points, the outer
+// pair products (over the GL points padded to a multiple of four) and inner
+// moments, and X and its ratio at the inner points.  All that inner_kc accepts
+// fits with KC = 1.
+static size_t diag_lds_bytes(int64_t ks, int64_t kgl, int64_t KC)
+{
+    const int64_t U = ks * (ks + 1) / 2, QP = (kgl + 3) / 4 * 4;
+    return sizeof(double) * (size_t)(kgl * (1 + kgl) * ks + 2 * kgl * kgl + (KC * kgl + QP) * U);
 }
 
 template <int KS>
@@ -116,134 +123,49 @@ __global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const doub
     }
 }
 
-// SYM: write Dsym[v][u1][u2][k] = D[v][u1][u2][k] + D[v][u2][u1][k] (what the
-// tensor consumes) for u1 <= u2 only, the symmetric matrix's upper triangle,
-// instead of D (what the sparse_6d container holds).
-template <int KS, bool SYM>
+// The diagonal cells.  SYM: write Dsym[v][u1][u2][k] = D[v][u1][u2][k] +
+// D[v][u2][u1][k] (what the tensor consumes) for u1 <= u2 only, the symmetric
+// matrix's upper triangle, instead of D (what the sparse_6d container holds).
+// Per workgroup: interval v and multipoles k0 .. k0+nk-1 (the chunks of one
+// interval sit on one XCD, so the K-contiguous records of D are completed in
+// one L2).
+//   stage 1: splines at the outer and inner points; X_k0[q][p] =
+//            s_q w_p rho^k0 / r_q^(k0+1) (from X_0 by k0 multiplications with
+//            the ratio rho / r_q, so that every chunking gives the same bits);
+//   stage 2: WB[q][u] = w_q B_a B_c (r_q);
+// then for KC multipoles at a time
+//   stage 3: J'[kk][q][u] = sum_p X_k[q][p] B_b B_d (rho_qp), the powers by
+//            repeated multiplication with the ratio;
+//   stage 4: per 16 x 16 tile of (uo, ui) and two multipoles, on
+//            v_mfma_f64_16x16x4: D = WB^T J' (SYM: Dsym = WB^T J' + J'^T WB,
+//            the two products in separate accumulators, upper-triangle tiles
+//            and elements only), zero-padded to a multiple of four GL points.
+// The FP64 matrix cores run at the vector rate; they are used because a tile
+// reads its operands from LDS 16 times less often.  Bound by latency: the
+// stages are short and wait for one another, so what counts is the number of
+// workgroups a CU holds (KC as small as keeps the two multipoles of a tile
+// busy: the inner moments of all multipoles at once took 104 KB of LDS at
+// order 9, one workgroup per CU) and a loop body that stays in the instruction
+// cache.
+template <int KS, bool SYM, int KC>
 __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks,
                                                       const double* __restrict__ t, const double* __restrict__ bp,
                                                       const double* __restrict__ x, const double* __restrict__ w,
                                                       double* __restrict__ D)
 {
     constexpr int U = KS * (KS + 1) / 2;
-    constexpr int KCMAX = 4;
-    extern __shared__ double lds[];
-    double* sBo = lds;                       // [kgl][KS]       outer points
-    double* sBi = sBo + kgl * KS;            // [kgl][kgl][KS]  inner points
-    double* sR = sBi + kgl * kgl * KS;       // [kgl]
-    double* sRho = sR + kgl;                 // [kgl][kgl]
-    double* sWB = sRho + kgl * kgl;          // [kgl][U]        w_q B_a B_c at r_q
-    double* sX = sWB + kgl * U;              // [kc][kgl][kgl]  s_q w_p rho^k / r_q^(k+1)
-    double* sJ = sX + kc * kgl * kgl;        // [kc][kgl][U]
-
-    const int v = blockIdx.x / kchunks;
-    const int k0 = (blockIdx.x - v * kchunks) * kc;
-    const int nk = (K - k0) < kc ? (K - k0) : kc;
-    const int tid = threadIdx.x;
-    const double lim1 = bp[v], lim2 = bp[v + 1];
-    const double h = 0.5 * (lim2 - lim1);
-    const double c = 0.5 * (lim2 + lim1);
-    const int i1 = KS - 1 + (v + 1);
-
-    for (int e = tid; e < kgl * (1 + kgl); e += kPThreads) {
-        if (e < kgl) {
-            const double r = h * x[e] + c;
-            sR[e] = r;
-            splines_at<KS>(t, i1, r, sBo + e * KS, 1);
-        } else {
-            const int q = (e - kgl) / kgl, p = (e - kgl) - q * kgl;
-            const double rq = h * x[q] + c;
-            const double rho = 0.5 * (rq - lim1) * x[p] + 0.5 * (rq + lim1);
-            sRho[q * kgl + p] = rho;
-            splines_at<KS>(t, i1, rho, sBi + (q * kgl + p) * KS, 1);
-        }
-    }
-    __syncthreads();
-    for (int e = tid; e < kgl * U; e += kPThreads) {
-        const int q = e / U, u = e - q * U;
-        int ta, tc;
-        local_pair(u, KS, ta, tc);
-        sWB[e] = w[q] * sBo[q * KS + ta] * sBo[q * KS + tc];
-    }
-    for (int e = tid; e < nk * kgl * kgl; e += kPThreads) {
-        const int kk = e / (kgl * kgl), qp = e - kk * kgl * kgl;
-        const int q = qp / kgl, p = qp - q * kgl;
-        const int k = k0 + kk;
-        const double rq = sR[q];
-        sX[e] = 0.5 * (rq - lim1) * w[p] * ipow_d(sRho[qp], k) / ipow_d(rq, k + 1);
-    }
-    __syncthreads();
-    // J'[kk][q][u] = sum_p X[kk][q][p] B_b(rho_qp) B_d(rho_qp)
-    for (int e = tid; e < kgl * U; e += kPThreads) {
-        const int q = e / U, u = e - q * U;
-        int ta, tc;
-        local_pair(u, KS, ta, tc);
-        double acc[KCMAX] = {0.0, 0.0, 0.0, 0.0};
-        const double* bq = sBi + q * kgl * KS;
-        for (int p = 0; p < kgl; ++p) {
-            const double bb = bq[p * KS + ta] * bq[p * KS + tc];
-#pragma unroll
-            for (int kk = 0; kk < KCMAX; ++kk)
-                if (kk < nk) acc[kk] += sX[(kk * kgl + q) * kgl + p] * bb;
-        }
-#pragma unroll
-        for (int kk = 0; kk < KCMAX; ++kk)
-            if (kk < nk) sJ[(kk * kgl + q) * U + u] = acc[kk];
-    }
-    __syncthreads();
-    // D[v][uo][ui][k0 .. k0+nk) = h * sum_q WB[q][uo] J'[kk][q][ui]
-    for (int e = tid; e < U * U; e += kPThreads) {
-        const int uo = e / U, ui = e - uo * U;
-        if (SYM && uo > ui) continue;   // the lower triangle mirrors the upper
-        double acc[KCMAX] = {0.0, 0.0, 0.0, 0.0};
-        for (int q = 0; q < kgl; ++q) {
-            const double a = sWB[q * U + uo];
-            const double b = SYM ? sWB[q * U + ui] : 0.0;
-#pragma unroll
-            for (int kk = 0; kk < KCMAX; ++kk)
-                if (kk < nk) {
-                    acc[kk] += a * sJ[(kk * kgl + q) * U + ui];
-                    if (SYM) acc[kk] += b * sJ[(kk * kgl + q) * U + uo];
-                }
-        }
-        double* dst = D + (((size_t)v * U + uo) * U + ui) * K + k0;
-#pragma unroll
-        for (int kk = 0; kk < KCMAX; ++kk)
-            if (kk < nk) dst[kk] = h * acc[kk];
-    }
-}
-
-// Matrix-core variant of kp_inner for orders <= kMfOrder.  Per workgroup:
-// interval v and multipoles k0 .. k0+nk-1 (the chunks of one interval sit on
-// one XCD, so the K-contiguous records of D are completed in one L2).
-//   stage 1: splines at the outer and inner points; X_k0[q][p] =
-//            s_q w_p rho^k0 / r_q^(k0+1) (from X_0 by k0 multiplications with
-//            the ratio rho / r_q, so that every chunking gives the same bits);
-//   stage 2: WB[q][u] = w_q B_a B_c (r_q);
-//   stage 3: J'[kk][q][u] = sum_p X_k[q][p] B_b B_d (rho_qp), the powers for
-//            k > k0 by repeated multiplication with the ratio;
-//   stage 4: per 16 x 16 tile of (uo, ui) and multipole, on v_mfma_f64_16x16x4:
-//            D = WB^T J' (SYM: Dsym = WB^T J' + J'^T WB, the two products in
-//            separate accumulators, upper-triangle tiles and elements only),
-//            zero-padded to whole tiles and to 16 GL points; two multipoles
-//            per pass.
-template <int KS, bool SYM>
-__global__ __launch_bounds__(kPThreads) void kp_inner_mf(int K, int kgl, int kc, int kchunks,
-                                                         const double* __restrict__ t, const double* __restrict__ bp,
-                                                         const double* __restrict__ x, const double* __restrict__ w,
-                                                         double* __restrict__ D)
-{
-    constexpr int U = KS * (KS + 1) / 2;
     constexpr int TU = (U + 15) / 16;
+    constexpr int NT = SYM ? TU * (TU + 1) / 2 : TU * TU;
+    constexpr int NP = (KC + 1) / 2;         // pairs of multipoles per group
     typedef double d4_t __attribute__((ext_vector_type(4)));
+    typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
     extern __shared__ double lds[];
-    double* sBo = lds;                       // [kgl][KS]       outer points
-    double* sBi = sBo + kgl * KS;            // [kgl][kgl][KS]  inner points
-    double* sR = sBi + kgl * kgl * KS;       // [kgl]
-    double* sWB = sR + kgl;                  // [kgl][U]        w_q B_a B_c at r_q
-    double* sX0 = sWB + kgl * U;             // [kgl][kgl]      X_k0
-    double* sXr = sX0 + kgl * kgl;           // [kgl][kgl]      rho / r_q
-    double* sJ = sXr + kgl * kgl;            // [kc][kgl][U]
+    const int npt = kgl * (1 + kgl), QP = (kgl + 3) & ~3;
+    double* sB = lds;                        // [kgl + kgl * kgl][KS]: outer points, then inner points
+    double* sX = sB + npt * KS;              // [kgl][kgl]      X of the group's first multipole
+    double* sXr = sX + kgl * kgl;            // [kgl][kgl]      rho / r_q
+    double* sJ = sXr + kgl * kgl;            // [KC][kgl][U]    (read past kgl: the next rows, times a zero of sWB)
+    double* sWB = sJ + KC * kgl * U;         // [QP][U]         w_q B_a B_c at r_q (zero past kgl)
 
     const int64_t lg = xcd_block(blockIdx.x, gridDim.x);
     const int v = (int)(lg / kchunks);
@@ -255,119 +177,102 @@ __global__ __launch_bounds__(kPThreads) void kp_inner_mf(int K, int kgl, int kc,
     const double c = 0.5 * (lim2 + lim1);
     const int i1 = KS - 1 + (v + 1);
 
-    for (int e = tid; e < kgl * (1 + kgl); e += kPThreads) {
-        if (e < kgl) {
-            const double r = h * x[e] + c;
-            sR[e] = r;
-            splines_at<KS>(t, i1, r, sBo + e * KS, 1);
-        } else {
-            const int q = (e - kgl) / kgl, pp = (e - kgl) - q * kgl;
-            const double rq = h * x[q] + c;
-            const double rho = 0.5 * (rq - lim1) * x[pp] + 0.5 * (rq + lim1);
-            splines_at<KS>(t, i1, rho, sBi + (q * kgl + pp) * KS, 1);
+#pragma unroll 1
+    for (int e = tid; e < npt; e += kPThreads) {
+        const bool inner = e >= kgl;
+        const int q = inner ? e / kgl - 1 : e, pp = inner ? e - (q + 1) * kgl : 0;
+        const double rq = h * x[q] + c;
+        const double rho = inner ? 0.5 * (rq - lim1) * x[pp] + 0.5 * (rq + lim1) : rq;
+        splines_at<KS>(t, i1, rho, sB + e * KS, 1);
+        if (inner) {
             // X_k = s_q w_p rho^k / r_q^(k+1) = X_0 (rho / r_q)^k, the same
             // multiplication sequence from k = 0 for every chunking
             const double ratio = rho / rq;
             double xk = 0.5 * (rq - lim1) * w[pp] / rq;
             for (int j = 0; j < k0; ++j) xk *= ratio;
-            sX0[q * kgl + pp] = xk;
-            sXr[q * kgl + pp] = ratio;
+            sX[e - kgl] = xk;
+            sXr[e - kgl] = ratio;
         }
     }
+    for (int e = kgl * U + tid; e < QP * U; e += kPThreads) sWB[e] = 0.0;
     __syncthreads();
+#pragma unroll 1
     for (int e = tid; e < kgl * U; e += kPThreads) {
         const int q = e / U, u = e - q * U;
         int ta, tc;
         local_pair(u, KS, ta, tc);
-        sWB[e] = w[q] * sBo[q * KS + ta] * sBo[q * KS + tc];
+        sWB[e] = w[q] * sB[q * KS + ta] * sB[q * KS + tc];
     }
-    for (int e = tid; e < kgl * U; e += kPThreads) {
-        const int q = e / U, u = e - q * U;
-        int ta, tc;
-        local_pair(u, KS, ta, tc);
-        double acc[kMfMaxKc];
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int li = lane & 15, lk = lane >> 4;
+#pragma unroll 1
+    for (int g = 0; g < nk; g += KC) {
+#pragma unroll 1
+        for (int e = tid; e < kgl * U; e += kPThreads) {
+            const int q = e / U, u = e - q * U;
+            int ta, tc;
+            local_pair(u, KS, ta, tc);
+            double acc[KC];
 #pragma unroll
-        for (int kk = 0; kk < kMfMaxKc; ++kk) acc[kk] = 0.0;
-        const double* bq = sBi + q * kgl * KS;
-        for (int pp = 0; pp < kgl; ++pp) {
-            const double bb = bq[pp * KS + ta] * bq[pp * KS + tc];
-            double xk = sX0[q * kgl + pp];
-            const double ratio = sXr[q * kgl + pp];
+            for (int kk = 0; kk < KC; ++kk) acc[kk] = 0.0;
+            const double* bq = sB + (kgl + q * kgl) * KS;
+            const double* xq = sX + q * kgl;
+            const double* rq = sXr + q * kgl;
+#pragma unroll 2
+            for (int pp = 0; pp < kgl; ++pp) {
+                const double bb = bq[pp * KS + ta] * bq[pp * KS + tc];
+                double xk = xq[pp];
+                const double ratio = rq[pp];
 #pragma unroll
-            for (int kk = 0; kk < kMfMaxKc; ++kk)
-                if (kk < nk) {
+                for (int kk = 0; kk < KC; ++kk) {   // (past the chunk's last multipole: not used)
                     acc[kk] += xk * bb;
                     xk *= ratio;
                 }
-        }
-#pragma unroll
-        for (int kk = 0; kk < kMfMaxKc; ++kk)
-            if (kk < nk) sJ[(kk * kgl + q) * U + u] = acc[kk];
-    }
-    __syncthreads();
-    const int wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, lk = lane >> 4;
-    // Operands are read from clamped addresses and zeroed outside the U x kgl
-    // range (no lane-predicated loads), so the loads of a pass issue back to
-    // back ahead of its matrix instructions.
-    constexpr int NT = SYM ? TU * (TU + 1) / 2 : TU * TU;
-    for (int tile = wave; tile < NT; tile += kPThreads / 64) {
-        int ta, tb;
-        if (SYM) {   // upper-triangle tiles, row by row
-            ta = 0;
-            int r = tile;
-            while (r >= TU - ta) {
-                r -= TU - ta;
-                ++ta;
             }
-            tb = ta + r;
-        } else {
-            ta = tile / TU;
-            tb = tile - ta * TU;
-        }
-        const int uo_a = ta * 16 + li, ui_b = tb * 16 + li;   // operand row / column of this lane
-        const bool va = uo_a < U, vb = ui_b < U;
-        const int ua = va ? uo_a : U - 1, ub = vb ? ui_b : U - 1;
-        int qo[kMfSteps];
-        bool qv[kMfSteps];
 #pragma unroll
-        for (int st = 0; st < kMfSteps; ++st) {
-            const int q = st * 4 + lk;
-            qv[st] = q < kgl;
-            qo[st] = (qv[st] ? q : kgl - 1) * U;
+            for (int kk = 0; kk < KC; ++kk) sJ[kk * kgl * U + e] = acc[kk];
         }
-        // WB operands do not depend on the multipole: loaded once per tile
-        double a1[kMfSteps], b2[kMfSteps];
+        __syncthreads();
+        for (int e = tid; e < kgl * kgl; e += kPThreads) {   // (read again after the next barrier)
+            double xk = sX[e];
 #pragma unroll
-        for (int st = 0; st < kMfSteps; ++st) {
-            const double x1 = sWB[qo[st] + ua], x2 = sWB[qo[st] + ub];
-            a1[st] = (qv[st] && va) ? x1 : 0.0;
-            b2[st] = (qv[st] && vb) ? x2 : 0.0;
+            for (int kk = 0; kk < KC; ++kk) xk *= sXr[e];
+            sX[e] = xk;
         }
-        for (int kk = 0; kk < nk; kk += 2) {
-            const bool two = kk + 1 < nk;   // two multipoles per pass: four independent chains
-            const double* J0 = sJ + (size_t)kk * kgl * U;
-            const double* J1 = J0 + (two ? kgl * U : 0);
-            double b10[kMfSteps], b11[kMfSteps], a20[kMfSteps], a21[kMfSteps];
-#pragma unroll
-            for (int st = 0; st < kMfSteps; ++st) {
-                const double y0 = J0[qo[st] + ub], y1 = J1[qo[st] + ub];
-                b10[st] = (qv[st] && vb) ? y0 : 0.0;
-                b11[st] = (qv[st] && vb) ? y1 : 0.0;
-                if (SYM) {
-                    const double z0 = J0[qo[st] + ua], z1 = J1[qo[st] + ua];
-                    a20[st] = (qv[st] && va) ? z0 : 0.0;
-                    a21[st] = (qv[st] && va) ? z1 : 0.0;
+        const int left = nk - g;             // multipoles from this group on
+#pragma unroll 1
+        for (int item = wave; item < NT * NP; item += kPThreads / 64) {
+            const int tile = item / NP, kk = 2 * (item - tile * NP);
+            if (kk >= left) continue;
+            const bool two = KC > 1 && kk + 1 < left;
+            int ta, tb;
+            if (SYM) {   // upper-triangle tiles, row by row
+                ta = 0;
+                int r = tile;
+                while (r >= TU - ta) {
+                    r -= TU - ta;
+                    ++ta;
                 }
+                tb = ta + r;
+            } else {
+                ta = tile / TU;
+                tb = tile - ta * TU;
             }
+            // operand row / column of this lane (clamped: elements past U are not stored)
+            const int ua = min(ta * 16 + li, U - 1), ub = min(tb * 16 + li, U - 1);
+            const double* W = sWB + lk * U;
+            const double* J0 = sJ + (kk * kgl + lk) * U;
+            const double* J1 = KC > 1 ? J0 + kgl * U : J0;
             d4_t c0 = {0.0, 0.0, 0.0, 0.0}, c1 = c0, e0 = c0, e1 = c0;
-#pragma unroll
-            for (int st = 0; st < kMfSteps; ++st) {
-                c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b10[st], c0, 0, 0, 0);
-                c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[st], b11[st], c1, 0, 0, 0);
+#pragma unroll 2
+            for (int q = 0; q < QP; q += 4) {
+                const double a1 = W[q * U + ua], b0 = J0[q * U + ub], b1 = J1[q * U + ub];
+                c0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, c0, 0, 0, 0);
+                if (KC > 1) c1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, c1, 0, 0, 0);
                 if (SYM) {
-                    e0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a20[st], b2[st], e0, 0, 0, 0);
-                    e1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a21[st], b2[st], e1, 0, 0, 0);
+                    const double b2 = W[q * U + ub], a20 = J0[q * U + ua], a21 = J1[q * U + ua];
+                    e0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a20, b2, e0, 0, 0, 0);
+                    if (KC > 1) e1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a21, b2, e1, 0, 0, 0);
                 }
             }
             // result row (lane >> 4) + 4 r, column lane & 15 of the tile
@@ -375,12 +280,14 @@ __global__ __launch_bounds__(kPThreads) void kp_inner_mf(int K, int kgl, int kc,
             for (int r = 0; r < 4; ++r) {
                 const int uo = ta * 16 + lk + 4 * r, ui = tb * 16 + li;
                 if (uo < U && ui < U && (!SYM || uo <= ui)) {
-                    double* dst = D + (((size_t)v * U + uo) * U + ui) * K + k0 + kk;
-                    dst[0] = h * (SYM ? c0[r] + e0[r] : c0[r]);
-                    if (two) dst[1] = h * (SYM ? c1[r] + e1[r] : c1[r]);
+                    double* dst = D + (((size_t)v * U + uo) * U + ui) * K + k0 + g + kk;
+                    const double d0 = h * (SYM ? c0[r] + e0[r] : c0[r]), d1 = h * (SYM ? c1[r] + e1[r] : c1[r]);
+                    if (two) *(d2u_t*)dst = d2u_t{d0, d1};
+                    else *dst = d0;
                 }
             }
         }
+        __syncthreads();
     }
 }
 
@@ -469,24 +376,47 @@ static void launch_outer(const Plan& p, const DevTables& d, hipStream_t s)
                        d.x, d.w, d.Pl, d.Ql);
 }
 
+// Multipoles that a diagonal-cell workgroup holds at a time: four; two where
+// groups of four would leave CUs without a workgroup (a shorter chain: order
+// 8, 41 intervals, 5 multipoles 10.1 us against 12.0), or their tables do not
+// fit (then one).  Groups of eight: 0.123 ms against 0.118 at order 9, 593
+// intervals, 25 multipoles; 0.088 against 0.047 at order 10, 175 intervals, 9.
+static int inner_group(const Plan& p)
+{
+    if (p.n_iv * ((p.K + 3) / 4) > 256 && diag_lds_bytes(p.k_s, p.k_gl, 4) <= kLdsPerWorkgroup) return 4;
+    return diag_lds_bytes(p.k_s, p.k_gl, 2) <= kLdsPerWorkgroup ? 2 : 1;
+}
+
+// Whole groups per workgroup, as many as leave two workgroups per CU (every
+// workgroup evaluates its interval's splines): order 8, 195 intervals, 11
+// multipoles in chunks of 4 18.9 us, in one chunk 23.0, of 2 25.3.
+int inner_kc_used(const Plan& p)
+{
+    const int kmax = inner_kc(p.k_s, p.k_gl, p.K);
+    if (p.inner_kc >= 1 && p.inner_kc <= kmax) return p.inner_kc;
+    const int64_t KC = inner_group(p), chunks = (512 + p.n_iv - 1) / p.n_iv;
+    const int64_t kc = ((p.K + chunks - 1) / chunks + KC - 1) / KC * KC;
+    return (int)std::min<int64_t>(kc, std::max(kmax, 1));
+}
+
+template <int KS, bool SYM, int KC>
+static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    const int kc = inner_kc_used(p), kchunks = (int)((p.K + kc - 1) / kc);
+    const size_t lds = diag_lds_bytes(KS, p.k_gl, KC);
+    const auto fn = kp_inner<KS, SYM, KC>;
+    if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
+    hipLaunchKernelGGL(fn, dim3((unsigned)(p.n_iv * kchunks)), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc,
+                       kchunks, d.t, d.bp, d.x, d.w, d.D);
+}
+
 template <int KS, bool SYM>
 static void launch_inner(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    const int kmax = inner_kc(KS, p.k_gl, p.K);
-    const int kc = (p.inner_kc >= 1 && p.inner_kc <= kmax) ? p.inner_kc : kmax;
-    const int kchunks = (int)((p.K + kc - 1) / kc);
-    const size_t lds = inner_lds_bytes(KS, p.k_gl, kc);
-    if (KS <= kMfOrder && p.k_gl <= 4 * kMfSteps) {
-        const auto fn = kp_inner_mf<KS <= kMfOrder ? KS : 2, SYM>;
-        if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-        hipLaunchKernelGGL(fn, dim3((unsigned)(p.n_iv * kchunks)), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc,
-                           kchunks, d.t, d.bp, d.x, d.w, d.D);
-    } else {
-        const auto fn = kp_inner<KS, SYM>;
-        if (allow_lds((const void*)fn, lds) != hipSuccess) return;
-        hipLaunchKernelGGL(fn, dim3((unsigned)(p.n_iv * kchunks)), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc,
-                           kchunks, d.t, d.bp, d.x, d.w, d.D);
-    }
+    const int KC = inner_group(p);
+    if (KC == 4) launch_inner_kc<KS, SYM, 4>(p, d, s);
+    else if (KC == 2) launch_inner_kc<KS, SYM, 2>(p, d, s);
+    else launch_inner_kc<KS, SYM, 1>(p, d, s);
 }
 
 template <int KS>
