@@ -382,13 +382,23 @@ static int64_t run_primitives_serial(bs2e_ctx* ctx, bs2e_rk* rk)
     return BS2E_OK;
 }
 
-// The full build.  Main stream: local moments -> pair windows -> rank-one
-// fill.  Side stream (forked once the pair windows exist, so that those two
-// short critical-path kernels run alone): diagonal cells -> near elements,
-// concurrently with the rank-one fill.  The main stream waits for the side
+// The full build.
+// Up to kOneStreamBytes of tensor: three launches on the main stream, the
+// local moments with the diagonal cells, the pair windows, and the near
+// elements with the rank-one fill (mixed precision: the moments in a launch of
+// their own).  Larger: main stream local moments -> pair windows -> rank-one
+// fill; side stream (forked once the pair windows exist, so that those two
+// short critical-path kernels run alone) diagonal cells -> near elements,
+// concurrently with the rank-one fill; the main stream waits for the side
 // stream at the end, so the build is one unit of work on the caller's stream.
+// The line lies where hiding the cells behind the fill gains more than the
+// second stream's events cost (about 20 us).  Builds one after another, one
+// stream against two: 0.0014 GB of tensor 13 us against 46, 0.016 GB 24 / 49,
+// 0.15 GB 45 / 59, 0.26 GB 73 / 79, 0.55 GB 131 / 135, 0.76 GB 153 / 147, 0.81 GB
+// 175 / 155, 2.7 GB 0.467 / 0.452 ms.
 // Profiling events, all relative to ev[0]: ev[1] windows done, ev[2] far
 // fill done, ev[3] diagonal cells done, ev[4] near elements done, ev[5] end.
+static constexpr size_t kOneStreamBytes = (size_t)576 << 20;
 static constexpr size_t kMaxProfiledBuilds = 1 << 16;
 
 static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
@@ -413,22 +423,42 @@ static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
         ev = rk->evpool[rk->evused++].data();
     }
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[0], m));
+    const Plan& p = rk->plan;
+    if (sizeof(double) * rk->R_elems <= kOneStreamBytes) {
+        if (!rk->from_primitives) {
+            if (rk->precision == BS2E_PREC_MIXED) {
+                HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
+                HIP_TRY(ctx, launch_diag_cells(p, rk->d, m, true));
+            } else {
+                HIP_TRY(ctx, launch_moments_and_cells(p, rk->d, m));
+            }
+            if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
+            HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
+        } else if (prof) {
+            HIP_TRY(ctx, hipEventRecord(ev[3], m));
+        }
+        if (prof) HIP_TRY(ctx, hipEventRecord(ev[1], m));
+        HIP_TRY(ctx, launch_tensor_fill(p, rk->d, rk->R, !rk->from_primitives, m));
+        if (prof)
+            for (int i : {2, 4, 5}) HIP_TRY(ctx, hipEventRecord(ev[i], m));
+        return BS2E_OK;
+    }
     if (!rk->from_primitives) {
         if (rk->precision == BS2E_PREC_MIXED)
-            HIP_TRY(ctx, launch_outer_moments_mixed(rk->plan, rk->d, m));
+            HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
         else
-            HIP_TRY(ctx, launch_outer_moments(rk->plan, rk->d, m));
-        HIP_TRY(ctx, launch_pair_windows(rk->plan, rk->d, m));
+            HIP_TRY(ctx, launch_outer_moments(p, rk->d, m));
+        HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
     }
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[1], m));
     HIP_TRY(ctx, hipEventRecord(rk->windows, m));
     HIP_TRY(ctx, hipStreamWaitEvent(s, rk->windows, 0));
-    if (!rk->from_primitives) HIP_TRY(ctx, launch_diag_cells(rk->plan, rk->d, s, true));
+    if (!rk->from_primitives) HIP_TRY(ctx, launch_diag_cells(p, rk->d, s, true));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], s));
-    HIP_TRY(ctx, launch_tensor_near(rk->plan, rk->d, rk->R, !rk->from_primitives, s));
+    HIP_TRY(ctx, launch_tensor_near(p, rk->d, rk->R, !rk->from_primitives, s));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[4], s));
     HIP_TRY(ctx, hipEventRecord(rk->join, s));
-    HIP_TRY(ctx, launch_tensor_far(rk->plan, rk->d, rk->R, m));
+    HIP_TRY(ctx, launch_tensor_far(p, rk->d, rk->R, m));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[2], m));
     HIP_TRY(ctx, hipStreamWaitEvent(m, rk->join, 0));
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[5], m));
@@ -668,7 +698,7 @@ int64_t bs2e_rk_compute(bs2e_rk* rk)
     rk->mirror_valid = false;
     if (rk->use_graph) {
         if (!rk->graph_exec) {
-            // capture the two-stream build once; its kernels and event
+            // capture the build once; its kernels and event
             // dependencies become the graph's nodes (no memset nodes)
             HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
             int64_t rc = run_build(ctx, rk);
@@ -745,7 +775,7 @@ int64_t bs2e_rk_autotune(bs2e_rk* rk, int64_t force)
     }
     const bool prof = rk->profiling;
     rk->profiling = false;
-    // Each candidate is timed over whole two-stream builds: the fill shares
+    // Each candidate is timed over whole builds: the fill shares
     // the chip with the diagonal cells and the near ranges, and the fastest
     // shape on its own is not always the fastest beside them.
     int64_t rc = BS2E_OK;

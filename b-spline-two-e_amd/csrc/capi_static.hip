@@ -133,14 +133,16 @@ int64_t bs2e_rk_build_static(int64_t k, int64_t n_knots, const double* knots, in
     // the scratch); the wait lets the host image go before the call returns.
     e = hipMemcpyAsync(base, host.data(), L.small_end, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    // one stream: moments, pair windows, diagonal cells (symmetrised), near
-    // elements, rank-one fill; the same kernels and values as bs2e_rk_compute
-    if (e == hipSuccess)
-        e = precision == BS2E_PREC_MIXED ? launch_outer_moments_mixed(p, d, s) : launch_outer_moments(p, d, s);
+    // one stream: moments and diagonal cells (symmetrised), pair windows, near
+    // elements and rank-one fill; the values of bs2e_rk_compute
+    if (e == hipSuccess && precision == BS2E_PREC_MIXED) {
+        e = launch_outer_moments_mixed(p, d, s);
+        if (e == hipSuccess) e = launch_diag_cells(p, d, s, true);
+    } else if (e == hipSuccess) {
+        e = launch_moments_and_cells(p, d, s);
+    }
     if (e == hipSuccess) e = launch_pair_windows(p, d, s);
-    if (e == hipSuccess) e = launch_diag_cells(p, d, s, true);
-    if (e == hipSuccess) e = launch_tensor_near(p, d, R, true, s);
-    if (e == hipSuccess) e = launch_tensor_far(p, d, R, s);
+    if (e == hipSuccess) e = launch_tensor_fill(p, d, R, true, s);
     if (e != hipSuccess)
         return fail(nullptr, BS2E_EDEVICE, std::string("bs2e_rk_build_static: ") + hipGetErrorString(e));
     return BS2E_OK;

@@ -77,19 +77,18 @@ static size_t diag_lds_bytes(int64_t ks, int64_t kgl, int64_t KC)
     return sizeof(double) * (size_t)(kgl * (1 + kgl) * ks + 2 * kgl * kgl + (KC * kgl + QP) * U);
 }
 
+// local moments of interval v
 template <int KS>
-__global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const double* __restrict__ t,
-                                                      const double* __restrict__ bp, const double* __restrict__ x,
-                                                      const double* __restrict__ w, double* __restrict__ Pl,
-                                                      double* __restrict__ Ql)
+__device__ __forceinline__ void outer_interval(int v, int K, int kgl, const double* __restrict__ t,
+                                               const double* __restrict__ bp, const double* __restrict__ x,
+                                               const double* __restrict__ w, double* __restrict__ Pl,
+                                               double* __restrict__ Ql, double* lds)
 {
     constexpr int U = KS * (KS + 1) / 2;
-    extern __shared__ double lds[];
     double* sB = lds;                 // [kgl][KS]
     double* sR = sB + kgl * KS;       // [kgl]
     double* sPow = sR + kgl;          // [kgl][K]  r^k
     double* sInv = sPow + kgl * K;    // [kgl][K]  1 / r^(k+1)
-    const int v = blockIdx.x;
     const int tid = threadIdx.x;
     const double lim1 = bp[v], lim2 = bp[v + 1];
     const double h = 0.5 * (lim2 - lim1);
@@ -123,6 +122,16 @@ __global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const doub
     }
 }
 
+template <int KS>
+__global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const double* __restrict__ t,
+                                                      const double* __restrict__ bp, const double* __restrict__ x,
+                                                      const double* __restrict__ w, double* __restrict__ Pl,
+                                                      double* __restrict__ Ql)
+{
+    extern __shared__ double lds[];
+    outer_interval<KS>((int)blockIdx.x, K, kgl, t, bp, x, w, Pl, Ql, lds);
+}
+
 // The diagonal cells.  SYM: write Dsym[v][u1][u2][k] = D[v][u1][u2][k] +
 // D[v][u2][u1][k] (what the tensor consumes) for u1 <= u2 only, the symmetric
 // matrix's upper triangle, instead of D (what the sparse_6d container holds).
@@ -147,11 +156,14 @@ __global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const doub
 // busy: the inner moments of all multipoles at once took 104 KB of LDS at
 // order 9, one workgroup per CU) and a loop body that stays in the instruction
 // cache.
-template <int KS, bool SYM, int KC>
-__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks,
+// OUTER: the workgroups past the n_cells of the cells take the local moments,
+// one interval each.
+template <int KS, bool SYM, int KC, bool OUTER>
+__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells,
                                                       const double* __restrict__ t, const double* __restrict__ bp,
                                                       const double* __restrict__ x, const double* __restrict__ w,
-                                                      double* __restrict__ D)
+                                                      double* __restrict__ D, double* __restrict__ Pl,
+                                                      double* __restrict__ Ql)
 {
     constexpr int U = KS * (KS + 1) / 2;
     constexpr int TU = (U + 15) / 16;
@@ -160,6 +172,10 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     typedef double d4_t __attribute__((ext_vector_type(4)));
     typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
     extern __shared__ double lds[];
+    if (OUTER && (int)blockIdx.x >= n_cells) {
+        outer_interval<KS>((int)blockIdx.x - n_cells, K, kgl, t, bp, x, w, Pl, Ql, lds);
+        return;
+    }
     const int npt = kgl * (1 + kgl), QP = (kgl + 3) & ~3;
     double* sB = lds;                        // [kgl + kgl * kgl][KS]: outer points, then inner points
     double* sX = sB + npt * KS;              // [kgl][kgl]      X of the group's first multipole
@@ -167,7 +183,7 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     double* sJ = sXr + kgl * kgl;            // [KC][kgl][U]    (read past kgl: the next rows, times a zero of sWB)
     double* sWB = sJ + KC * kgl * U;         // [QP][U]         w_q B_a B_c at r_q (zero past kgl)
 
-    const int64_t lg = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t lg = xcd_block(blockIdx.x, n_cells);
     const int v = (int)(lg / kchunks);
     const int k0 = (int)(lg - (int64_t)v * kchunks) * kc;
     const int nk = (K - k0) < kc ? (K - k0) : kc;
@@ -399,36 +415,44 @@ int inner_kc_used(const Plan& p)
     return (int)std::min<int64_t>(kc, std::max(kmax, 1));
 }
 
-template <int KS, bool SYM, int KC>
+template <int KS, bool SYM, int KC, bool OUTER>
 static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int kc = inner_kc_used(p), kchunks = (int)((p.K + kc - 1) / kc);
-    const size_t lds = diag_lds_bytes(KS, p.k_gl, KC);
-    const auto fn = kp_inner<KS, SYM, KC>;
+    const int n_cells = (int)(p.n_iv * kchunks);
+    size_t lds = diag_lds_bytes(KS, p.k_gl, KC);
+    if (OUTER) lds = std::max(lds, outer_lds_bytes(KS, p.k_gl, p.K));
+    const auto fn = kp_inner<KS, SYM, KC, OUTER>;
     if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(fn, dim3((unsigned)(p.n_iv * kchunks)), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc,
-                       kchunks, d.t, d.bp, d.x, d.w, d.D);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(n_cells + (OUTER ? p.n_iv : 0))), dim3(kPThreads), lds, s, (int)p.K,
+                       (int)p.k_gl, kc, kchunks, n_cells, d.t, d.bp, d.x, d.w, d.D, d.Pl, d.Ql);
 }
 
-template <int KS, bool SYM>
+template <int KS, bool SYM, bool OUTER>
 static void launch_inner(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int KC = inner_group(p);
-    if (KC == 4) launch_inner_kc<KS, SYM, 4>(p, d, s);
-    else if (KC == 2) launch_inner_kc<KS, SYM, 2>(p, d, s);
-    else launch_inner_kc<KS, SYM, 1>(p, d, s);
+    if (KC == 4) launch_inner_kc<KS, SYM, 4, OUTER>(p, d, s);
+    else if (KC == 2) launch_inner_kc<KS, SYM, 2, OUTER>(p, d, s);
+    else launch_inner_kc<KS, SYM, 1, OUTER>(p, d, s);
 }
 
 template <int KS>
 static void launch_inner_sym(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    launch_inner<KS, true>(p, d, s);
+    launch_inner<KS, true, false>(p, d, s);
 }
 
 template <int KS>
 static void launch_inner_plain(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    launch_inner<KS, false>(p, d, s);
+    launch_inner<KS, false, false>(p, d, s);
+}
+
+template <int KS>
+static void launch_inner_outer(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    launch_inner<KS, true, true>(p, d, s);
 }
 
 #define BS2E_ORDER_SWITCH(FN)                                                                                \
@@ -464,6 +488,12 @@ hipError_t launch_diag_cells(const Plan& p, const DevTables& d, hipStream_t s, b
     } else {
         BS2E_ORDER_SWITCH(launch_inner_plain)
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_moments_and_cells(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    BS2E_ORDER_SWITCH(launch_inner_outer)
     return hipGetLastError();
 }
 

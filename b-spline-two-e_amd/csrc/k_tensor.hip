@@ -27,8 +27,8 @@
 //         + sum_{w in W_p and W_q} Q_q(w) PP_p(w-1) + P_q(w) QS_p(w+1) + Dsym[w; p, q]
 //     (the general formula with PP_p = 0 left of W_p and Ptot_p right of it,
 //     QS_p = Qtot_p left of W_p and 0 right of it); the first two sums are
-//     q's own prefix / suffix sums.  It runs on a second stream, concurrently
-//     with k3_far.
+//     q's own prefix / suffix sums.  It runs beside k3_far: on a second
+//     stream, or for small tensors in one launch with it (k3_fill).
 #include <algorithm>
 
 #include "bs2e_internal.h"
@@ -71,17 +71,29 @@ __device__ __forceinline__ int pair_at(const int32_t* __restrict__ c_first, int 
 // pairs' indices found once per pair in LDS rather than once per element.
 // Alone, FOLD against every column with a search per element: 2944 pairs x 11
 // multipoles 0.038 -> 0.019 ms, 10128 x 25 0.284 -> 0.181 ms.
+struct NearArgs {
+    int n_pairs, n_b, n_iv, K, ks, U;
+    unsigned rK;
+    int n_rows;
+    const PairInfo* pairs;
+    const int32_t* c_first;
+    const int32_t* rows;
+    const double *Pw, *Qw, *PP, *QS, *Dsym;
+    double* R;
+};
+
+// near workgroup blk of A.n_rows
 template <bool FOLD>
-__global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int n_iv, int K, int ks, int U, unsigned rK,
-                                                    const PairInfo* __restrict__ pairs,
-                                                    const int32_t* __restrict__ c_first,
-                                                    const int32_t* __restrict__ rows,
-                                                    const double* __restrict__ Pw, const double* __restrict__ Qw,
-                                                    const double* __restrict__ PP, const double* __restrict__ QS,
-                                                    const double* __restrict__ Dsym, double* __restrict__ R)
+__device__ __forceinline__ void near_row(const NearArgs& A, unsigned blk, double* lds)
 {
     constexpr int kLanes = kNearMaxSeg;                    // one wavefront scans the runs
-    extern __shared__ __align__(16) double lds[];
+    const int n_pairs = A.n_pairs, n_b = A.n_b, n_iv = A.n_iv, K = A.K, ks = A.ks, U = A.U;
+    const unsigned rK = A.rK;
+    const PairInfo* __restrict__ pairs = A.pairs;
+    const int32_t* __restrict__ c_first = A.c_first;
+    const double *__restrict__ Pw = A.Pw, *__restrict__ Qw = A.Qw, *__restrict__ PP = A.PP, *__restrict__ QS = A.QS;
+    const double* __restrict__ Dsym = A.Dsym;
+    double* __restrict__ R = A.R;
     int4* sCol = (int4*)lds;                               // [(2 ks - 1)^2]: q, (d, b)'s pair or -1, min, max of b, d
     double* sPPx = lds + 2 * (2 * ks - 1) * (2 * ks - 1);  // [(ks+1)][K]
     double* sQSx = sPPx + (ks + 1) * K;                    // [(ks+1)][K]
@@ -89,7 +101,7 @@ __global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int n_
     int* sJ0 = sUp + kMaxOrder;                            // [kNearMaxSeg + 1]: first column pair of each spline d
     int* sB0 = sJ0 + kNearMaxSeg + 1;                      // [kNearMaxSeg]: its first b
     const int tid = threadIdx.x;
-    const int p = rows[xcd_block(blockIdx.x, gridDim.x)];   // neighbouring rows gather the same Dsym cells
+    const int p = A.rows[xcd_block(blk, A.n_rows)];         // neighbouring rows gather the same Dsym cells
     const PairInfo pp = pairs[p];
     const int lo = pp.v0, m = pp.m, hi = pp.v0 + pp.m - 1;
     const int pt = (pp.a == pp.c) ? -1 : pair_at(c_first, ks, pp.c, pp.a);   // the identical row (c, a)
@@ -183,6 +195,13 @@ __global__ __launch_bounds__(kThreads) void k3_near(int n_pairs, int n_b, int n_
     }
 }
 
+template <bool FOLD>
+__global__ __launch_bounds__(kThreads) void k3_near(NearArgs A)
+{
+    extern __shared__ __align__(16) double lds[];
+    near_row<FOLD>(A, blockIdx.x, lds);
+}
+
 // Far workgroups: ROWS rows x one chunk of 512 ITERS elements of rank-one
 // products, two consecutive elements per thread and 16-byte store; the
 // elements whose pairs' windows overlap are left to k3_near.
@@ -226,22 +245,35 @@ constexpr int kFarLd = kMaxK + 2;       // a row's factors in LDS, the first one
 constexpr unsigned kFarGridY = 32768;   // row groups per grid layer
 constexpr int64_t kFarSliceBytes = (int64_t)2 << 20;   // factor tables beyond which the XCDs take slices
 
+struct FarArgs {
+    int n_pairs, n_b, K, ks;
+    unsigned rK, rK1;
+    int far_cols, x_cols;
+    const PairInfo* pairs;
+    const int32_t* c_first;
+    const double *Ptot, *Qtot;
+    double* R;
+};
+
+// far workgroup of row group grp and chunk column bx of the launch
 template <int ROWS, int ITERS, bool SHIFT>
-__global__ __launch_bounds__(kThreads) void k3_far(int n_pairs, int n_b, int K, int ks, unsigned rK, unsigned rK1,
-                                                   int far_cols, int x_cols, const PairInfo* __restrict__ pairs,
-                                                   const int32_t* __restrict__ c_first,
-                                                   const double* __restrict__ Ptot,
-                                                   const double* __restrict__ Qtot, double* __restrict__ R)
+__device__ __forceinline__ void far_chunk(const FarArgs& A, int grp, unsigned bx)
 {
     constexpr int CH = 2 * kThreads * ITERS, NF = SHIFT ? ROWS : 1;
     __shared__ double sP[ROWS * kFarLd], sQ[ROWS * kFarLd];   // Ptot, Qtot of the rows
+    const int n_pairs = A.n_pairs, n_b = A.n_b, K = A.K, ks = A.ks;
+    const unsigned rK = A.rK, rK1 = A.rK1;
+    const PairInfo* __restrict__ pairs = A.pairs;
+    const int32_t* __restrict__ c_first = A.c_first;
+    const double *__restrict__ Ptot = A.Ptot, *__restrict__ Qtot = A.Qtot;
+    double* __restrict__ R = A.R;
     const int tid = threadIdx.x;
     const int rowlen = n_pairs * K;        // < 2^31 (checked on the host)
-    const int p0 = (int)(blockIdx.z * kFarGridY + blockIdx.y) * ROWS;
+    const int p0 = grp * ROWS;
     if (p0 >= n_pairs) return;             // (the last grid layer can be short)
     const int nrows = (n_pairs - p0) < ROWS ? (n_pairs - p0) : ROWS;
-    const int cx = x_cols ? (int)(blockIdx.x % kXcds) * x_cols + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
-    if (cx >= far_cols) return;            // (the last XCD's slice can be short)
+    const int cx = A.x_cols ? (int)(bx % kXcds) * A.x_cols + (int)(bx / kXcds) : (int)bx;
+    if (cx >= A.far_cols) return;          // (the last XCD's slice can be short)
     const int e0 = cx * CH;
     const unsigned uK = (unsigned)K;
     int lo[ROWS], hi[ROWS], shift[ROWS];   // uniform: scalar registers
@@ -340,6 +372,27 @@ __global__ __launch_bounds__(kThreads) void k3_far(int n_pairs, int n_b, int K, 
     }
 }
 
+template <int ROWS, int ITERS, bool SHIFT>
+__global__ __launch_bounds__(kThreads) void k3_far(FarArgs A)
+{
+    far_chunk<ROWS, ITERS, SHIFT>(A, (int)(blockIdx.z * kFarGridY + blockIdx.y), blockIdx.x);
+}
+
+// Both in one launch: the first near_y layers of workgroups take the near
+// rows, the others the rank-one fill.
+template <int ROWS, int ITERS, bool SHIFT, bool FOLD>
+__global__ __launch_bounds__(kThreads) void k3_fill(FarArgs A, NearArgs N, unsigned near_y)
+{
+    extern __shared__ __align__(16) double lds[];
+    const unsigned y = blockIdx.z * kFarGridY + blockIdx.y;
+    if (y < near_y) {
+        const unsigned blk = y * gridDim.x + blockIdx.x;
+        if (blk < (unsigned)N.n_rows) near_row<FOLD>(N, blk, lds);
+    } else {
+        far_chunk<ROWS, ITERS, SHIFT>(A, (int)(y - near_y), blockIdx.x);
+    }
+}
+
 // The store ceiling the rank-one fill is measured against: zeros over n16
 // 16-byte elements, one store per thread (NT: with the non-temporal hint),
 // the write pattern that reached the highest rate among those timed (more
@@ -409,13 +462,18 @@ int64_t count_near_elements(const Plan& p)
     return n;
 }
 
+static NearArgs near_args(const Plan& p, const DevTables& d, double* R)
+{
+    return NearArgs{(int)p.n_pairs, (int)p.n_b, (int)p.n_iv, (int)p.K, (int)p.k_s, (int)p.U, recip32(p.K),
+                    (int)p.rows.size(), d.pairs, d.c_first, d.rows, d.Pw, d.Qw, d.PP, d.QS, d.D, R};
+}
+
 hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s)
 {
     if (p.rows.empty()) return hipSuccess;
     const auto kern = symmetric ? k3_near<true> : k3_near<false>;
     hipLaunchKernelGGL(kern, dim3((unsigned)p.rows.size()), dim3(kThreads), near_lds_bytes(p.k_s, p.K), s,
-                       (int)p.n_pairs, (int)p.n_b, (int)p.n_iv, (int)p.K, (int)p.k_s, (int)p.U, recip32(p.K), d.pairs,
-                       d.c_first, d.rows, d.Pw, d.Qw, d.PP, d.QS, d.D, R);
+                       near_args(p, d, R));
     return hipGetLastError();
 }
 
@@ -442,35 +500,56 @@ bool far_variant_valid(const Plan& p, int v)
 // 10128 x 25 (lines) 3.26 against 3.24; of 4444 x 17 0.534 against 0.463.
 int far_variant_default(const Plan& p) { return (p.n_pairs * p.K) % kFarLine == 0 ? 0 : 5; }
 
+// The rank-one fill alone (near < 0), or behind the near rows in one launch
+// (near: whether the moments are symmetric).
 template <int V>
-static void launch_far_shape(const Plan& p, const DevTables& d, double* R, hipStream_t s)
+static void launch_far_shape(const Plan& p, const DevTables& d, double* R, int near, hipStream_t s)
 {
     constexpr FarShape f = kFarShapes[V];
     const int64_t rowlen = p.n_pairs * p.K;
     const int64_t per = 2 * (int64_t)kThreads * f.iters;
     // (a shifted row's last elements lie up to 15 past its last chunk)
     const unsigned cols = (unsigned)((rowlen + (f.shift ? kFarLine - 1 : 0) + per - 1) / per);
-    const unsigned rows = (unsigned)((p.n_pairs + f.rows - 1) / f.rows);
     const unsigned x_cols = 2 * sizeof(double) * rowlen > kFarSliceBytes ? (cols + kXcds - 1) / kXcds : 0;
-    const dim3 grid(x_cols ? kXcds * x_cols : cols, std::min(rows, kFarGridY), (rows + kFarGridY - 1) / kFarGridY);
-    hipLaunchKernelGGL((k3_far<f.rows, f.iters, f.shift>), grid, dim3(kThreads), 0, s, (int)p.n_pairs, (int)p.n_b,
-                       (int)p.K, (int)p.k_s, recip32(p.K), recip32(p.K + 1), (int)cols, (int)x_cols, d.pairs,
-                       d.c_first, d.Ptot, d.Qtot, R);
+    const unsigned gx = x_cols ? kXcds * x_cols : cols;
+    const unsigned near_y = near >= 0 ? (unsigned)((p.rows.size() + gx - 1) / gx) : 0;
+    const unsigned gy = (unsigned)((p.n_pairs + f.rows - 1) / f.rows) + near_y;
+    const dim3 grid(gx, std::min(gy, kFarGridY), (gy + kFarGridY - 1) / kFarGridY);
+    const FarArgs a{(int)p.n_pairs, (int)p.n_b, (int)p.K, (int)p.k_s, recip32(p.K), recip32(p.K + 1), (int)cols,
+                    (int)x_cols, d.pairs, d.c_first, d.Ptot, d.Qtot, R};
+    if (near < 0)
+        hipLaunchKernelGGL((k3_far<f.rows, f.iters, f.shift>), grid, dim3(kThreads), 0, s, a);
+    else if (near > 0)
+        hipLaunchKernelGGL((k3_fill<f.rows, f.iters, f.shift, true>), grid, dim3(kThreads), near_lds_bytes(p.k_s, p.K), s,
+                           a, near_args(p, d, R), near_y);
+    else
+        hipLaunchKernelGGL((k3_fill<f.rows, f.iters, f.shift, false>), grid, dim3(kThreads), near_lds_bytes(p.k_s, p.K), s,
+                           a, near_args(p, d, R), near_y);
+}
+
+static hipError_t launch_far(const Plan& p, const DevTables& d, double* R, int near, hipStream_t s)
+{
+    const int v = far_variant_valid(p, p.far_variant) ? p.far_variant : far_variant_default(p);
+    switch (v) {
+    case 0: launch_far_shape<0>(p, d, R, near, s); break;
+    case 1: launch_far_shape<1>(p, d, R, near, s); break;
+    case 2: launch_far_shape<2>(p, d, R, near, s); break;
+    case 3: launch_far_shape<3>(p, d, R, near, s); break;
+    case 4: launch_far_shape<4>(p, d, R, near, s); break;
+    case 5: launch_far_shape<5>(p, d, R, near, s); break;
+    default: launch_far_shape<6>(p, d, R, near, s); break;
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_tensor_far(const Plan& p, const DevTables& d, double* R, hipStream_t s)
 {
-    const int v = far_variant_valid(p, p.far_variant) ? p.far_variant : far_variant_default(p);
-    switch (v) {
-    case 0: launch_far_shape<0>(p, d, R, s); break;
-    case 1: launch_far_shape<1>(p, d, R, s); break;
-    case 2: launch_far_shape<2>(p, d, R, s); break;
-    case 3: launch_far_shape<3>(p, d, R, s); break;
-    case 4: launch_far_shape<4>(p, d, R, s); break;
-    case 5: launch_far_shape<5>(p, d, R, s); break;
-    default: launch_far_shape<6>(p, d, R, s); break;
-    }
-    return hipGetLastError();
+    return launch_far(p, d, R, -1, s);
+}
+
+hipError_t launch_tensor_fill(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s)
+{
+    return launch_far(p, d, R, symmetric ? 1 : 0, s);
 }
 
 hipError_t launch_symmetrize(const Plan& p, const DevTables& d, hipStream_t s)

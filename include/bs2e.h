@@ -139,16 +139,18 @@ int64_t bs2e_rk_copy_rows(const bs2e_rk *rk, int64_t row_lo, int64_t n_rows, dou
  * outside |a-c| < k, |b-d| < k (the reference error-stops there). */
 int64_t bs2e_rk_get_val(const bs2e_rk *rk, const int64_t *indices, double *values, int64_t n_values);
 /* Device timeline of the builds computed while profiling is on (HIP events
- * on the build's two streams), in ms since each build's start, averaged over
+ * on the build's streams), in ms since each build's start, averaged over
  * the builds since profiling was switched on or since the previous
  * bs2e_rk_stage_times call: [0] local moments + pair windows done,
  * [1] rank-one fill done, [2] diagonal cells done (second stream), [3] near
- * elements done (second stream), [4] end of the build. */
+ * elements done (second stream), [4] end of the build.  A small tensor's build
+ * runs on one stream, the cells before the pair windows, the near elements and
+ * the fill in one launch ([1] = [3]). */
 int64_t bs2e_rk_set_profiling(bs2e_rk *rk, int64_t on);
 int64_t bs2e_rk_stage_times(bs2e_rk *rk, double *ms, int64_t n);
-/* on != 0: the next bs2e_rk_compute captures the build (both streams) into a
+/* on != 0: the next bs2e_rk_compute captures the build into a
  * hipGraph and every compute then launches that graph, with one launch call
- * instead of five kernels and the stream events; 0 drops the graph.  Not
+ * instead of its kernels and stream events; 0 drops the graph.  Not
  * combinable with profiling.  (No reference counterpart.) */
 int64_t bs2e_rk_set_graph(bs2e_rk *rk, int64_t on);
 /* Autotuner: times, on this handle's own tables, each shape of the rank-one
@@ -311,7 +313,7 @@ int64_t bs2e_blockset_row_counts(const bs2e_blockset *set, int64_t row_lo, int64
  * for.  (No reference counterpart.) */
 int64_t bs2e_blockset_refill(bs2e_blockset *set);
 /* on != 0: captures the whole branch of the set into one hipGraph: its
- * tensor's two-stream build, the count pass, the device prefix sums of the
+ * tensor's build, the count pass, the device prefix sums of the
  * row counts, the fill's layouts and the fill over every symmetry and channel
  * (one-electron matrices of the last bs2e_blockset_fill, which must have
  * filled the whole set, not a window: BS2E_ESTATE otherwise); 0 drops it.  A
