@@ -35,7 +35,7 @@ int64_t bs2e_create(bs2e_ctx** out, int64_t device)
     if (device < 0 || device >= n) return fail(nullptr, BS2E_EINVAL, "bs2e_create: device index out of range");
     bs2e_ctx* c = new (std::nothrow) bs2e_ctx();
     if (!c) return fail(nullptr, BS2E_ENOMEM, "bs2e_create: host allocation failed");
-    c->device = (int)device;
+    c->device = c->pool.device = (int)device;
     e = hipSetDevice(c->device);
     // both streams at the default priority
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking);
@@ -58,6 +58,8 @@ static void ctx_free_now(bs2e_ctx* ctx)
             (void)hipStreamSynchronize(s);
             (void)hipStreamDestroy(s);
         }
+    ctx->copier.reset();
+    ctx->pool.trim(0);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->up) (void)hipHostFree(ctx->up);
     if (ctx->up_ev) (void)hipEventDestroy(ctx->up_ev);
@@ -212,6 +214,7 @@ size_t bs2e::Arena::largest_free() const
 // ---------------------------------------------------------------------------
 static void free_tables(bs2e_rk* rk)
 {
+    QuietScope quiet;
     DevTables& d = rk->d;
     ctx_free(rk->ctx, rk->small);   // knots, breakpoints, GL rule, pairs, near rows, c_first
     d.t = d.bp = d.x = d.w = nullptr;
@@ -493,9 +496,9 @@ int64_t bs2e_slater_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const 
         std::vector<void*> extra;
         ~Guard()
         {
+            QuietScope quiet;
             free_tables(h);
-            for (void* e : extra)
-                if (e) (void)hipFree(e);
+            for (void* e : extra) ctx_free(h->ctx, e);
         }
     } guard{&h, {}};
     rc = alloc_tables(ctx, &h, false);
@@ -504,38 +507,33 @@ int64_t bs2e_slater_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const 
     double *d_rk = nullptr, *d_rmk = nullptr, *d_rdk = nullptr;
     int64_t *d_i4 = nullptr, *d_i6 = nullptr, *d_off4 = nullptr;
     DiagEntry* d_diag = nullptr;
-    HIP_TRY(ctx, dev_alloc(&d_rk, (size_t)nnz4 * K));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_rk, (size_t)nnz4 * K));
     guard.extra.push_back(d_rk);
-    HIP_TRY(ctx, dev_alloc(&d_rmk, (size_t)nnz4 * K));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_rmk, (size_t)nnz4 * K));
     guard.extra.push_back(d_rmk);
-    HIP_TRY(ctx, dev_alloc(&d_i4, (size_t)nnz4 * 3));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_i4, (size_t)nnz4 * 3));
     guard.extra.push_back(d_i4);
-    HIP_TRY(ctx, dev_alloc(&d_off4, (size_t)p.n_pairs));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_off4, (size_t)p.n_pairs));
     guard.extra.push_back(d_off4);
-    HIP_TRY(ctx, dev_alloc(&d_rdk, (size_t)nnz6 * K));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_rdk, (size_t)nnz6 * K));
     guard.extra.push_back(d_rdk);
-    HIP_TRY(ctx, dev_alloc(&d_i6, (size_t)nnz6 * 5));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_i6, (size_t)nnz6 * 5));
     guard.extra.push_back(d_i6);
-    HIP_TRY(ctx, dev_alloc(&d_diag, p.diag.size()));
+    HIP_TRY(ctx, ctx_alloc(ctx, &d_diag, p.diag.size()));
     guard.extra.push_back(d_diag);
     hipStream_t s = ctx->stream;
-    HIP_TRY(ctx, hipMemcpyAsync(d_off4, p.off4.data(), sizeof(int64_t) * p.n_pairs, hipMemcpyHostToDevice, s));
-    HIP_TRY(ctx, hipMemcpyAsync(d_diag, p.diag.data(), sizeof(DiagEntry) * p.diag.size(), hipMemcpyHostToDevice, s));
+    HIP_TRY(ctx, copy_to_device(ctx, {{d_off4, p.off4.data(), sizeof(int64_t) * p.n_pairs},
+                                      {d_diag, p.diag.data(), sizeof(DiagEntry) * p.diag.size()}}));
     rc = run_primitives_serial(ctx, &h);
     if (rc) return rc;
     HIP_TRY(ctx, launch_scatter_4d(p, h.d, d_off4, d_rk, d_rmk, d_i4, d_i4 + nnz4, d_i4 + 2 * nnz4, s));
     HIP_TRY(ctx, launch_scatter_6d(p, h.d, d_diag, (int64_t)p.diag.size(), d_rdk, d_i6, d_i6 + nnz6,
                                    d_i6 + 2 * nnz6, d_i6 + 3 * nnz6, d_i6 + 4 * nnz6, s));
-    HIP_TRY(ctx, hipMemcpyAsync(rk, d_rk, sizeof(double) * nnz4 * K, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipMemcpyAsync(rmk, d_rmk, sizeof(double) * nnz4 * K, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipMemcpyAsync(iv4, d_i4, sizeof(int64_t) * nnz4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipMemcpyAsync(i4, d_i4 + nnz4, sizeof(int64_t) * nnz4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipMemcpyAsync(j4, d_i4 + 2 * nnz4, sizeof(int64_t) * nnz4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipMemcpyAsync(rdk, d_rdk, sizeof(double) * nnz6 * K, hipMemcpyDeviceToHost, s));
-    int64_t* outs6[5] = {iv6, i6, ip6, j6, jp6};
-    for (int a = 0; a < 5; ++a)
-        HIP_TRY(ctx, hipMemcpyAsync(outs6[a], d_i6 + a * nnz6, sizeof(int64_t) * nnz6, hipMemcpyDeviceToHost, s));
-    HIP_TRY(ctx, hipStreamSynchronize(s));
+    const size_t b4 = sizeof(int64_t) * nnz4, b6 = sizeof(int64_t) * nnz6;   // one column of 8 bytes each
+    HIP_TRY(ctx, copy_to_host(ctx, {{rk, d_rk, b4 * K}, {rmk, d_rmk, b4 * K}, {iv4, d_i4, b4}, {i4, d_i4 + nnz4, b4},
+                                    {j4, d_i4 + 2 * nnz4, b4}, {rdk, d_rdk, b6 * K}, {iv6, d_i6, b6},
+                                    {i6, d_i6 + nnz6, b6}, {ip6, d_i6 + 2 * nnz6, b6}, {j6, d_i6 + 3 * nnz6, b6},
+                                    {jp6, d_i6 + 4 * nnz6, b6}}));
     return BS2E_OK;
 }
 
@@ -617,8 +615,8 @@ int64_t bs2e_rk_from_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const
     const int64_t K = p.K;
     std::vector<void*> tmp;
     auto cleanup = [&]() {
-        for (void* e : tmp)
-            if (e) (void)hipFree(e);
+        QuietScope quiet;
+        for (void*& e : tmp) ctx_free(ctx, e);
     };
     auto bail = [&](int64_t code) {
         cleanup();
@@ -637,33 +635,27 @@ int64_t bs2e_rk_from_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const
     int64_t *d_i4 = nullptr, *d_i6 = nullptr;
     int32_t* d_cf = nullptr;
     int* d_bad = nullptr;
-    STEP(dev_alloc(&d_rk, (size_t)nnz4 * K));
+    STEP(ctx_alloc(ctx, &d_rk, (size_t)nnz4 * K));
     tmp.push_back(d_rk);
-    STEP(dev_alloc(&d_rmk, (size_t)nnz4 * K));
+    STEP(ctx_alloc(ctx, &d_rmk, (size_t)nnz4 * K));
     tmp.push_back(d_rmk);
-    STEP(dev_alloc(&d_i4, (size_t)nnz4 * 3));
+    STEP(ctx_alloc(ctx, &d_i4, (size_t)nnz4 * 3));
     tmp.push_back(d_i4);
-    STEP(dev_alloc(&d_rdk, (size_t)nnz6 * K));
+    STEP(ctx_alloc(ctx, &d_rdk, (size_t)nnz6 * K));
     tmp.push_back(d_rdk);
-    STEP(dev_alloc(&d_i6, (size_t)nnz6 * 5));
+    STEP(ctx_alloc(ctx, &d_i6, (size_t)nnz6 * 5));
     tmp.push_back(d_i6);
-    STEP(dev_alloc(&d_cf, p.c_first.size()));
+    STEP(ctx_alloc(ctx, &d_cf, p.c_first.size()));
     tmp.push_back(d_cf);
-    STEP(dev_alloc(&d_bad, 1));
+    STEP(ctx_alloc(ctx, &d_bad, 1));
     tmp.push_back(d_bad);
     hipStream_t s = ctx->stream;
-    STEP(hipMemcpyAsync(d_rk, rk4, sizeof(double) * nnz4 * K, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_rmk, rmk, sizeof(double) * nnz4 * K, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_i4, iv4, sizeof(int64_t) * nnz4, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_i4 + nnz4, i4, sizeof(int64_t) * nnz4, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_i4 + 2 * nnz4, j4, sizeof(int64_t) * nnz4, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_rdk, rdk, sizeof(double) * nnz6 * K, hipMemcpyHostToDevice, s));
-    const int64_t* in6[5] = {iv6, i6, ip6, j6, jp6};
-    for (int a = 0; a < 5; ++a)
-        STEP(hipMemcpyAsync(d_i6 + a * nnz6, in6[a], sizeof(int64_t) * nnz6, hipMemcpyHostToDevice, s));
-    STEP(hipMemcpyAsync(d_cf, p.c_first.data(), sizeof(int32_t) * p.c_first.size(), hipMemcpyHostToDevice, s));
+    const size_t b4 = sizeof(int64_t) * nnz4, b6 = sizeof(int64_t) * nnz6;   // one column of 8 bytes each
     const int zero = 0;
-    STEP(hipMemcpyAsync(d_bad, &zero, sizeof(int), hipMemcpyHostToDevice, s));
+    STEP(copy_to_device(ctx, {{d_rk, rk4, b4 * K}, {d_rmk, rmk, b4 * K}, {d_i4, iv4, b4}, {d_i4 + nnz4, i4, b4},
+                              {d_i4 + 2 * nnz4, j4, b4}, {d_rdk, rdk, b6 * K}, {d_i6, iv6, b6}, {d_i6 + nnz6, i6, b6},
+                              {d_i6 + 2 * nnz6, ip6, b6}, {d_i6 + 3 * nnz6, j6, b6}, {d_i6 + 4 * nnz6, jp6, b6},
+                              {d_cf, p.c_first.data(), sizeof(int32_t) * p.c_first.size()}, {d_bad, &zero, sizeof(int)}}));
     const size_t slots = (size_t)p.n_pairs * p.k_s * p.K;
     clear_stale_error();
     STEP(launch_fill(rk->d.Pw, (int64_t)slots, 0.0, s));
@@ -935,15 +927,15 @@ int64_t bs2e_rk_copy_to_host(bs2e_rk* rk, double* dst, int64_t n_elems)
     if (dst && n_elems != (int64_t)rk->R_elems)
         return fail(ctx, BS2E_EINVAL, "bs2e_rk_copy_to_host: n_elems differs from the tensor size");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    try {
-        rk->mirror.resize(rk->R_elems);
-    } catch (...) {
-        return fail(ctx, BS2E_ENOMEM, "bs2e_rk_copy_to_host: host mirror allocation failed");
-    }
-    HIP_TRY(ctx, hipMemcpy(rk->mirror.data(), rk->R, sizeof(double) * rk->R_elems, hipMemcpyDeviceToHost));
+    const size_t bytes = sizeof(double) * rk->R_elems;
+    if (!rk->mirror) rk->mirror.reset(new (std::nothrow) double[rk->R_elems]);
+    if (!rk->mirror) return fail(ctx, BS2E_ENOMEM, "bs2e_rk_copy_to_host: host mirror allocation failed");
+    HIP_TRY(ctx, copy_to_host(ctx, {{rk->mirror.get(), rk->R, bytes}}));
     rk->mirror_valid = true;
-    if (dst) std::memcpy(dst, rk->mirror.data(), sizeof(double) * rk->R_elems);
+    if (dst) {
+        if (HostCopier* h = ctx_copier(ctx)) h->copy(dst, rk->mirror.get(), bytes);
+        else std::memcpy(dst, rk->mirror.get(), bytes);
+    }
     return BS2E_OK;
 }
 
@@ -957,13 +949,11 @@ int64_t bs2e_rk_copy_rows(const bs2e_rk* rk, int64_t row_lo, int64_t n_rows, dou
     if (!rk->computed) return fail(ctx, BS2E_ESTATE, "bs2e_rk_copy_rows: tensor not computed");
     const size_t row = (size_t)p.n_pairs * p.K;
     if (rk->mirror_valid) {
-        std::memcpy(dst, rk->mirror.data() + (size_t)row_lo * row, sizeof(double) * row * (size_t)n_rows);
+        std::memcpy(dst, rk->mirror.get() + (size_t)row_lo * row, sizeof(double) * row * (size_t)n_rows);
         return BS2E_OK;
     }
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    HIP_TRY(ctx, hipMemcpy(dst, rk->R + (size_t)row_lo * row, sizeof(double) * row * (size_t)n_rows,
-                           hipMemcpyDeviceToHost));
+    HIP_TRY(ctx, copy_to_host(ctx, {{dst, rk->R + (size_t)row_lo * row, sizeof(double) * row * (size_t)n_rows}}));
     return BS2E_OK;
 }
 
@@ -982,7 +972,7 @@ int64_t bs2e_rk_get_val(const bs2e_rk* rk, const int64_t* idx, double* values, i
     }
     const size_t off = ((size_t)pa * p.n_pairs + pb) * p.K;
     if (rk->mirror_valid) {
-        std::memcpy(values, rk->mirror.data() + off, sizeof(double) * p.K);
+        std::memcpy(values, rk->mirror.get() + off, sizeof(double) * p.K);
         return BS2E_OK;
     }
     if (!rk->computed) return fail(rk->ctx, BS2E_ESTATE, "bs2e_rk_get_val: tensor not computed");

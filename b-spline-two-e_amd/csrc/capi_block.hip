@@ -168,6 +168,7 @@ struct bs2e_block : bs2e_blockset {};
 
 static void set_drop_graph(bs2e_blockset* b)
 {
+    QuietScope quiet;
     if (b->graph_exec) (void)hipGraphExecDestroy(b->graph_exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->graph_exec = nullptr;
@@ -180,6 +181,7 @@ static void set_drop_graph(bs2e_blockset* b)
 // when it has one (a build service's slot), else hipMalloc.
 static void set_drop_outputs(bs2e_blockset* b)
 {
+    QuietScope quiet;
     set_drop_graph(b);   // its nodes address these buffers
     bs2e_ctx* c = b->rk->ctx;
     ctx_free(c, b->d_Hl);
@@ -195,6 +197,7 @@ static void set_drop_outputs(bs2e_blockset* b)
 
 static void set_free(bs2e_blockset* b)
 {
+    QuietScope quiet;
     bs2e_ctx* c = b->rk->ctx;
     set_drop_outputs(b);
     ctx_free(c, b->d_cfg);
@@ -535,6 +538,7 @@ int64_t bs2e::set_fill_alloc(bs2e_blockset* b, int64_t n_l, const char* who)
     const size_t nn = (size_t)p.n_b * p.n_b;
     const size_t nf = (size_t)p.n_pairs * p.K;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
+    QuietScope quiet;
     set_drop_graph(b);   // its nodes address the buffers reallocated here
     ctx_free(ctx, b->d_T);
     ctx_free(ctx, b->d_ixH);
@@ -632,9 +636,8 @@ static int64_t set_fill(bs2e_blockset* b, int64_t max_l_1p, const double* Hl, co
     set_drop_outputs(b);
     HIP_TRY(ctx, ctx_alloc(ctx, &b->d_Hl, 2 * nn * (size_t)(max_l_1p + 1)));
     HIP_TRY(ctx, ctx_alloc(ctx, &b->d_S, 2 * nn));
-    hipStream_t st = ctx->stream;
-    HIP_TRY(ctx, hipMemcpyAsync(b->d_Hl, Hl, sizeof(double) * 2 * nn * (max_l_1p + 1), hipMemcpyHostToDevice, st));
-    HIP_TRY(ctx, hipMemcpyAsync(b->d_S, S, sizeof(double) * 2 * nn, hipMemcpyHostToDevice, st));
+    HIP_TRY(ctx, copy_to_device(ctx, {{b->d_Hl, Hl, sizeof(double) * 2 * nn * (size_t)(max_l_1p + 1)},
+                                      {b->d_S, S, sizeof(double) * 2 * nn}}));
     return set_fill_device(b, max_l_1p + 1, b->d_Hl, b->d_S, true, who);
 }
 
@@ -650,18 +653,12 @@ static int64_t set_get(const bs2e_blockset* b, int64_t s, int64_t* ip_H, int64_t
     if (b->row0[s] < b->win_lo || b->row0[s + 1] > b->win_lo + b->win_n)
         return fail(ctx, BS2E_ESTATE, std::string(who) + ": the filled row window does not hold the whole symmetry");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
     const int64_t nH = b->nnzH[s], nS = b->nnzS[s];
     const int64_t aH = b->offH[s] - b->winH, aS = b->offS[s] - b->winS;   // within the outputs
-    if (nH > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(ix_H, b->d_ixH + aH, sizeof(int64_t) * nH, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(d_H, b->d_dH + 2 * aH, sizeof(double) * 2 * nH, hipMemcpyDeviceToHost, st));
-    }
-    if (nS > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(ix_S, b->d_ixS + aS, sizeof(int64_t) * nS, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(d_S, b->d_dS + 2 * aS, sizeof(double) * 2 * nS, hipMemcpyDeviceToHost, st));
-    }
-    HIP_TRY(ctx, hipStreamSynchronize(st));
+    HIP_TRY(ctx, copy_to_host(ctx, {{ix_H, b->d_ixH + aH, sizeof(int64_t) * (size_t)nH},
+                                    {d_H, b->d_dH + 2 * aH, sizeof(double) * 2 * (size_t)nH},
+                                    {ix_S, b->d_ixS + aS, sizeof(int64_t) * (size_t)nS},
+                                    {d_S, b->d_dS + 2 * aS, sizeof(double) * 2 * (size_t)nS}}));
     ip_H[0] = 1;
     ip_S[0] = 1;
     const int64_t r0 = b->row0[s], n = b->row0[s + 1] - r0;
@@ -864,17 +861,11 @@ int64_t bs2e_blockset_get_rows(const bs2e_blockset* b, int64_t sym, int64_t row_
         return fail(ctx, BS2E_ESTATE, "bs2e_blockset_get_rows: rows outside the filled row window");
     const int64_t aH = b->prefH[g] - b->winH, aS = b->prefS[g] - b->winS;   // first entry within the outputs
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
     const int64_t nH = ip_H[n_rows] - 1, nS = ip_S[n_rows] - 1;
-    if (nH > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(ix_H, b->d_ixH + aH, sizeof(int64_t) * nH, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(d_H, b->d_dH + 2 * aH, sizeof(double) * 2 * nH, hipMemcpyDeviceToHost, st));
-    }
-    if (nS > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(ix_S, b->d_ixS + aS, sizeof(int64_t) * nS, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(d_S, b->d_dS + 2 * aS, sizeof(double) * 2 * nS, hipMemcpyDeviceToHost, st));
-    }
-    HIP_TRY(ctx, hipStreamSynchronize(st));
+    HIP_TRY(ctx, copy_to_host(ctx, {{ix_H, b->d_ixH + aH, sizeof(int64_t) * (size_t)nH},
+                                    {d_H, b->d_dH + 2 * aH, sizeof(double) * 2 * (size_t)nH},
+                                    {ix_S, b->d_ixS + aS, sizeof(int64_t) * (size_t)nS},
+                                    {d_S, b->d_dS + 2 * aS, sizeof(double) * 2 * (size_t)nS}}));
     return BS2E_OK;
 }
 
@@ -895,6 +886,7 @@ int64_t bs2e_blockset_row_counts(const bs2e_blockset* b, int64_t row_lo, int64_t
 // contents dropped) only when smaller.
 static int64_t set_reserve(bs2e_blockset* b, int64_t nH, int64_t nS)
 {
+    QuietScope quiet;
     bs2e_ctx* ctx = b->rk->ctx;
     if (nH > b->capH || !b->d_ixH) {
         set_drop_graph(b);
@@ -946,16 +938,16 @@ int64_t bs2e_blockset_fill_rows(bs2e_blockset* b, int64_t max_l_1p, const double
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     set_drop_graph(b);   // its fill addresses the whole set's outputs
     b->filled = false;
-    hipStream_t st = ctx->stream;
     if (Hl) {
+        QuietScope quiet;
         ctx_free(ctx, b->d_Hl);
         ctx_free(ctx, b->d_S);
         ctx_free(ctx, b->d_T);
         b->n_l = max_l_1p + 1;
         HIP_TRY(ctx, ctx_alloc(ctx, &b->d_Hl, 2 * nn * (size_t)b->n_l));
         HIP_TRY(ctx, ctx_alloc(ctx, &b->d_S, 2 * nn));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_Hl, Hl, sizeof(double) * 2 * nn * b->n_l, hipMemcpyHostToDevice, st));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_S, S, sizeof(double) * 2 * nn, hipMemcpyHostToDevice, st));
+        HIP_TRY(ctx, copy_to_device(ctx, {{b->d_Hl, Hl, sizeof(double) * 2 * nn * (size_t)b->n_l},
+                                          {b->d_S, S, sizeof(double) * 2 * nn}}));
     }
     if (!b->d_T) HIP_TRY(ctx, ctx_alloc(ctx, &b->d_T, 2 * nn * (size_t)(b->n_l + 1) + 2 * nf));
     // the outputs grow to the window (kept when they already hold it)

@@ -34,13 +34,14 @@ struct bs2e_dip {
 
 static void dip_free(bs2e_dip* b)
 {
-    dev_free(b->d_cfg1);
-    dev_free(b->d_cfg_chan1);
-    dev_free(b->d_chan2);
-    dev_free(b->d_seg2);
-    dev_free(b->d_coef);
-    dev_free(b->d_cnt);
-    dev_free(b->d_ptr);
+    QuietScope quiet;
+    ctx_free(b->ctx, b->d_cfg1);
+    ctx_free(b->ctx, b->d_cfg_chan1);
+    ctx_free(b->ctx, b->d_chan2);
+    ctx_free(b->ctx, b->d_seg2);
+    ctx_free(b->ctx, b->d_coef);
+    ctx_free(b->ctx, b->d_cnt);
+    ctx_free(b->ctx, b->d_ptr);
 }
 
 // mat_els.f90:739-770 dip_red_mat and :811-828 ang_dip_red, per (row channel
@@ -124,36 +125,34 @@ int64_t bs2e_setup_radial_dip(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const d
     DevTables d;
     double *B = nullptr, *B1 = nullptr, *rw = nullptr, *dM1 = nullptr, *dM2 = nullptr;
     auto cleanup = [&]() {
-        dev_free(d.t);
-        dev_free(d.bp);
-        dev_free(d.x);
-        dev_free(d.w);
-        dev_free(B);
-        dev_free(B1);
-        dev_free(rw);
-        dev_free(dM1);
-        dev_free(dM2);
+        QuietScope quiet;
+        ctx_free(ctx, d.t);
+        ctx_free(ctx, d.bp);
+        ctx_free(ctx, d.x);
+        ctx_free(ctx, d.w);
+        ctx_free(ctx, B);
+        ctx_free(ctx, B1);
+        ctx_free(ctx, rw);
+        ctx_free(ctx, dM1);
+        ctx_free(ctx, dM2);
     };
     auto run = [&]() -> int64_t {
-        HIP_TRY(ctx, dev_alloc(&d.t, p.n_knots));
-        HIP_TRY(ctx, dev_alloc(&d.bp, p.n_iv + 1));
-        HIP_TRY(ctx, dev_alloc(&d.x, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&d.w, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&B, tab));
-        HIP_TRY(ctx, dev_alloc(&B1, tab));
-        HIP_TRY(ctx, dev_alloc(&rw, 2 * (size_t)p.n_iv * p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&dM1, 2 * nn));
-        if (gauge == 1) HIP_TRY(ctx, dev_alloc(&dM2, 2 * nn));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.t, p.n_knots));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.bp, p.n_iv + 1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.x, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.w, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B1, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &rw, 2 * (size_t)p.n_iv * p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dM1, 2 * nn));
+        if (gauge == 1) HIP_TRY(ctx, ctx_alloc(ctx, &dM2, 2 * nn));
         hipStream_t s = ctx->stream;
-        HIP_TRY(ctx, hipMemcpyAsync(d.t, p.t.data(), 8 * p.n_knots, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.bp, p.bp.data(), 8 * (p.n_iv + 1), hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.x, p.x.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.w, p.w.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx, copy_to_device(ctx, {{d.t, p.t.data(), 8 * (size_t)p.n_knots},
+                                          {d.bp, p.bp.data(), 8 * (size_t)(p.n_iv + 1)},
+                                          {d.x, p.x.data(), 8 * (size_t)p.k_gl}, {d.w, p.w.data(), 8 * (size_t)p.k_gl}}));
         clear_stale_error();
         HIP_TRY(ctx, launch_radial_dipole(p, d, B, B1, rw, (int)gauge, dM1, dM2, s));
-        HIP_TRY(ctx, hipMemcpyAsync(m1, dM1, 16 * nn, hipMemcpyDeviceToHost, s));
-        if (gauge == 1) HIP_TRY(ctx, hipMemcpyAsync(m2, dM2, 16 * nn, hipMemcpyDeviceToHost, s));
-        HIP_TRY(ctx, hipStreamSynchronize(s));
+        HIP_TRY(ctx, copy_to_host(ctx, {{m1, dM1, 16 * nn}, {m2, dM2, gauge == 1 ? 16 * nn : 0}}));
         return BS2E_OK;
     };
     const int64_t rc = run();
@@ -210,22 +209,19 @@ int64_t bs2e_dip_block_create(bs2e_ctx* ctx, int64_t k, int64_t n_b, int64_t L1,
             b->coef[i * nc2 + j] = dip_coef(L1, L2, b->chan1[i].l1, b->chan1[i].l2, b->chan2[j].l1, b->chan2[j].l2);
     auto run = [&]() -> int64_t {
         HIP_TRY(ctx, hipSetDevice(ctx->device));
-        HIP_TRY(ctx, dev_alloc(&b->d_cfg1, (size_t)5 * n1));
-        HIP_TRY(ctx, dev_alloc(&b->d_cfg_chan1, (size_t)n1));
-        HIP_TRY(ctx, dev_alloc(&b->d_chan2, nc2));
-        HIP_TRY(ctx, dev_alloc(&b->d_seg2, b->seg2.size()));
-        HIP_TRY(ctx, dev_alloc(&b->d_coef, b->coef.size()));
-        HIP_TRY(ctx, dev_alloc(&b->d_cnt, (size_t)n1));
-        HIP_TRY(ctx, dev_alloc(&b->d_ptr, (size_t)n1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_cfg1, (size_t)5 * n1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_cfg_chan1, (size_t)n1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_chan2, nc2));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_seg2, b->seg2.size()));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_coef, b->coef.size()));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_cnt, (size_t)n1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &b->d_ptr, (size_t)n1));
         hipStream_t s = ctx->stream;
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_cfg1, cf1, sizeof(int64_t) * 5 * n1, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_cfg_chan1, b->cfg_chan1.data(), sizeof(int32_t) * n1, hipMemcpyHostToDevice,
-                                    s));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_chan2, b->chan2.data(), sizeof(BlockChan) * nc2, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_seg2, b->seg2.data(), sizeof(BlockSeg) * b->seg2.size(),
-                                    hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(b->d_coef, b->coef.data(), sizeof(DipCoef) * b->coef.size(),
-                                    hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx, copy_to_device(ctx, {{b->d_cfg1, cf1, sizeof(int64_t) * 5 * (size_t)n1},
+                                          {b->d_cfg_chan1, b->cfg_chan1.data(), sizeof(int32_t) * (size_t)n1},
+                                          {b->d_chan2, b->chan2.data(), sizeof(BlockChan) * nc2},
+                                          {b->d_seg2, b->seg2.data(), sizeof(BlockSeg) * b->seg2.size()},
+                                          {b->d_coef, b->coef.data(), sizeof(DipCoef) * b->coef.size()}}));
         clear_stale_error();
         DipArgs a = dip_args(b);
         a.cnt = b->d_cnt;
@@ -292,25 +288,24 @@ int64_t bs2e_dip_block_fill(bs2e_dip* b, int64_t gauge, const double* S, const d
     double *dS = nullptr, *dR1 = nullptr, *dR2 = nullptr, *dd = nullptr, *dT = nullptr;
     int64_t* dix = nullptr;
     auto cleanup = [&]() {
-        dev_free(dT);
-        dev_free(dS);
-        dev_free(dR1);
-        dev_free(dR2);
-        dev_free(dd);
-        dev_free(dix);
+        QuietScope quiet;
+        ctx_free(ctx, dT);
+        ctx_free(ctx, dS);
+        ctx_free(ctx, dR1);
+        ctx_free(ctx, dR2);
+        ctx_free(ctx, dd);
+        ctx_free(ctx, dix);
     };
     auto run = [&]() -> int64_t {
         HIP_TRY(ctx, hipSetDevice(ctx->device));
-        HIP_TRY(ctx, dev_alloc(&dS, 2 * nn));
-        HIP_TRY(ctx, dev_alloc(&dR1, 2 * nn));
-        if (gauge == 1) HIP_TRY(ctx, dev_alloc(&dR2, 2 * nn));
-        HIP_TRY(ctx, dev_alloc(&dT, 2 * nn * (gauge == 1 ? 3 : 2)));   // row-major S, rad1 (, rad2)
-        HIP_TRY(ctx, dev_alloc(&dd, 2 * (size_t)b->nnz));
-        HIP_TRY(ctx, dev_alloc(&dix, (size_t)b->nnz));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dS, 2 * nn));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dR1, 2 * nn));
+        if (gauge == 1) HIP_TRY(ctx, ctx_alloc(ctx, &dR2, 2 * nn));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dT, 2 * nn * (gauge == 1 ? 3 : 2)));   // row-major S, rad1 (, rad2)
+        HIP_TRY(ctx, ctx_alloc(ctx, &dd, 2 * (size_t)b->nnz));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dix, (size_t)b->nnz));
         hipStream_t s = ctx->stream;
-        HIP_TRY(ctx, hipMemcpyAsync(dS, S, 16 * nn, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(dR1, rad1, 16 * nn, hipMemcpyHostToDevice, s));
-        if (gauge == 1) HIP_TRY(ctx, hipMemcpyAsync(dR2, rad2, 16 * nn, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx, copy_to_device(ctx, {{dS, S, 16 * nn}, {dR1, rad1, 16 * nn}, {dR2, rad2, gauge == 1 ? 16 * nn : 0}}));
         clear_stale_error();
         DipArgs a = dip_args(b);
         a.gauge = (int)gauge;
@@ -335,9 +330,7 @@ int64_t bs2e_dip_block_fill(bs2e_dip* b, int64_t gauge, const double* S, const d
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         HIP_TRY(ctx, le);
-        HIP_TRY(ctx, hipMemcpyAsync(ix, dix, sizeof(int64_t) * b->nnz, hipMemcpyDeviceToHost, s));
-        HIP_TRY(ctx, hipMemcpyAsync(data, dd, 16 * (size_t)b->nnz, hipMemcpyDeviceToHost, s));
-        HIP_TRY(ctx, hipStreamSynchronize(s));
+        HIP_TRY(ctx, copy_to_host(ctx, {{ix, dix, sizeof(int64_t) * (size_t)b->nnz}, {data, dd, 16 * (size_t)b->nnz}}));
         return BS2E_OK;
     };
     const int64_t rc = run();

@@ -2,9 +2,14 @@
 #pragma once
 
 #include <array>
+#include <condition_variable>
+#include <deque>
+#include <initializer_list>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/bs2e.h"
@@ -33,6 +38,86 @@ private:
     mutable std::mutex mu_;
 };
 
+// Device blocks of a context: a released block is kept for a later allocation
+// of about its size, because the driver clears what it hands out again (a
+// 0.76 GB tensor released and created: 25 ms, most of it the clearing).  At
+// most kMaxKept bytes and kMaxBlocks blocks are kept, the longest unused go
+// first; all of them go when an allocation fails and with the context.  A
+// release waits for the device, as hipFree does, once per QuietScope.
+class DevicePool {
+public:
+    hipError_t alloc(void** out, size_t bytes);
+    void release(void* p);
+    void trim(size_t keep);
+    int device = 0;
+
+private:
+    struct Kept {
+        void* ptr;
+        uint64_t stamp;
+    };
+    static constexpr size_t kMaxKept = (size_t)4 << 30, kMaxBlocks = 256;
+    std::mutex mu_;
+    std::map<void*, size_t> live_;
+    std::multimap<size_t, Kept> kept_;   // by size
+    size_t kept_bytes_ = 0;
+    uint64_t stamp_ = 0;
+};
+
+// Releases of the calling thread inside one scope wait for the device once.
+struct QuietScope {
+    QuietScope();
+    ~QuietScope();
+    QuietScope(const QuietScope&) = delete;
+};
+
+// One part of a copy between device memory and a caller's array.
+struct Piece {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+
+// Copies between the device and pageable memory through a ring of pinned
+// buffers, with several threads between the buffers and the caller's pages: a
+// fresh array's page faults, the clearing of its pages and the copy are what
+// bounds such a transfer (the bus carries 57 GB/s).  292 MB of CSR into fresh
+// arrays: one thread of the runtime 28 ms, so 10.1 ms (6.1 into touched ones);
+// with buffers of 2 MiB 15.4, of 4 MiB 12.0, with four threads 12.5.
+class HostCopier {
+public:
+    ~HostCopier();
+    // to_host: returns when every piece is in place; otherwise when the
+    // pieces have been read and their copies enqueued on s.
+    hipError_t transfer(const Piece* pieces, size_t n, bool to_host, hipStream_t s);
+    void copy(void* dst, const void* src, size_t bytes);   // host to host
+
+private:
+    static constexpr int kBufs = 8;
+    static constexpr size_t kMinBuf = (size_t)64 << 10, kMaxBuf = (size_t)8 << 20, kSlice = (size_t)256 << 10;
+    struct Slice {
+        void* dst;
+        const void* src;
+        size_t bytes;
+        int buf;
+    };
+    bool prepare(size_t total);
+    void drop_ring();
+    void run();
+    void spread(void* dst, const void* src, size_t bytes, int buf);
+    void wait_slices(int buf);
+    std::mutex call_mu_, mu_;
+    std::condition_variable work_, done_;
+    std::deque<Slice> queue_;
+    int pending_[kBufs] = {};
+    bool stop_ = false;
+    std::vector<std::thread> threads_;
+    char* pin_ = nullptr;
+    size_t buf_ = 0;
+    hipEvent_t ev_[kBufs] = {};
+    bool in_flight_[kBufs] = {};
+};
+
 }  // namespace bs2e
 
 struct bs2e_ctx {
@@ -44,6 +129,8 @@ struct bs2e_ctx {
     hipStream_t stream = nullptr;   // the build's stream (own, or the caller's)
     hipStream_t side = nullptr;     // diagonal cells + near ranges, concurrent with the rank-one fill
     std::string err;
+    bs2e::DevicePool pool;          // the context's device blocks (without an arena)
+    std::shared_ptr<bs2e::HostCopier> copier;   // made with the first copy (a service's contexts share one)
     // pinned host staging for per-row tables: a block set's tables on their
     // way up and its counts on their way back (grown by doubling, freed with
     // the context; pin_mu held while it is in use)
@@ -67,7 +154,7 @@ struct bs2e_rk {
     double* R = nullptr;
     size_t R_elems = 0;
     int64_t precision = BS2E_PREC_FP64;
-    std::vector<double> mirror;
+    std::unique_ptr<double[]> mirror;   // R_elems
     bool mirror_valid = false;
     bool profiling = false;
     // profiling: one set of 6 timing events per build since profiling was
@@ -105,39 +192,31 @@ void rk_attach(bs2e_ctx* ctx, bs2e_rk* rk);
 void rk_delete(bs2e_rk* rk);      // deletes the handle object, then drops its context reference
 int64_t rk_release_now(bs2e_rk* rk);
 
-template <class T>
-inline hipError_t dev_alloc(T** p, size_t n)
-{
-    *p = nullptr;
-    if (n == 0) n = 1;
-    return hipMalloc((void**)p, n * sizeof(T));
-}
-
-template <class T>
-inline void dev_free(T*& p)
-{
-    if (p) (void)hipFree(p);
-    p = nullptr;
-}
-
-// Allocation of a context's tensors: its arena when it has one.
+// Allocation of a context: its arena when it has one, else its kept blocks.
 template <class T>
 inline hipError_t ctx_alloc(bs2e_ctx* c, T** p, size_t n)
 {
-    if (c && c->arena) {
-        *p = (T*)c->arena->alloc((n ? n : 1) * sizeof(T));
+    const size_t bytes = (n ? n : 1) * sizeof(T);
+    if (c->arena) {
+        *p = (T*)c->arena->alloc(bytes);
         return *p ? hipSuccess : hipErrorOutOfMemory;
     }
-    return dev_alloc(p, n);
+    return c->pool.alloc((void**)p, bytes);
 }
 
 template <class T>
 inline void ctx_free(bs2e_ctx* c, T*& p)
 {
-    if (p && c && c->arena) c->arena->release(p);
-    else if (p) (void)hipFree(p);
+    if (p && c->arena) c->arena->release(p);
+    else if (p) c->pool.release(p);
     p = nullptr;
 }
+
+// Copies on the context's stream between its device memory and host arrays;
+// copy_to_host returns when they are done.
+hipError_t copy_to_host(bs2e_ctx* c, std::initializer_list<Piece> pieces);
+hipError_t copy_to_device(bs2e_ctx* c, std::initializer_list<Piece> pieces);
+HostCopier* ctx_copier(bs2e_ctx* c);   // nullptr: no memory for one
 
 // Device bytes a tensor build of this plan allocates (tables and tensor,
 // with the arena's alignment); the plan's near rows must be built.

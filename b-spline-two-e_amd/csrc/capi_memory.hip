@@ -1,0 +1,334 @@
+// capi_memory.hip -- a context's device blocks and its copies between device
+// memory and a caller's pageable arrays.
+#include <sched.h>
+
+#include <algorithm>
+#include <cstring>
+
+#include "capi_internal.h"
+
+namespace bs2e {
+
+// ---------------------------------------------------------------------------
+// device blocks
+// ---------------------------------------------------------------------------
+namespace {
+thread_local int t_quiet_depth = 0;
+thread_local bool t_quiet = false;   // the device was idle since the outermost scope began
+}  // namespace
+
+QuietScope::QuietScope() { ++t_quiet_depth; }
+QuietScope::~QuietScope()
+{
+    if (--t_quiet_depth == 0) t_quiet = false;
+}
+
+hipError_t DevicePool::alloc(void** out, size_t bytes)
+{
+    *out = nullptr;
+    const size_t need = (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        // the smallest kept block that holds it without wasting more than a quarter
+        auto it = kept_.lower_bound(need);
+        if (it != kept_.end() && it->first <= need + need / 4 + ((size_t)64 << 10)) {
+            *out = it->second.ptr;
+            live_[*out] = it->first;
+            kept_bytes_ -= it->first;
+            kept_.erase(it);
+            return hipSuccess;
+        }
+    }
+    hipError_t e = hipMalloc(out, need);
+    if (e == hipErrorOutOfMemory) {   // give everything back and try once more
+        (void)hipGetLastError();
+        trim(0);
+        e = hipMalloc(out, need);
+    }
+    if (e != hipSuccess) {
+        *out = nullptr;
+        return e;
+    }
+    std::lock_guard<std::mutex> lk(mu_);
+    live_[*out] = need;
+    return hipSuccess;
+}
+
+void DevicePool::release(void* p)
+{
+    if (!p) return;
+    // As hipFree would, wait for the device: kernels of any stream, the
+    // caller's own among them, may still read the block.
+    (void)hipSetDevice(device);
+    bool idle = t_quiet;
+    if (!idle) {
+        idle = hipDeviceSynchronize() == hipSuccess;
+        if (t_quiet_depth > 0) t_quiet = idle;
+    }
+    size_t size = 0;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto it = live_.find(p);
+        if (it != live_.end()) {
+            size = it->second;
+            live_.erase(it);
+        }
+        if (idle && size > 0 && size <= kMaxKept) {
+            kept_.emplace(size, Kept{p, ++stamp_});
+            kept_bytes_ += size;
+            p = nullptr;
+        }
+    }
+    if (p) (void)hipFree(p);
+    trim(kMaxKept);
+}
+
+void DevicePool::trim(size_t keep)
+{
+    for (;;) {
+        void* victim = nullptr;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (kept_bytes_ <= keep && kept_.size() <= kMaxBlocks) return;
+            if (kept_.empty()) return;
+            auto oldest = kept_.begin();
+            for (auto it = kept_.begin(); it != kept_.end(); ++it)
+                if (it->second.stamp < oldest->second.stamp) oldest = it;
+            victim = oldest->second.ptr;
+            kept_bytes_ -= oldest->first;
+            kept_.erase(oldest);
+        }
+        (void)hipFree(victim);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// copies to and from pageable memory
+// ---------------------------------------------------------------------------
+HostCopier::~HostCopier()
+{
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        stop_ = true;
+    }
+    work_.notify_all();
+    for (std::thread& t : threads_) t.join();
+    drop_ring();
+}
+
+void HostCopier::drop_ring()
+{
+    for (int b = 0; b < kBufs; ++b) {
+        if (ev_[b]) {
+            if (in_flight_[b]) (void)hipEventSynchronize(ev_[b]);
+            (void)hipEventDestroy(ev_[b]);
+        }
+        ev_[b] = nullptr;
+        in_flight_[b] = false;
+    }
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    buf_ = 0;
+}
+
+// kBufs pinned buffers, an eighth of the copy each (64 KiB to 8 MiB), and for
+// copies of some size the threads.
+bool HostCopier::prepare(size_t total)
+{
+    size_t want = kMinBuf;
+    while (want < kMaxBuf && want * kBufs < total) want *= 2;
+    if (want > buf_) {
+        drop_ring();
+        if (hipHostMalloc((void**)&pin_, want * kBufs, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            pin_ = nullptr;
+            return false;
+        }
+        buf_ = want;
+        for (int b = 0; b < kBufs; ++b)
+            if (hipEventCreateWithFlags(&ev_[b], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                ev_[b] = nullptr;
+                drop_ring();
+                return false;
+            }
+    }
+    if (threads_.empty() && total > kSlice) {
+        cpu_set_t set;
+        int n = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) / 2 : 1;
+        n = std::min(8, n);
+        try {
+            for (int i = 0; i < n; ++i) threads_.emplace_back([this] { run(); });
+        } catch (...) {   // fewer threads, or none: the caller copies
+        }
+    }
+    return true;
+}
+
+void HostCopier::run()
+{
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+        work_.wait(lk, [this] { return stop_ || !queue_.empty(); });
+        if (queue_.empty()) return;
+        const Slice s = queue_.front();
+        queue_.pop_front();
+        lk.unlock();
+        std::memcpy(s.dst, s.src, s.bytes);
+        lk.lock();
+        if (--pending_[s.buf] == 0) done_.notify_all();
+    }
+}
+
+// Copies src to dst in slices on the threads (counted for buffer buf), or here
+// when it is short or there are none.
+void HostCopier::spread(void* dst, const void* src, size_t bytes, int buf)
+{
+    if (threads_.empty() || bytes <= kSlice / 2) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+    {
+        std::unique_lock<std::mutex> lk(mu_);
+        for (size_t o = 0; o < bytes; o += kSlice) {
+            try {
+                queue_.push_back(Slice{(char*)dst + o, (const char*)src + o, std::min(kSlice, bytes - o), buf});
+            } catch (...) {   // no memory for the entry: the rest here
+                lk.unlock();
+                std::memcpy((char*)dst + o, (const char*)src + o, bytes - o);
+                break;
+            }
+            ++pending_[buf];
+        }
+    }
+    work_.notify_all();
+}
+
+void HostCopier::wait_slices(int buf)
+{
+    std::unique_lock<std::mutex> lk(mu_);
+    done_.wait(lk, [this, buf] { return pending_[buf] == 0; });
+}
+
+void HostCopier::copy(void* dst, const void* src, size_t bytes)
+{
+    std::lock_guard<std::mutex> call(call_mu_);
+    if (!prepare(bytes)) {
+        std::memcpy(dst, src, bytes);
+        return;
+    }
+    spread(dst, src, bytes, 0);
+    wait_slices(0);
+}
+
+hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hipStream_t s)
+{
+    std::lock_guard<std::mutex> call(call_mu_);
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) total += pieces[i].bytes;
+    if (total == 0) return to_host ? hipStreamSynchronize(s) : hipSuccess;
+    const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+    if (!prepare(total)) {
+        for (size_t i = 0; i < n; ++i)
+            if (pieces[i].bytes > 0) {
+                const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, kind, s);
+                if (e != hipSuccess) return e;
+            }
+        return hipStreamSynchronize(s);
+    }
+    struct Part {
+        void* dst;
+        const void* src;
+        size_t bytes;
+    };
+    constexpr int kParts = 16;
+    Part parts[kBufs][kParts];        // what each buffer holds
+    int n_parts[kBufs] = {};
+    size_t pi = 0, po = 0;            // next byte to issue
+    int64_t head = 0, tail = 0;       // buffers issued, buffers handed on
+    hipError_t e = hipSuccess;
+    while (e == hipSuccess && (pi < n || tail < head)) {
+        if (pi < n && head - tail < kBufs) {
+            const int b = (int)(head % kBufs);
+            wait_slices(b);
+            if (in_flight_[b]) {
+                e = hipEventSynchronize(ev_[b]);
+                in_flight_[b] = false;
+            }
+            char* const base = pin_ + (size_t)b * buf_;
+            size_t used = 0;
+            n_parts[b] = 0;
+            while (pi < n && used < buf_ && n_parts[b] < kParts) {
+                const Piece& p = pieces[pi];
+                const size_t m = std::min(p.bytes - po, buf_ - used);
+                if (m > 0) {
+                    char* const mine = base + used;
+                    char* const dst = (char*)p.dst + po;
+                    const char* const src = (const char*)p.src + po;
+                    if (to_host) {
+                        if (e == hipSuccess) e = hipMemcpyAsync(mine, src, m, kind, s);
+                    } else {
+                        spread(mine, src, m, b);
+                    }
+                    parts[b][n_parts[b]++] = Part{dst, mine, m};
+                    used += (m + 255) / 256 * 256;
+                    po += m;
+                }
+                if (po == p.bytes) {
+                    ++pi;
+                    po = 0;
+                }
+            }
+            if (!to_host) {
+                wait_slices(b);
+                for (int i = 0; i < n_parts[b] && e == hipSuccess; ++i)
+                    e = hipMemcpyAsync(parts[b][i].dst, parts[b][i].src, parts[b][i].bytes, kind, s);
+            }
+            if (e == hipSuccess) e = hipEventRecord(ev_[b], s);
+            in_flight_[b] = e == hipSuccess;
+            ++head;
+            if (!to_host) tail = head;   // (the buffer is free once its event has passed)
+            continue;
+        }
+        const int b = (int)(tail % kBufs);
+        e = hipEventSynchronize(ev_[b]);
+        in_flight_[b] = false;
+        if (e == hipSuccess)
+            for (int i = 0; i < n_parts[b]; ++i) spread(parts[b][i].dst, parts[b][i].src, parts[b][i].bytes, b);
+        ++tail;
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing reads or writes the buffers any more
+    if (to_host)
+        for (int b = 0; b < kBufs; ++b) wait_slices(b);
+    return e;
+}
+
+HostCopier* ctx_copier(bs2e_ctx* c)
+{
+    std::lock_guard<std::mutex> lk(c->up_mu);
+    if (!c->copier) {
+        try {
+            c->copier = std::make_shared<HostCopier>();
+        } catch (...) {
+            return nullptr;
+        }
+    }
+    return c->copier.get();
+}
+
+static hipError_t transfer(bs2e_ctx* c, std::initializer_list<Piece> pieces, bool to_host)
+{
+    if (HostCopier* h = ctx_copier(c)) return h->transfer(pieces.begin(), pieces.size(), to_host, c->stream);
+    for (const Piece& p : pieces)
+        if (p.bytes > 0) {
+            const hipError_t e = hipMemcpyAsync(p.dst, p.src, p.bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice,
+                                                c->stream);
+            if (e != hipSuccess) return e;
+        }
+    return hipStreamSynchronize(c->stream);
+}
+
+hipError_t copy_to_host(bs2e_ctx* c, std::initializer_list<Piece> pieces) { return transfer(c, pieces, true); }
+hipError_t copy_to_device(bs2e_ctx* c, std::initializer_list<Piece> pieces) { return transfer(c, pieces, false); }
+
+}  // namespace bs2e

@@ -27,37 +27,35 @@ static int64_t one_body(bs2e_ctx* ctx, const char* who, int64_t k, int64_t n_kno
     DevTables d;
     double *B = nullptr, *B2 = nullptr, *rw = nullptr, *dS = nullptr, *dH = nullptr;
     auto cleanup = [&]() {
-        dev_free(d.t);
-        dev_free(d.bp);
-        dev_free(d.x);
-        dev_free(d.w);
-        dev_free(B);
-        dev_free(B2);
-        dev_free(rw);
-        dev_free(dS);
-        dev_free(dH);
+        QuietScope quiet;
+        ctx_free(ctx, d.t);
+        ctx_free(ctx, d.bp);
+        ctx_free(ctx, d.x);
+        ctx_free(ctx, d.w);
+        ctx_free(ctx, B);
+        ctx_free(ctx, B2);
+        ctx_free(ctx, rw);
+        ctx_free(ctx, dS);
+        ctx_free(ctx, dH);
     };
     auto run = [&]() -> int64_t {
-        HIP_TRY(ctx, dev_alloc(&d.t, p.n_knots));
-        HIP_TRY(ctx, dev_alloc(&d.bp, p.n_iv + 1));
-        HIP_TRY(ctx, dev_alloc(&d.x, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&d.w, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&B, tab));
-        HIP_TRY(ctx, dev_alloc(&B2, tab));
-        HIP_TRY(ctx, dev_alloc(&rw, 2 * (size_t)p.n_iv * p.k_gl));
-        if (S_out) HIP_TRY(ctx, dev_alloc(&dS, 2 * nn));
-        if (H_out) HIP_TRY(ctx, dev_alloc(&dH, 2 * nn * n_l));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.t, p.n_knots));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.bp, p.n_iv + 1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.x, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.w, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B2, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &rw, 2 * (size_t)p.n_iv * p.k_gl));
+        if (S_out) HIP_TRY(ctx, ctx_alloc(ctx, &dS, 2 * nn));
+        if (H_out) HIP_TRY(ctx, ctx_alloc(ctx, &dH, 2 * nn * n_l));
         hipStream_t s = ctx->stream;
-        HIP_TRY(ctx, hipMemcpyAsync(d.t, p.t.data(), 8 * p.n_knots, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.bp, p.bp.data(), 8 * (p.n_iv + 1), hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.x, p.x.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.w, p.w.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx, copy_to_device(ctx, {{d.t, p.t.data(), 8 * (size_t)p.n_knots},
+                                          {d.bp, p.bp.data(), 8 * (size_t)(p.n_iv + 1)},
+                                          {d.x, p.x.data(), 8 * (size_t)p.k_gl}, {d.w, p.w.data(), 8 * (size_t)p.k_gl}}));
         clear_stale_error();
         HIP_TRY(ctx, launch_one_body(p, d, B, B2, rw, (int)l_min, n_l, (int)Z, (int)cap_order, cap_r0, eta_re, eta_im,
                                      dS, dH, s));
-        if (S_out) HIP_TRY(ctx, hipMemcpyAsync(S_out, dS, 16 * nn, hipMemcpyDeviceToHost, s));
-        if (H_out) HIP_TRY(ctx, hipMemcpyAsync(H_out, dH, 16 * nn * n_l, hipMemcpyDeviceToHost, s));
-        HIP_TRY(ctx, hipStreamSynchronize(s));
+        HIP_TRY(ctx, copy_to_host(ctx, {{S_out, dS, S_out ? 16 * nn : 0}, {H_out, dH, H_out ? 16 * nn * n_l : 0}}));
         return BS2E_OK;
     };
     const int64_t rc = run();
@@ -83,33 +81,32 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
     DevTables d;
     double *B = nullptr, *B2 = nullptr, *rw = nullptr, *dout = nullptr;
     auto cleanup = [&]() {
-        dev_free(d.t);
-        dev_free(d.bp);
-        dev_free(d.x);
-        dev_free(d.w);
-        dev_free(B);
-        dev_free(B2);
-        dev_free(rw);
-        dev_free(dout);
+        QuietScope quiet;
+        ctx_free(ctx, d.t);
+        ctx_free(ctx, d.bp);
+        ctx_free(ctx, d.x);
+        ctx_free(ctx, d.w);
+        ctx_free(ctx, B);
+        ctx_free(ctx, B2);
+        ctx_free(ctx, rw);
+        ctx_free(ctx, dout);
     };
     auto run = [&]() -> int64_t {
-        HIP_TRY(ctx, dev_alloc(&d.t, p.n_knots));
-        HIP_TRY(ctx, dev_alloc(&d.bp, p.n_iv + 1));
-        HIP_TRY(ctx, dev_alloc(&d.x, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&d.w, p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&B, tab));
-        HIP_TRY(ctx, dev_alloc(&B2, tab));
-        HIP_TRY(ctx, dev_alloc(&rw, 2 * (size_t)p.n_iv * p.k_gl));
-        HIP_TRY(ctx, dev_alloc(&dout, n_out));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.t, p.n_knots));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.bp, p.n_iv + 1));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.x, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.w, p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &B2, tab));
+        HIP_TRY(ctx, ctx_alloc(ctx, &rw, 2 * (size_t)p.n_iv * p.k_gl));
+        HIP_TRY(ctx, ctx_alloc(ctx, &dout, n_out));
         hipStream_t s = ctx->stream;
-        HIP_TRY(ctx, hipMemcpyAsync(d.t, p.t.data(), 8 * p.n_knots, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.bp, p.bp.data(), 8 * (p.n_iv + 1), hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.x, p.x.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
-        HIP_TRY(ctx, hipMemcpyAsync(d.w, p.w.data(), 8 * p.k_gl, hipMemcpyHostToDevice, s));
+        HIP_TRY(ctx, copy_to_device(ctx, {{d.t, p.t.data(), 8 * (size_t)p.n_knots},
+                                          {d.bp, p.bp.data(), 8 * (size_t)(p.n_iv + 1)},
+                                          {d.x, p.x.data(), 8 * (size_t)p.k_gl}, {d.w, p.w.data(), 8 * (size_t)p.k_gl}}));
         clear_stale_error();
         HIP_TRY(ctx, launch_rk_int(p, d, B, B2, rw, (int)max_k, r0, dout, s));
-        HIP_TRY(ctx, hipMemcpyAsync(out, dout, 8 * n_out, hipMemcpyDeviceToHost, s));
-        HIP_TRY(ctx, hipStreamSynchronize(s));
+        HIP_TRY(ctx, copy_to_host(ctx, {{out, dout, 8 * n_out}}));
         return BS2E_OK;
     };
     const int64_t rc = run();

@@ -475,6 +475,8 @@ int64_t bs2e_server_create(int64_t device, int64_t hbm_bytes, int64_t slots, bs2
         rc = bs2e_create(&c, device);
         if (rc) break;
         c->arena = &s->arena;
+        if (!s->slots.empty()) c->copier = s->slots.front()->copier;   // one set of copy threads and buffers
+        else (void)ctx_copier(c);
         s->slots.push_back(c);
         s->slot_job.push_back(-1);
     }

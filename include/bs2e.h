@@ -51,6 +51,10 @@ typedef struct bs2e_rk bs2e_rk;   /* one basis and its device-resident R^k tenso
 /* Creates a context on HIP device `device` with its own default-priority
  * stream.  (No reference counterpart: the reference runs on the host.) */
 int64_t bs2e_create(bs2e_ctx **ctx, int64_t device);
+/* A context keeps up to 4 GiB of the device memory its handles have released
+ * for later ones, and up to 64 MiB of pinned host memory and eight threads for
+ * copies of results to the host; bs2e_destroy gives all of it back, and an
+ * allocation that fails the kept device memory. */
 int64_t bs2e_destroy(bs2e_ctx *ctx);
 const char *bs2e_last_error(const bs2e_ctx *ctx);
 /* Runs the context's device work on `hip_stream` (a hipStream_t) instead of
