@@ -248,9 +248,9 @@ int64_t count_configs(int64_t L, int64_t term_pi, int64_t max_l_1p, int64_t n_b,
                       int64_t n_all_l, int64_t l_2_max, int64_t* out, int64_t cap);
 
 // Kernel launchers (each .hip file launches its own kernels).
-hipError_t launch_outer_moments(const Plan& p, const DevTables& d, hipStream_t s);           // Pl, Ql
+hipError_t launch_windows(const Plan& p, const DevTables& d, hipStream_t s);                 // Pw/Qw + sums
 hipError_t launch_diag_cells(const Plan& p, const DevTables& d, hipStream_t s, bool symmetrised);  // D / Dsym
-hipError_t launch_moments_and_cells(const Plan& p, const DevTables& d, hipStream_t s);              // Pl, Ql and Dsym in one launch
+hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, hipStream_t s);             // with Dsym in one launch
 hipError_t launch_symmetrize(const Plan& p, const DevTables& d, hipStream_t s);                    // D -> Dsym
 size_t near_lds_bytes(int64_t ks, int64_t K);
 constexpr int kNearMaxSeg = 64;   // column segments of one near row (<= 2k - 1 <= 39 for k <= 20)
@@ -258,7 +258,7 @@ constexpr int kNearMaxSeg = 64;   // column segments of one near row (<= 2k - 1 
 hipError_t launch_outer_moments_mixed(const Plan& p, const DevTables& d, hipStream_t s);
 bool mixed_supported(int64_t ks, int64_t kgl, int64_t K);   // order <= 16, k_GL <= 16
 size_t mixed_lds_bytes(int64_t ks, int64_t K);
-hipError_t launch_pair_windows(const Plan& p, const DevTables& d, hipStream_t s);            // Pw/Qw + sums
+hipError_t launch_pair_windows(const Plan& p, const DevTables& d, hipStream_t s);            // Pw/Qw + sums from Pl, Ql
 hipError_t launch_tensor_far(const Plan& p, const DevTables& d, double* R, hipStream_t s);   // rank-one part
 // both in one launch
 hipError_t launch_tensor_fill(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s);

@@ -316,8 +316,10 @@ static int64_t alloc_tables(bs2e_ctx* ctx, bs2e_rk* rk, bool with_tensor)
     d.pairs = (PairInfo*)(rk->small + L.pairs);
     d.rows = with_tensor ? (int32_t*)(rk->small + L.rows) : nullptr;
     d.c_first = (int32_t*)(rk->small + L.c_first);
-    HIP_TRY(ctx, ctx_alloc(ctx, &d.Pl, (size_t)p.n_iv * p.U * p.K));
-    HIP_TRY(ctx, ctx_alloc(ctx, &d.Ql, (size_t)p.n_iv * p.U * p.K));
+    if (rk->precision == BS2E_PREC_MIXED) {
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.Pl, (size_t)p.n_iv * p.U * p.K));
+        HIP_TRY(ctx, ctx_alloc(ctx, &d.Ql, (size_t)p.n_iv * p.U * p.K));
+    }
     HIP_TRY(ctx, ctx_alloc(ctx, &d.Pw, slots));
     HIP_TRY(ctx, ctx_alloc(ctx, &d.Qw, slots));
     HIP_TRY(ctx, ctx_alloc(ctx, &d.PP, slots));
@@ -379,19 +381,18 @@ static int64_t run_primitives_serial(bs2e_ctx* ctx, bs2e_rk* rk)
 {
     clear_stale_error();
     hipStream_t s = ctx->stream;
-    HIP_TRY(ctx, launch_outer_moments(rk->plan, rk->d, s));
+    HIP_TRY(ctx, launch_windows(rk->plan, rk->d, s));
     HIP_TRY(ctx, launch_diag_cells(rk->plan, rk->d, s, false));
-    HIP_TRY(ctx, launch_pair_windows(rk->plan, rk->d, s));
     return BS2E_OK;
 }
 
 // The full build.
-// Up to kOneStreamBytes of tensor: three launches on the main stream, the
-// local moments with the diagonal cells, the pair windows, and the near
-// elements with the rank-one fill (mixed precision: the moments in a launch of
-// their own).  Larger: main stream local moments -> pair windows -> rank-one
-// fill; side stream (forked once the pair windows exist, so that those two
-// short critical-path kernels run alone) diagonal cells -> near elements,
+// Up to kOneStreamBytes of tensor: two launches on the main stream, the pair
+// windows with the diagonal cells, and the near elements with the rank-one
+// fill (mixed precision: local moments, cells and pair windows in a launch
+// each).  Larger: main stream pair windows (mixed precision: after the local
+// moments) -> rank-one fill; side stream (forked once the pair windows exist,
+// so that the short critical path runs alone) diagonal cells -> near elements,
 // concurrently with the rank-one fill; the main stream waits for the side
 // stream at the end, so the build is one unit of work on the caller's stream.
 // The line lies where hiding the cells behind the fill gains more than the
@@ -432,11 +433,12 @@ static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
             if (rk->precision == BS2E_PREC_MIXED) {
                 HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
                 HIP_TRY(ctx, launch_diag_cells(p, rk->d, m, true));
+                if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
+                HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
             } else {
-                HIP_TRY(ctx, launch_moments_and_cells(p, rk->d, m));
+                HIP_TRY(ctx, launch_windows_and_cells(p, rk->d, m));
+                if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
             }
-            if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
-            HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
         } else if (prof) {
             HIP_TRY(ctx, hipEventRecord(ev[3], m));
         }
@@ -447,11 +449,12 @@ static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
         return BS2E_OK;
     }
     if (!rk->from_primitives) {
-        if (rk->precision == BS2E_PREC_MIXED)
+        if (rk->precision == BS2E_PREC_MIXED) {
             HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
-        else
-            HIP_TRY(ctx, launch_outer_moments(p, rk->d, m));
-        HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
+            HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
+        } else {
+            HIP_TRY(ctx, launch_windows(p, rk->d, m));
+        }
     }
     if (prof) HIP_TRY(ctx, hipEventRecord(ev[1], m));
     HIP_TRY(ctx, hipEventRecord(rk->windows, m));

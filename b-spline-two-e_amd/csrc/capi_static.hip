@@ -55,6 +55,7 @@ ScratchLayout scratch_layout(const Plan& p)
     L.rows = o, o += r(4 * p.rows.size());
     L.c_first = o, o += r(4 * p.c_first.size());
     L.small_end = o;
+    // (Pl, Ql: mixed precision only, laid out in both modes: which bases fit does not depend on the mode)
     const size_t local = 8 * (size_t)p.n_iv * p.U * p.K, slots = 8 * (size_t)p.n_pairs * p.k_s * p.K;
     L.Pl = o, o += r(local);
     L.Ql = o, o += r(local);
@@ -138,10 +139,10 @@ int64_t bs2e_rk_build_static(int64_t k, int64_t n_knots, const double* knots, in
     if (e == hipSuccess && precision == BS2E_PREC_MIXED) {
         e = launch_outer_moments_mixed(p, d, s);
         if (e == hipSuccess) e = launch_diag_cells(p, d, s, true);
+        if (e == hipSuccess) e = launch_pair_windows(p, d, s);
     } else if (e == hipSuccess) {
-        e = launch_moments_and_cells(p, d, s);
+        e = launch_windows_and_cells(p, d, s);
     }
-    if (e == hipSuccess) e = launch_pair_windows(p, d, s);
     if (e == hipSuccess) e = launch_tensor_fill(p, d, R, true, s);
     if (e != hipSuccess)
         return fail(nullptr, BS2E_EDEVICE, std::string("bs2e_rk_build_static: ") + hipGetErrorString(e));

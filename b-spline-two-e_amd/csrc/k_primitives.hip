@@ -7,11 +7,14 @@
 // forms (bspline_tools.f90:205-211); its per-spline recurrence (:213-220)
 // gives the same values to rounding.
 //
-// kp_outer  (one workgroup per interval): spline values at the k_GL outer GL
-//   points and the local pair moments of the U = k(k+1)/2 unordered local
-//   spline pairs u = (a,c)
-//     Pl[v][u][k] = h_v sum_q w_q B_a B_c r_q^k,
-//     Ql[v][u][k] = h_v sum_q w_q B_a B_c / r_q^(k+1)       (mat_els.f90:413-428)
+// kp_windows  (one workgroup per two columns c and chunk of multipoles): spline
+//   values at the k_GL outer GL points of the columns' intervals, the local
+//   pair moments there
+//     P^k[v;a,c] = h_v sum_q w_q B_a B_c r_q^k,
+//     Q^k[v;a,c] = h_v sum_q w_q B_a B_c / r_q^(k+1)         (mat_els.f90:413-428)
+//   and, per banded pair p = (a, c), (c, a) and multipole k, the window moments
+//   Pw/Qw[p][j][k] (j-th interval of p's support window), their prefix (P) and
+//   suffix (Q) sums and totals.
 // kp_inner  (one workgroup per interval and chunk of kc multipoles): spline
 //   values at the k_GL^2 inner points of the triangle rule and the diagonal
 //   cells of mat_els.f90:460-483 as the contraction over the outer points
@@ -19,9 +22,9 @@
 //     J'[k][q][u]     = s_q / r_q^(k+1) * sum_p w_p rho_qp^k B_b B_d(rho_qp),
 //   with s_q = (r_q - bp_v)/2 and rho_qp = s_q x_p + (r_q + bp_v)/2, on the
 //   FP64 matrix cores, a few multipoles at a time staged in LDS.
-// kw_pair_windows: per banded pair p and multipole k, the window moments
-//   Pw/Qw[p][j][k] (j-th interval of p's support window), their prefix (P)
-//   and suffix (Q) sums and totals, gathered from Pl/Ql.
+// kw_pair_windows: the same window tables gathered from the local moments
+//   Pl/Ql[v][u][k] of the U = k(k+1)/2 unordered local spline pairs u (what the
+//   mixed-precision moments write).
 #include <algorithm>
 
 #include "bs2e_internal.h"
@@ -77,59 +80,134 @@ static size_t diag_lds_bytes(int64_t ks, int64_t kgl, int64_t KC)
     return sizeof(double) * (size_t)(kgl * (1 + kgl) * ks + 2 * kgl * kgl + (KC * kgl + QP) * U);
 }
 
-// local moments of interval v
+// Columns and multipoles of one window workgroup.
+struct WindowShape {
+    int cols, kc, kchunks, n_wg;
+};
+
+static size_t window_lds_bytes(int64_t ks, int64_t kgl, int64_t cols, int64_t kc)
+{
+    const int64_t npt = (ks + cols - 1) * kgl;
+    return sizeof(double) * (size_t)(npt * (ks + 1 + 2 * kc) + cols * ks * (ks + 1) * kc);
+}
+
+// The window moments of the pairs (a, c) of `cols` columns c and kc multipoles,
+// and their sums.  Moments and window sums in one pass: the local moments of an
+// interval in a launch of their own and a gather of the windows after it took a
+// launch more, which a small build waits for (order 8, 46 splines, 5 multipoles,
+// whole build 23.5 us, now 19.6; 65 splines 24.9, now 21.1); a column evaluates
+// the splines of its k intervals again for that.  The local pair (ta, tc), ta <= tc, of interval c + 1 - tc is
+// the pair (c - tc + ta, c) there, so a column takes every local pair once; the
+// pair (c, a) has the same numbers.
 template <int KS>
-__device__ __forceinline__ void outer_interval(int v, int K, int kgl, const double* __restrict__ t,
-                                               const double* __restrict__ bp, const double* __restrict__ x,
-                                               const double* __restrict__ w, double* __restrict__ Pl,
-                                               double* __restrict__ Ql, double* lds)
+__device__ __forceinline__ void window_columns(int wg, WindowShape ws, int n_b, int n_iv, int K, int kgl,
+                                               const double* __restrict__ t, const double* __restrict__ bp,
+                                               const double* __restrict__ x, const double* __restrict__ w,
+                                               const int32_t* __restrict__ c_first, double* __restrict__ Pw,
+                                               double* __restrict__ Qw, double* __restrict__ PP,
+                                               double* __restrict__ QS, double* __restrict__ Ptot,
+                                               double* __restrict__ Qtot, double* lds)
 {
     constexpr int U = KS * (KS + 1) / 2;
-    double* sB = lds;                 // [kgl][KS]
-    double* sR = sB + kgl * KS;       // [kgl]
-    double* sPow = sR + kgl;          // [kgl][K]  r^k
-    double* sInv = sPow + kgl * K;    // [kgl][K]  1 / r^(k+1)
+    const int blk = wg / ws.kchunks, k0 = (wg - blk * ws.kchunks) * ws.kc;
+    const int nk = min(ws.kc, K - k0);
+    const int c0 = blk * ws.cols + 1, nc = min(ws.cols, n_b + 1 - c0);
+    const int iv0 = max(1, c0 + 2 - KS), npt = (min(n_iv, c0 + nc) + 1 - iv0) * kgl;
+    double* sB = lds;                        // [npt][KS]
+    double* sR = sB + npt * KS;              // [npt]
+    double* sPow = sR + npt;                 // [npt][nk]  r^k
+    double* sInv = sPow + npt * nk;          // [npt][nk]  1 / r^(k+1)
+    double* sP = sInv + npt * nk;            // [nc][U][nk]
+    double* sQ = sP + nc * U * nk;           // [nc][U][nk]
     const int tid = threadIdx.x;
-    const double lim1 = bp[v], lim2 = bp[v + 1];
-    const double h = 0.5 * (lim2 - lim1);
-    const double c = 0.5 * (lim2 + lim1);
-    const int i1 = KS - 1 + (v + 1);
-    for (int q = tid; q < kgl; q += kPThreads) {
-        const double r = h * x[q] + c;
-        sR[q] = r;
-        splines_at<KS>(t, i1, r, sB + q * KS, 1);
+    for (int e = tid; e < npt; e += kPThreads) {
+        const int iv = iv0 + e / kgl, q = e - (iv - iv0) * kgl;
+        const double lim1 = bp[iv - 1], lim2 = bp[iv];
+        const double r = 0.5 * (lim2 - lim1) * x[q] + 0.5 * (lim2 + lim1);
+        sR[e] = r;
+        splines_at<KS>(t, KS - 1 + iv, r, sB + e * KS, 1);
     }
     __syncthreads();
-    for (int e = tid; e < kgl * K; e += kPThreads) {
-        const int q = e / K, k = e - q * K;
-        const double r = sR[q];
+    for (int e = tid; e < npt * nk; e += kPThreads) {
+        const int i = e / nk, k = k0 + e - i * nk;
+        const double r = sR[i];
         sPow[e] = ipow_d(r, k);
         sInv[e] = 1.0 / ipow_d(r, k + 1);
     }
     __syncthreads();
-    for (int e = tid; e < U * K; e += kPThreads) {
-        const int u = e / K, k = e - u * K;
+    for (int e = tid; e < nc * U * nk; e += kPThreads) {
+        const int cu = e / nk, kk = e - cu * nk, c = c0 + cu / U, u = cu - (c - c0) * U;
         int ta, tc;
         local_pair(u, KS, ta, tc);
+        const int iv = c + 1 - tc;
+        if (iv < 1 || iv > n_iv) continue;
+        const int i0 = (iv - iv0) * kgl;
         double accp = 0.0, accq = 0.0;
         for (int q = 0; q < kgl; ++q) {
-            const double bb = w[q] * sB[q * KS + ta] * sB[q * KS + tc];
-            accp = accp + bb * sPow[q * K + k];
-            accq = accq + bb * sInv[q * K + k];
+            const double* b = sB + (i0 + q) * KS;
+            const double bb = w[q] * b[ta] * b[tc];
+            accp = accp + bb * sPow[(i0 + q) * nk + kk];
+            accq = accq + bb * sInv[(i0 + q) * nk + kk];
         }
-        Pl[((size_t)v * U + u) * K + k] = h * accp;
-        Ql[((size_t)v * U + u) * K + k] = h * accq;
+        const double h = 0.5 * (bp[iv] - bp[iv - 1]);
+        sP[e] = h * accp;
+        sQ[e] = h * accq;
+    }
+    __syncthreads();
+    for (int e = tid; e < 2 * nc * KS * nk; e += kPThreads) {
+        int r = e / nk;
+        const int kk = e - r * nk, i = r % KS;      // a = c - i
+        r /= KS;
+        const int c = c0 + (r >> 1), a = c - i;
+        const bool mirror = r & 1;
+        if (a < 1 || (mirror && i == 0)) continue;
+        const int row = mirror ? c : a, col = mirror ? a : c;
+        const size_t pair = (size_t)(c_first[col] + row - max(1, col + 1 - KS));
+        const int v0 = max(1, c + 2 - KS), m = min(n_iv, a + 1) + 1 - v0;
+        const size_t base = pair * KS * K + k0 + kk;
+        const int uc = (c - c0) * U;
+        double pw[KS], qw[KS];
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            pw[j] = 0.0;
+            qw[j] = 0.0;
+            if (j < m) {
+                const int tc = c + 1 - v0 - j, u = uc + sym_local(tc - i, tc, KS);
+                pw[j] = sP[u * nk + kk];
+                qw[j] = sQ[u * nk + kk];
+            }
+        }
+        double run = 0.0;
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            run += pw[j];
+            Pw[base + (size_t)j * K] = pw[j];
+            Qw[base + (size_t)j * K] = qw[j];
+            PP[base + (size_t)j * K] = (j < m) ? run : 0.0;
+        }
+        Ptot[pair * K + k0 + kk] = run;
+        run = 0.0;
+#pragma unroll
+        for (int j = KS - 1; j >= 0; --j) {
+            run += qw[j];
+            QS[base + (size_t)j * K] = (j < m) ? run : 0.0;
+        }
+        Qtot[pair * K + k0 + kk] = run;
     }
 }
 
 template <int KS>
-__global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const double* __restrict__ t,
-                                                      const double* __restrict__ bp, const double* __restrict__ x,
-                                                      const double* __restrict__ w, double* __restrict__ Pl,
-                                                      double* __restrict__ Ql)
+__global__ __launch_bounds__(kPThreads) void kp_windows(WindowShape ws, int n_b, int n_iv, int K, int kgl,
+                                                        const double* __restrict__ t, const double* __restrict__ bp,
+                                                        const double* __restrict__ x, const double* __restrict__ w,
+                                                        const int32_t* __restrict__ c_first, double* __restrict__ Pw,
+                                                        double* __restrict__ Qw, double* __restrict__ PP,
+                                                        double* __restrict__ QS, double* __restrict__ Ptot,
+                                                        double* __restrict__ Qtot)
 {
     extern __shared__ double lds[];
-    outer_interval<KS>((int)blockIdx.x, K, kgl, t, bp, x, w, Pl, Ql, lds);
+    window_columns<KS>((int)xcd_block(blockIdx.x, ws.n_wg), ws, n_b, n_iv, K, kgl, t, bp, x, w, c_first, Pw, Qw, PP,
+                       QS, Ptot, Qtot, lds);
 }
 
 // The diagonal cells.  SYM: write Dsym[v][u1][u2][k] = D[v][u1][u2][k] +
@@ -156,14 +234,16 @@ __global__ __launch_bounds__(kPThreads) void kp_outer(int K, int kgl, const doub
 // busy: the inner moments of all multipoles at once took 104 KB of LDS at
 // order 9, one workgroup per CU) and a loop body that stays in the instruction
 // cache.
-// OUTER: the workgroups past the n_cells of the cells take the local moments,
-// one interval each.
-template <int KS, bool SYM, int KC, bool OUTER>
-__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells,
-                                                      const double* __restrict__ t, const double* __restrict__ bp,
-                                                      const double* __restrict__ x, const double* __restrict__ w,
-                                                      double* __restrict__ D, double* __restrict__ Pl,
-                                                      double* __restrict__ Ql)
+// WINDOWS: the workgroups past the n_cells of the cells take the window moments.
+template <int KS, bool SYM, int KC, bool WINDOWS>
+__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells, WindowShape ws,
+                                                      int n_b, int n_iv, const double* __restrict__ t,
+                                                      const double* __restrict__ bp, const double* __restrict__ x,
+                                                      const double* __restrict__ w,
+                                                      const int32_t* __restrict__ c_first, double* __restrict__ D,
+                                                      double* __restrict__ Pw, double* __restrict__ Qw,
+                                                      double* __restrict__ PP, double* __restrict__ QS,
+                                                      double* __restrict__ Ptot, double* __restrict__ Qtot)
 {
     constexpr int U = KS * (KS + 1) / 2;
     constexpr int TU = (U + 15) / 16;
@@ -172,8 +252,9 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     typedef double d4_t __attribute__((ext_vector_type(4)));
     typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
     extern __shared__ double lds[];
-    if (OUTER && (int)blockIdx.x >= n_cells) {
-        outer_interval<KS>((int)blockIdx.x - n_cells, K, kgl, t, bp, x, w, Pl, Ql, lds);
+    if (WINDOWS && (int)blockIdx.x >= n_cells) {
+        window_columns<KS>((int)blockIdx.x - n_cells, ws, n_b, n_iv, K, kgl, t, bp, x, w, c_first, Pw, Qw, PP, QS,
+                           Ptot, Qtot, lds);
         return;
     }
     const int npt = kgl * (1 + kgl), QP = (kgl + 3) & ~3;
@@ -383,13 +464,31 @@ __global__ __launch_bounds__(256) void kw_window_sums(int n_pairs, int K, int ks
 
 static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
-template <int KS>
-static void launch_outer(const Plan& p, const DevTables& d, hipStream_t s)
+// Two columns and at most four multipoles per workgroup, in equal chunks: the
+// kernel is a chain of short stages (splines, powers, moments, sums), so it
+// takes many small workgroups; more columns share the splines of more
+// intervals, fewer give more workgroups.  Columns x multipoles, until the
+// windows are done (order 9, 600 splines, 25 multipoles / order 9, 400, 17 /
+// order 8, 200, 11, with the launch): 2 x 4 38 / 23 / 16 us, 1 x 4 44 / 26 / 14,
+// 4 x 4 58 / 26 / 16, 8 x 4 62 / 28 / 20, 2 x 8 52 / 25 / 16, 1 x 16 48 / 37 / 15.
+static WindowShape window_shape(const Plan& p)
 {
-    const size_t lds = outer_lds_bytes(KS, p.k_gl, p.K);
-    if (allow_lds((const void*)kp_outer<KS>, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(kp_outer<KS>, dim3((unsigned)p.n_iv), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, d.t, d.bp,
-                       d.x, d.w, d.Pl, d.Ql);
+    int cols = 2, kchunks = (int)((p.K + 3) / 4);
+    int kc = (int)((p.K + kchunks - 1) / kchunks);
+    if (window_lds_bytes(p.k_s, p.k_gl, cols, kc) > 64 * 1024) cols = 1;
+    while (kc > 1 && window_lds_bytes(p.k_s, p.k_gl, cols, kc) > kLdsPerWorkgroup) --kc;
+    kchunks = (int)((p.K + kc - 1) / kc);
+    return {cols, kc, kchunks, (int)((p.n_b + cols - 1) / cols) * kchunks};
+}
+
+template <int KS>
+static void launch_windows(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    const WindowShape ws = window_shape(p);
+    const size_t lds = window_lds_bytes(KS, p.k_gl, ws.cols, ws.kc);
+    if (allow_lds((const void*)kp_windows<KS>, lds) != hipSuccess) return;   // the error stays for hipGetLastError
+    hipLaunchKernelGGL(kp_windows<KS>, dim3((unsigned)ws.n_wg), dim3(kPThreads), lds, s, ws, (int)p.n_b, (int)p.n_iv,
+                       (int)p.K, (int)p.k_gl, d.t, d.bp, d.x, d.w, d.c_first, d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot);
 }
 
 // Multipoles that a diagonal-cell workgroup holds at a time: four; two where
@@ -415,26 +514,28 @@ int inner_kc_used(const Plan& p)
     return (int)std::min<int64_t>(kc, std::max(kmax, 1));
 }
 
-template <int KS, bool SYM, int KC, bool OUTER>
+template <int KS, bool SYM, int KC, bool WINDOWS>
 static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int kc = inner_kc_used(p), kchunks = (int)((p.K + kc - 1) / kc);
     const int n_cells = (int)(p.n_iv * kchunks);
     size_t lds = diag_lds_bytes(KS, p.k_gl, KC);
-    if (OUTER) lds = std::max(lds, outer_lds_bytes(KS, p.k_gl, p.K));
-    const auto fn = kp_inner<KS, SYM, KC, OUTER>;
+    const WindowShape ws = window_shape(p);
+    if (WINDOWS) lds = std::max(lds, window_lds_bytes(KS, p.k_gl, ws.cols, ws.kc));
+    const auto fn = kp_inner<KS, SYM, KC, WINDOWS>;
     if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(fn, dim3((unsigned)(n_cells + (OUTER ? p.n_iv : 0))), dim3(kPThreads), lds, s, (int)p.K,
-                       (int)p.k_gl, kc, kchunks, n_cells, d.t, d.bp, d.x, d.w, d.D, d.Pl, d.Ql);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(n_cells + (WINDOWS ? ws.n_wg : 0))), dim3(kPThreads), lds, s, (int)p.K,
+                       (int)p.k_gl, kc, kchunks, n_cells, ws, (int)p.n_b, (int)p.n_iv, d.t, d.bp, d.x, d.w, d.c_first,
+                       d.D, d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot);
 }
 
-template <int KS, bool SYM, bool OUTER>
+template <int KS, bool SYM, bool WINDOWS>
 static void launch_inner(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int KC = inner_group(p);
-    if (KC == 4) launch_inner_kc<KS, SYM, 4, OUTER>(p, d, s);
-    else if (KC == 2) launch_inner_kc<KS, SYM, 2, OUTER>(p, d, s);
-    else launch_inner_kc<KS, SYM, 1, OUTER>(p, d, s);
+    if (KC == 4) launch_inner_kc<KS, SYM, 4, WINDOWS>(p, d, s);
+    else if (KC == 2) launch_inner_kc<KS, SYM, 2, WINDOWS>(p, d, s);
+    else launch_inner_kc<KS, SYM, 1, WINDOWS>(p, d, s);
 }
 
 template <int KS>
@@ -450,7 +551,7 @@ static void launch_inner_plain(const Plan& p, const DevTables& d, hipStream_t s)
 }
 
 template <int KS>
-static void launch_inner_outer(const Plan& p, const DevTables& d, hipStream_t s)
+static void launch_inner_windows(const Plan& p, const DevTables& d, hipStream_t s)
 {
     launch_inner<KS, true, true>(p, d, s);
 }
@@ -475,9 +576,9 @@ static void launch_inner_outer(const Plan& p, const DevTables& d, hipStream_t s)
         default: return hipErrorInvalidValue;                                                                \
     }
 
-hipError_t launch_outer_moments(const Plan& p, const DevTables& d, hipStream_t s)
+hipError_t launch_windows(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    BS2E_ORDER_SWITCH(launch_outer)
+    BS2E_ORDER_SWITCH(launch_windows)
     return hipGetLastError();
 }
 
@@ -491,9 +592,9 @@ hipError_t launch_diag_cells(const Plan& p, const DevTables& d, hipStream_t s, b
     return hipGetLastError();
 }
 
-hipError_t launch_moments_and_cells(const Plan& p, const DevTables& d, hipStream_t s)
+hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    BS2E_ORDER_SWITCH(launch_inner_outer)
+    BS2E_ORDER_SWITCH(launch_inner_windows)
     return hipGetLastError();
 }
 

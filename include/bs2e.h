@@ -148,8 +148,8 @@ int64_t bs2e_rk_get_val(const bs2e_rk *rk, const int64_t *indices, double *value
  * bs2e_rk_stage_times call: [0] local moments + pair windows done,
  * [1] rank-one fill done, [2] diagonal cells done (second stream), [3] near
  * elements done (second stream), [4] end of the build.  A small tensor's build
- * runs on one stream, the cells before the pair windows, the near elements and
- * the fill in one launch ([1] = [3]). */
+ * runs on one stream, the cells before or beside the pair windows, the near
+ * elements and the fill in one launch ([1] = [3]). */
 int64_t bs2e_rk_set_profiling(bs2e_rk *rk, int64_t on);
 int64_t bs2e_rk_stage_times(bs2e_rk *rk, double *ms, int64_t n);
 /* on != 0: the next bs2e_rk_compute captures the build into a

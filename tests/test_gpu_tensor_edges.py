@@ -55,6 +55,19 @@ def test_diagonal_containers_at_edges(k, n_b, k_GL, max_k, oracle):
     assert np.all(np.abs(r_d_k.data - ref) <= 1e-12 * np.abs(ref))
 
 
+@pytest.mark.parametrize("k,n_b,k_GL,max_k", [(2, 2, 4, 0), (2, 9, 4, 4), (5, 4, 7, 3), (8, 8, 10, 8), (9, 12, 14, 5),
+                                              (11, 23, 17, 16), (14, 16, 29, 4), (16, 17, 26, 2)])
+def test_window_moments_at_edges(k, n_b, k_GL, max_k, oracle):
+    """One column and odd counts of columns, fewer splines than the order, multipoles in one and several chunks."""
+    t = _knots(k, n_b)
+    spl = bs2e.b_spline(k, t)
+    r_k, r_m_k, r_d_k = (x().init(max_k, spl) for x in (bs2e.sparse_4d, bs2e.sparse_4d, bs2e.sparse_6d))
+    bs2e.setup_Slater_integrals(spl, max_k, k_GL, r_k, r_m_k, r_d_k)
+    ref = oracle.slater_off_diag(k, t, k_GL, max_k)
+    for got, name in ((r_k, "rk"), (r_m_k, "rmk")):
+        assert np.all(np.abs(got.data - ref[name]) <= 1e-12 * np.abs(ref[name])), name
+
+
 @pytest.mark.parametrize("k,n_b,k_GL,max_k", CASES)
 def test_fill_shapes_at_edges(k, n_b, k_GL, max_k, oracle):
     t = _knots(k, n_b)
