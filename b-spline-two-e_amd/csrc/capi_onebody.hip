@@ -44,10 +44,12 @@ static int64_t one_body(bs2e_ctx* ctx, const char* who, int64_t k, int64_t n_kno
         HIP_TRY(ctx, ctx_alloc(ctx, &d.x, p.k_gl));
         HIP_TRY(ctx, ctx_alloc(ctx, &d.w, p.k_gl));
         HIP_TRY(ctx, ctx_alloc(ctx, &B, tab));
-        HIP_TRY(ctx, ctx_alloc(ctx, &B2, tab));
         HIP_TRY(ctx, ctx_alloc(ctx, &rw, 2 * (size_t)p.n_iv * p.k_gl));
         if (S_out) HIP_TRY(ctx, ctx_alloc(ctx, &dS, 2 * nn));
-        if (H_out) HIP_TRY(ctx, ctx_alloc(ctx, &dH, 2 * nn * n_l));
+        if (H_out) {
+            HIP_TRY(ctx, ctx_alloc(ctx, &B2, tab));
+            HIP_TRY(ctx, ctx_alloc(ctx, &dH, 2 * nn * n_l));
+        }
         hipStream_t s = ctx->stream;
         HIP_TRY(ctx, copy_to_device(ctx, {{d.t, p.t.data(), 8 * (size_t)p.n_knots},
                                           {d.bp, p.bp.data(), 8 * (size_t)(p.n_iv + 1)},
@@ -79,7 +81,7 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
     const size_t n_out = (size_t)(max_k + 1) * p.n_b * p.n_b;
     const size_t tab = (size_t)p.n_iv * p.k_gl * p.k_s;
     DevTables d;
-    double *B = nullptr, *B2 = nullptr, *rw = nullptr, *dout = nullptr;
+    double *B = nullptr, *rw = nullptr, *dout = nullptr;
     auto cleanup = [&]() {
         QuietScope quiet;
         ctx_free(ctx, d.t);
@@ -87,7 +89,6 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
         ctx_free(ctx, d.x);
         ctx_free(ctx, d.w);
         ctx_free(ctx, B);
-        ctx_free(ctx, B2);
         ctx_free(ctx, rw);
         ctx_free(ctx, dout);
     };
@@ -97,7 +98,6 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
         HIP_TRY(ctx, ctx_alloc(ctx, &d.x, p.k_gl));
         HIP_TRY(ctx, ctx_alloc(ctx, &d.w, p.k_gl));
         HIP_TRY(ctx, ctx_alloc(ctx, &B, tab));
-        HIP_TRY(ctx, ctx_alloc(ctx, &B2, tab));
         HIP_TRY(ctx, ctx_alloc(ctx, &rw, 2 * (size_t)p.n_iv * p.k_gl));
         HIP_TRY(ctx, ctx_alloc(ctx, &dout, n_out));
         hipStream_t s = ctx->stream;
@@ -105,7 +105,7 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
                                           {d.bp, p.bp.data(), 8 * (size_t)(p.n_iv + 1)},
                                           {d.x, p.x.data(), 8 * (size_t)p.k_gl}, {d.w, p.w.data(), 8 * (size_t)p.k_gl}}));
         clear_stale_error();
-        HIP_TRY(ctx, launch_rk_int(p, d, B, B2, rw, (int)max_k, r0, dout, s));
+        HIP_TRY(ctx, launch_rk_int(p, d, B, rw, (int)max_k, r0, dout, s));
         HIP_TRY(ctx, copy_to_host(ctx, {{out, dout, 8 * n_out}}));
         return BS2E_OK;
     };
