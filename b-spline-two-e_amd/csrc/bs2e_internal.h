@@ -251,7 +251,8 @@ int64_t count_configs(int64_t L, int64_t term_pi, int64_t max_l_1p, int64_t n_b,
 // Kernel launchers (each .hip file launches its own kernels).
 hipError_t launch_windows(const Plan& p, const DevTables& d, hipStream_t s);                 // Pw/Qw + sums
 hipError_t launch_diag_cells(const Plan& p, const DevTables& d, hipStream_t s, bool symmetrised);  // D / Dsym
-hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, hipStream_t s);             // with Dsym in one launch
+// with Dsym in one launch; gather: from the Pl, Ql of an earlier one
+hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, bool gather, hipStream_t s);
 hipError_t launch_symmetrize(const Plan& p, const DevTables& d, hipStream_t s);                    // D -> Dsym
 size_t near_lds_bytes(int64_t ks, int64_t K);
 constexpr int kNearMaxSeg = 64;   // column segments of one near row (<= 2k - 1 <= 39 for k <= 20)

@@ -389,15 +389,14 @@ static int64_t run_primitives_serial(bs2e_ctx* ctx, bs2e_rk* rk)
 // The full build.
 // Up to kOneStreamBytes of tensor: two launches on the main stream, the pair
 // windows with the diagonal cells, and the near elements with the rank-one
-// fill (mixed precision: local moments, cells and pair windows in a launch
-// each).  Larger: main stream pair windows (mixed precision: after the local
+// fill (mixed precision: the local moments in a launch before them).  Larger: main stream pair windows (mixed precision: after the local
 // moments) -> rank-one fill; side stream (forked once the pair windows exist,
 // so that the short critical path runs alone) diagonal cells -> near elements,
 // concurrently with the rank-one fill; the main stream waits for the side
 // stream at the end, so the build is one unit of work on the caller's stream.
 // The line lies where hiding the cells behind the fill gains more than the
 // second stream's events cost (about 20 us).  Builds one after another, one
-// stream against two: 0.0014 GB of tensor 13 us against 46, 0.016 GB 24 / 49,
+// stream against two: 0.0014 GB of tensor 10 us against 46, 0.016 GB 20 / 49,
 // 0.15 GB 45 / 59, 0.26 GB 73 / 79, 0.55 GB 131 / 135, 0.76 GB 153 / 147, 0.81 GB
 // 175 / 155, 2.7 GB 0.467 / 0.452 ms.
 // Profiling events, all relative to ev[0]: ev[1] windows done, ev[2] far
@@ -430,15 +429,10 @@ static int64_t run_build(bs2e_ctx* ctx, bs2e_rk* rk)
     const Plan& p = rk->plan;
     if (sizeof(double) * rk->R_elems <= kOneStreamBytes) {
         if (!rk->from_primitives) {
-            if (rk->precision == BS2E_PREC_MIXED) {
-                HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
-                HIP_TRY(ctx, launch_diag_cells(p, rk->d, m, true));
-                if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
-                HIP_TRY(ctx, launch_pair_windows(p, rk->d, m));
-            } else {
-                HIP_TRY(ctx, launch_windows_and_cells(p, rk->d, m));
-                if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
-            }
+            const bool mixed = rk->precision == BS2E_PREC_MIXED;
+            if (mixed) HIP_TRY(ctx, launch_outer_moments_mixed(p, rk->d, m));
+            HIP_TRY(ctx, launch_windows_and_cells(p, rk->d, mixed, m));
+            if (prof) HIP_TRY(ctx, hipEventRecord(ev[3], m));
         } else if (prof) {
             HIP_TRY(ctx, hipEventRecord(ev[3], m));
         }

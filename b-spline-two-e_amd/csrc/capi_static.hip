@@ -134,15 +134,11 @@ int64_t bs2e_rk_build_static(int64_t k, int64_t n_knots, const double* knots, in
     // the scratch); the wait lets the host image go before the call returns.
     e = hipMemcpyAsync(base, host.data(), L.small_end, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    // one stream: moments and diagonal cells (symmetrised), pair windows, near
-    // elements and rank-one fill; the values of bs2e_rk_compute
-    if (e == hipSuccess && precision == BS2E_PREC_MIXED) {
-        e = launch_outer_moments_mixed(p, d, s);
-        if (e == hipSuccess) e = launch_diag_cells(p, d, s, true);
-        if (e == hipSuccess) e = launch_pair_windows(p, d, s);
-    } else if (e == hipSuccess) {
-        e = launch_windows_and_cells(p, d, s);
-    }
+    // one stream: (mixed precision: moments,) pair windows and diagonal cells
+    // (symmetrised), near elements and rank-one fill; the values of bs2e_rk_compute
+    const bool mixed = precision == BS2E_PREC_MIXED;
+    if (e == hipSuccess && mixed) e = launch_outer_moments_mixed(p, d, s);
+    if (e == hipSuccess) e = launch_windows_and_cells(p, d, mixed, s);
     if (e == hipSuccess) e = launch_tensor_fill(p, d, R, true, s);
     if (e != hipSuccess)
         return fail(nullptr, BS2E_EDEVICE, std::string("bs2e_rk_build_static: ") + hipGetErrorString(e));

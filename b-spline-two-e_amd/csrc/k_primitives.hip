@@ -34,6 +34,8 @@ namespace bs2e {
 
 constexpr int kPThreads = 256;
 
+static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
+
 hipError_t allow_lds(const void* fn, size_t bytes)
 {
     if (bytes <= 64 * 1024) return hipSuccess;
@@ -85,6 +87,17 @@ struct WindowShape {
     int cols, kc, kchunks, n_wg;
 };
 
+// What the window workgroups read and write; pairs, Pl and Ql for the gather
+// from local moments, c_first for the moments taken here.
+struct WindowArgs {
+    WindowShape ws;
+    int n_b, n_iv, n_pairs;
+    const int32_t* c_first;
+    const PairInfo* pairs;
+    const double *Pl, *Ql;
+    double *Pw, *Qw, *PP, *QS, *Ptot, *Qtot;
+};
+
 static size_t window_lds_bytes(int64_t ks, int64_t kgl, int64_t cols, int64_t kc)
 {
     const int64_t npt = (ks + cols - 1) * kgl;
@@ -100,14 +113,15 @@ static size_t window_lds_bytes(int64_t ks, int64_t kgl, int64_t cols, int64_t kc
 // the pair (c - tc + ta, c) there, so a column takes every local pair once; the
 // pair (c, a) has the same numbers.
 template <int KS>
-__device__ __forceinline__ void window_columns(int wg, WindowShape ws, int n_b, int n_iv, int K, int kgl,
+__device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int K, int kgl,
                                                const double* __restrict__ t, const double* __restrict__ bp,
-                                               const double* __restrict__ x, const double* __restrict__ w,
-                                               const int32_t* __restrict__ c_first, double* __restrict__ Pw,
-                                               double* __restrict__ Qw, double* __restrict__ PP,
-                                               double* __restrict__ QS, double* __restrict__ Ptot,
-                                               double* __restrict__ Qtot, double* lds)
+                                               const double* __restrict__ x, const double* __restrict__ w, double* lds)
 {
+    const WindowShape ws = A.ws;
+    const int n_b = A.n_b, n_iv = A.n_iv;
+    const int32_t* __restrict__ c_first = A.c_first;
+    double *__restrict__ Pw = A.Pw, *__restrict__ Qw = A.Qw, *__restrict__ PP = A.PP, *__restrict__ QS = A.QS;
+    double *__restrict__ Ptot = A.Ptot, *__restrict__ Qtot = A.Qtot;
     constexpr int U = KS * (KS + 1) / 2;
     const int blk = wg / ws.kchunks, k0 = (wg - blk * ws.kchunks) * ws.kc;
     const int nk = min(ws.kc, K - k0);
@@ -196,18 +210,65 @@ __device__ __forceinline__ void window_columns(int wg, WindowShape ws, int n_b, 
     }
 }
 
+// The same from local moments that an earlier launch wrote, one thread per
+// pair and multipole.
+template <int KSMAX>
+__device__ __forceinline__ void window_gather(int64_t gid, const WindowArgs& A, int K, int ks)
+{
+    if (gid >= (int64_t)A.n_pairs * K) return;
+    const int U = ks * (ks + 1) / 2;
+    const int p = (int)(gid / K), k = (int)(gid - (int64_t)p * K);
+    const PairInfo pi = A.pairs[p];
+    const double *__restrict__ Pl = A.Pl, *__restrict__ Ql = A.Ql;
+    double *__restrict__ Pw = A.Pw, *__restrict__ Qw = A.Qw, *__restrict__ PP = A.PP, *__restrict__ QS = A.QS;
+    double pw[KSMAX], qw[KSMAX];
+#pragma unroll
+    for (int j = 0; j < KSMAX; ++j) {
+        pw[j] = 0.0;
+        qw[j] = 0.0;
+        if (j < pi.m) {
+            const int v = pi.v0 - 1 + j;                         // 0-based interval
+            const int u = sym_local(pi.a - v, pi.c - v, ks);     // local splines s - iv
+            pw[j] = Pl[((size_t)v * U + u) * K + k];
+            qw[j] = Ql[((size_t)v * U + u) * K + k];
+        }
+    }
+    const size_t base = (size_t)p * ks * K + k;
+    double run = 0.0;
+#pragma unroll
+    for (int j = 0; j < KSMAX; ++j) {
+        if (j < ks) {
+            run += pw[j];
+            Pw[base + (size_t)j * K] = pw[j];
+            Qw[base + (size_t)j * K] = qw[j];
+            PP[base + (size_t)j * K] = (j < pi.m) ? run : 0.0;
+        }
+    }
+    A.Ptot[(size_t)p * K + k] = run;
+    run = 0.0;
+#pragma unroll
+    for (int j = KSMAX - 1; j >= 0; --j) {
+        if (j < ks) {
+            run += qw[j];
+            QS[base + (size_t)j * K] = (j < pi.m) ? run : 0.0;
+        }
+    }
+    A.Qtot[(size_t)p * K + k] = run;
+}
+
 template <int KS>
-__global__ __launch_bounds__(kPThreads) void kp_windows(WindowShape ws, int n_b, int n_iv, int K, int kgl,
-                                                        const double* __restrict__ t, const double* __restrict__ bp,
-                                                        const double* __restrict__ x, const double* __restrict__ w,
-                                                        const int32_t* __restrict__ c_first, double* __restrict__ Pw,
-                                                        double* __restrict__ Qw, double* __restrict__ PP,
-                                                        double* __restrict__ QS, double* __restrict__ Ptot,
-                                                        double* __restrict__ Qtot)
+__global__ __launch_bounds__(kPThreads) void kp_windows(WindowArgs A, int K, int kgl, const double* __restrict__ t,
+                                                        const double* __restrict__ bp, const double* __restrict__ x,
+                                                        const double* __restrict__ w)
 {
     extern __shared__ double lds[];
-    window_columns<KS>((int)xcd_block(blockIdx.x, ws.n_wg), ws, n_b, n_iv, K, kgl, t, bp, x, w, c_first, Pw, Qw, PP,
-                       QS, Ptot, Qtot, lds);
+    window_columns<KS>((int)xcd_block(blockIdx.x, A.ws.n_wg), A, K, kgl, t, bp, x, w, lds);
+}
+
+template <int KSMAX>
+__global__ __launch_bounds__(kPThreads) void kw_pair_windows(WindowArgs A, int K, int ks)
+{
+    window_gather<KSMAX>((int64_t)blockIdx.x * kPThreads + threadIdx.x, A, K, ks);
 }
 
 // The diagonal cells.  SYM: write Dsym[v][u1][u2][k] = D[v][u1][u2][k] +
@@ -234,16 +295,15 @@ __global__ __launch_bounds__(kPThreads) void kp_windows(WindowShape ws, int n_b,
 // busy: the inner moments of all multipoles at once took 104 KB of LDS at
 // order 9, one workgroup per CU) and a loop body that stays in the instruction
 // cache.
-// WINDOWS: the workgroups past the n_cells of the cells take the window moments.
-template <int KS, bool SYM, int KC, bool WINDOWS>
-__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells, WindowShape ws,
-                                                      int n_b, int n_iv, const double* __restrict__ t,
-                                                      const double* __restrict__ bp, const double* __restrict__ x,
-                                                      const double* __restrict__ w,
-                                                      const int32_t* __restrict__ c_first, double* __restrict__ D,
-                                                      double* __restrict__ Pw, double* __restrict__ Qw,
-                                                      double* __restrict__ PP, double* __restrict__ QS,
-                                                      double* __restrict__ Ptot, double* __restrict__ Qtot)
+// WITH: the workgroups past the n_cells of the cells take the window moments,
+// or gather them.
+enum class With { kNothing, kMoments, kGather };
+
+template <int KS, bool SYM, int KC, With WITH>
+__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells, WindowArgs A,
+                                                      const double* __restrict__ t, const double* __restrict__ bp,
+                                                      const double* __restrict__ x, const double* __restrict__ w,
+                                                      double* __restrict__ D)
 {
     constexpr int U = KS * (KS + 1) / 2;
     constexpr int TU = (U + 15) / 16;
@@ -252,9 +312,10 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     typedef double d4_t __attribute__((ext_vector_type(4)));
     typedef double d2u_t __attribute__((ext_vector_type(2), aligned(8)));
     extern __shared__ double lds[];
-    if (WINDOWS && (int)blockIdx.x >= n_cells) {
-        window_columns<KS>((int)blockIdx.x - n_cells, ws, n_b, n_iv, K, kgl, t, bp, x, w, c_first, Pw, Qw, PP, QS,
-                           Ptot, Qtot, lds);
+    if (WITH != With::kNothing && (int)blockIdx.x >= n_cells) {
+        const int wg = (int)blockIdx.x - n_cells;
+        if constexpr (WITH == With::kMoments) window_columns<KS>(wg, A, K, kgl, t, bp, x, w, lds);
+        else window_gather<KS>((int64_t)wg * kPThreads + threadIdx.x, A, K, KS);
         return;
     }
     const int npt = kgl * (1 + kgl), QP = (kgl + 3) & ~3;
@@ -388,54 +449,6 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     }
 }
 
-// Per (pair, k): window moments from the local tables, prefix/suffix sums.
-template <int KSMAX>
-__global__ __launch_bounds__(256) void kw_pair_windows(int n_pairs, int K, int ks, int U,
-                                                       const PairInfo* __restrict__ pairs,
-                                                       const double* __restrict__ Pl, const double* __restrict__ Ql,
-                                                       double* __restrict__ Pw, double* __restrict__ Qw,
-                                                       double* __restrict__ PP, double* __restrict__ QS,
-                                                       double* __restrict__ Ptot, double* __restrict__ Qtot)
-{
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= (int64_t)n_pairs * K) return;
-    const int p = (int)(gid / K), k = (int)(gid - (int64_t)p * K);
-    const PairInfo pi = pairs[p];
-    double pw[KSMAX], qw[KSMAX];
-#pragma unroll
-    for (int j = 0; j < KSMAX; ++j) {
-        pw[j] = 0.0;
-        qw[j] = 0.0;
-        if (j < pi.m) {
-            const int v = pi.v0 - 1 + j;                         // 0-based interval
-            const int u = sym_local(pi.a - v, pi.c - v, ks);     // local splines s - iv
-            pw[j] = Pl[((size_t)v * U + u) * K + k];
-            qw[j] = Ql[((size_t)v * U + u) * K + k];
-        }
-    }
-    const size_t base = (size_t)p * ks * K + k;
-    double run = 0.0;
-#pragma unroll
-    for (int j = 0; j < KSMAX; ++j) {
-        if (j < ks) {
-            run += pw[j];
-            Pw[base + (size_t)j * K] = pw[j];
-            Qw[base + (size_t)j * K] = qw[j];
-            PP[base + (size_t)j * K] = (j < pi.m) ? run : 0.0;
-        }
-    }
-    Ptot[(size_t)p * K + k] = run;
-    run = 0.0;
-#pragma unroll
-    for (int j = KSMAX - 1; j >= 0; --j) {
-        if (j < ks) {
-            run += qw[j];
-            QS[base + (size_t)j * K] = (j < pi.m) ? run : 0.0;
-        }
-    }
-    Qtot[(size_t)p * K + k] = run;
-}
-
 // Window prefix/suffix sums from Pw/Qw already in place (the moments were
 // gathered from caller-provided containers).
 __global__ __launch_bounds__(256) void kw_window_sums(int n_pairs, int K, int ks, const PairInfo* __restrict__ pairs,
@@ -462,8 +475,6 @@ __global__ __launch_bounds__(256) void kw_window_sums(int n_pairs, int K, int ks
     Qtot[(size_t)p * K + k] = run;
 }
 
-static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
-
 // Two columns and at most four multipoles per workgroup, in equal chunks: the
 // kernel is a chain of short stages (splines, powers, moments, sums), so it
 // takes many small workgroups; more columns share the splines of more
@@ -481,14 +492,20 @@ static WindowShape window_shape(const Plan& p)
     return {cols, kc, kchunks, (int)((p.n_b + cols - 1) / cols) * kchunks};
 }
 
+static WindowArgs window_args(const Plan& p, const DevTables& d)
+{
+    return {window_shape(p), (int)p.n_b, (int)p.n_iv, (int)p.n_pairs, d.c_first, d.pairs, d.Pl, d.Ql,
+            d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot};
+}
+
 template <int KS>
 static void launch_windows(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    const WindowShape ws = window_shape(p);
-    const size_t lds = window_lds_bytes(KS, p.k_gl, ws.cols, ws.kc);
+    const WindowArgs A = window_args(p, d);
+    const size_t lds = window_lds_bytes(KS, p.k_gl, A.ws.cols, A.ws.kc);
     if (allow_lds((const void*)kp_windows<KS>, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(kp_windows<KS>, dim3((unsigned)ws.n_wg), dim3(kPThreads), lds, s, ws, (int)p.n_b, (int)p.n_iv,
-                       (int)p.K, (int)p.k_gl, d.t, d.bp, d.x, d.w, d.c_first, d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot);
+    hipLaunchKernelGGL(kp_windows<KS>, dim3((unsigned)A.ws.n_wg), dim3(kPThreads), lds, s, A, (int)p.K, (int)p.k_gl,
+                       d.t, d.bp, d.x, d.w);
 }
 
 // Multipoles that a diagonal-cell workgroup holds at a time: four; two where
@@ -514,46 +531,56 @@ int inner_kc_used(const Plan& p)
     return (int)std::min<int64_t>(kc, std::max(kmax, 1));
 }
 
-template <int KS, bool SYM, int KC, bool WINDOWS>
+template <int KS, bool SYM, int KC, With WITH>
 static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int kc = inner_kc_used(p), kchunks = (int)((p.K + kc - 1) / kc);
     const int n_cells = (int)(p.n_iv * kchunks);
+    const WindowArgs A = window_args(p, d);
     size_t lds = diag_lds_bytes(KS, p.k_gl, KC);
-    const WindowShape ws = window_shape(p);
-    if (WINDOWS) lds = std::max(lds, window_lds_bytes(KS, p.k_gl, ws.cols, ws.kc));
-    const auto fn = kp_inner<KS, SYM, KC, WINDOWS>;
+    unsigned n_wg = (unsigned)n_cells;
+    if (WITH == With::kMoments) {
+        lds = std::max(lds, window_lds_bytes(KS, p.k_gl, A.ws.cols, A.ws.kc));
+        n_wg += (unsigned)A.ws.n_wg;
+    }
+    if (WITH == With::kGather) n_wg += blocks_for(p.n_pairs * p.K, kPThreads);
+    const auto fn = kp_inner<KS, SYM, KC, WITH>;
     if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(fn, dim3((unsigned)(n_cells + (WINDOWS ? ws.n_wg : 0))), dim3(kPThreads), lds, s, (int)p.K,
-                       (int)p.k_gl, kc, kchunks, n_cells, ws, (int)p.n_b, (int)p.n_iv, d.t, d.bp, d.x, d.w, d.c_first,
-                       d.D, d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot);
+    hipLaunchKernelGGL(fn, dim3(n_wg), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc, kchunks, n_cells, A, d.t,
+                       d.bp, d.x, d.w, d.D);
 }
 
-template <int KS, bool SYM, bool WINDOWS>
+template <int KS, bool SYM, With WITH>
 static void launch_inner(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int KC = inner_group(p);
-    if (KC == 4) launch_inner_kc<KS, SYM, 4, WINDOWS>(p, d, s);
-    else if (KC == 2) launch_inner_kc<KS, SYM, 2, WINDOWS>(p, d, s);
-    else launch_inner_kc<KS, SYM, 1, WINDOWS>(p, d, s);
+    if (KC == 4) launch_inner_kc<KS, SYM, 4, WITH>(p, d, s);
+    else if (KC == 2) launch_inner_kc<KS, SYM, 2, WITH>(p, d, s);
+    else launch_inner_kc<KS, SYM, 1, WITH>(p, d, s);
 }
 
 template <int KS>
 static void launch_inner_sym(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    launch_inner<KS, true, false>(p, d, s);
+    launch_inner<KS, true, With::kNothing>(p, d, s);
 }
 
 template <int KS>
 static void launch_inner_plain(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    launch_inner<KS, false, false>(p, d, s);
+    launch_inner<KS, false, With::kNothing>(p, d, s);
 }
 
 template <int KS>
 static void launch_inner_windows(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    launch_inner<KS, true, true>(p, d, s);
+    launch_inner<KS, true, With::kMoments>(p, d, s);
+}
+
+template <int KS>
+static void launch_inner_gather(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    launch_inner<KS, true, With::kGather>(p, d, s);
 }
 
 #define BS2E_ORDER_SWITCH(FN)                                                                                \
@@ -592,18 +619,21 @@ hipError_t launch_diag_cells(const Plan& p, const DevTables& d, hipStream_t s, b
     return hipGetLastError();
 }
 
-hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, hipStream_t s)
+hipError_t launch_windows_and_cells(const Plan& p, const DevTables& d, bool gather, hipStream_t s)
 {
-    BS2E_ORDER_SWITCH(launch_inner_windows)
+    if (gather) {
+        BS2E_ORDER_SWITCH(launch_inner_gather)
+    } else {
+        BS2E_ORDER_SWITCH(launch_inner_windows)
+    }
     return hipGetLastError();
 }
 
 template <int KSMAX>
 static void launch_kw(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    const int64_t n = p.n_pairs * p.K;
-    hipLaunchKernelGGL(kw_pair_windows<KSMAX>, dim3(blocks_for(n, 256)), dim3(256), 0, s, (int)p.n_pairs, (int)p.K,
-                       (int)p.k_s, (int)p.U, d.pairs, d.Pl, d.Ql, d.Pw, d.Qw, d.PP, d.QS, d.Ptot, d.Qtot);
+    hipLaunchKernelGGL(kw_pair_windows<KSMAX>, dim3(blocks_for(p.n_pairs * p.K, kPThreads)), dim3(kPThreads), 0, s,
+                       window_args(p, d), (int)p.K, (int)p.k_s);
 }
 
 hipError_t launch_pair_windows(const Plan& p, const DevTables& d, hipStream_t s)
