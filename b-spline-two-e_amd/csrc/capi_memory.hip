@@ -228,7 +228,7 @@ hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hip
     for (size_t i = 0; i < n; ++i) total += pieces[i].bytes;
     if (total == 0) return to_host ? hipStreamSynchronize(s) : hipSuccess;
     const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
-    if (!prepare(total)) {
+    if (total <= (to_host ? kDirectToHost : kDirectToDevice) || !prepare(total)) {
         for (size_t i = 0; i < n; ++i)
             if (pieces[i].bytes > 0) {
                 const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, kind, s);
