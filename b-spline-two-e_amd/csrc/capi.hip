@@ -936,6 +936,10 @@ int64_t bs2e_rk_copy_to_host(bs2e_rk* rk, double* dst, int64_t n_elems)
     return BS2E_OK;
 }
 
+// Up to here a blocking copy of a row takes 16 us, a copy on the stream and the
+// wait for it 25 (rows of 5 and 9 KB; of 22 KB 12 us on the stream).
+static constexpr size_t kShortRows = (size_t)16 << 10;
+
 int64_t bs2e_rk_copy_rows(const bs2e_rk* rk, int64_t row_lo, int64_t n_rows, double* dst)
 {
     if (!rk || !dst) return fail(nullptr, BS2E_EINVAL, "bs2e_rk_copy_rows: NULL argument");
@@ -950,7 +954,14 @@ int64_t bs2e_rk_copy_rows(const bs2e_rk* rk, int64_t row_lo, int64_t n_rows, dou
         return BS2E_OK;
     }
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, copy_to_host(ctx, {{dst, rk->R + (size_t)row_lo * row, sizeof(double) * row * (size_t)n_rows}}));
+    const double* src = rk->R + (size_t)row_lo * row;
+    const size_t bytes = sizeof(double) * row * (size_t)n_rows;
+    if (bytes <= kShortRows) {
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        HIP_TRY(ctx, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    } else {
+        HIP_TRY(ctx, copy_to_host(ctx, {{dst, src, bytes}}));
+    }
     return BS2E_OK;
 }
 

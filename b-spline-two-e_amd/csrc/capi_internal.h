@@ -85,9 +85,10 @@ struct Piece {
 // arrays: one thread of the runtime 28 ms, so 10.1 ms (6.1 into touched ones);
 // with buffers of 2 MiB 15.4, of 4 MiB 12.0, with four threads 12.5.
 // Short transfers go through the runtime's own staging: S and H of 3 l and 50
-// splines (results of 40 and 120 KB) 150 us, by way of the ring 212; of 7 l and
-// 90 splines (130 and 907 KB) 212 against 290.  With results up to 4 MiB direct,
-// 7 l and 190 splines (0.6 and 4.0 MB) take 515 us against 448.
+// splines (results of 40 and 120 KB) 127 us, by way of the ring 212; of 7 l and
+// 90 splines (130 and 907 KB) 189 against 290; a tensor of 1.3 MB 125 against
+// 150.  With results up to 4 MiB direct, S and H of 7 l and 190 splines (0.6 and
+// 4.0 MB) take 515 us against 465.
 class HostCopier {
 public:
     ~HostCopier();
@@ -99,7 +100,7 @@ public:
 private:
     static constexpr int kBufs = 8;
     static constexpr size_t kMinBuf = (size_t)64 << 10, kMaxBuf = (size_t)8 << 20, kSlice = (size_t)256 << 10;
-    static constexpr size_t kDirectToDevice = (size_t)64 << 10, kDirectToHost = (size_t)1 << 20;
+    static constexpr size_t kDirectToDevice = (size_t)64 << 10, kDirectToHost = (size_t)2 << 20;
     struct Slice {
         void* dst;
         const void* src;

@@ -234,7 +234,8 @@ hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hip
                 const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, kind, s);
                 if (e != hipSuccess) return e;
             }
-        return hipStreamSynchronize(s);
+        // (the runtime has read a pageable source when it returns)
+        return to_host ? hipStreamSynchronize(s) : hipSuccess;
     }
     struct Part {
         void* dst;
