@@ -389,9 +389,11 @@ static int64_t run_primitives_serial(bs2e_ctx* ctx, bs2e_rk* rk)
 // The full build.
 // Up to kOneStreamBytes of tensor: two launches on the main stream, the pair
 // windows with the diagonal cells, and the near elements with the rank-one
-// fill (mixed precision: the local moments in a launch before them).  Larger: main stream pair windows (mixed precision: after the local
-// moments) -> rank-one fill; side stream (forked once the pair windows exist,
-// so that the short critical path runs alone) diagonal cells -> near elements,
+// fill (mixed precision: the local moments in a launch before them).  Larger:
+// main stream pair windows (mixed precision: after the local moments) ->
+// rank-one fill; side stream (forked once the pair windows exist, so that the
+// short critical path runs alone: cells beside the mixed gather of the windows
+// made order 8, 200 splines 150 -> 159 us) diagonal cells -> near elements,
 // concurrently with the rank-one fill; the main stream waits for the side
 // stream at the end, so the build is one unit of work on the caller's stream.
 // The line lies where hiding the cells behind the fill gains more than the

@@ -41,11 +41,11 @@ HBM_PEAK_GBS = 8000.0
 # each scaled by what the counter reads for a device copy of known size
 # (profiles/rk_build_c2.md, profiles/rk_build_c5p.md), per (workload, fill
 # shape); absent for pairs not measured that way.
-FAR_TRAFFIC_BYTES = {("c2", 0): 739.26e6, ("c2", 1): 739.82e6, ("c2", 2): 740.34e6, ("c2", 3): 739.93e6,
-                     ("c2", 4): 739.86e6, ("c2", 5): 739.71e6, ("c2", 6): 739.04e6,
-                     ("c5p", 0): 20260.12e6, ("c5p", 1): 20263.29e6, ("c5p", 2): 20273.51e6,
-                     ("c5p", 3): 20267.81e6, ("c5p", 4): 20262.35e6, ("c5p", 5): 20271.02e6,
-                     ("c5p", 6): 20259.39e6}
+FAR_TRAFFIC_BYTES = {("c2", 0): 739.99e6, ("c2", 1): 739.77e6, ("c2", 2): 740.18e6, ("c2", 3): 739.57e6,
+                     ("c2", 4): 739.29e6, ("c2", 5): 739.73e6, ("c2", 6): 739.55e6,
+                     ("c5p", 0): 20253.14e6, ("c5p", 1): 20256.53e6, ("c5p", 2): 20260.23e6,
+                     ("c5p", 3): 20251.06e6, ("c5p", 4): 20248.50e6, ("c5p", 5): 20254.19e6,
+                     ("c5p", 6): 20257.51e6}
 
 
 def log(msg):
