@@ -398,7 +398,7 @@ static int64_t run_primitives_serial(bs2e_ctx* ctx, bs2e_rk* rk)
 // stream at the end, so the build is one unit of work on the caller's stream.
 // The line lies where hiding the cells behind the fill gains more than the
 // second stream's events cost (about 20 us).  Builds one after another, one
-// stream against two: 0.0014 GB of tensor 10 us against 46, 0.016 GB 20 / 49,
+// stream against two: 0.0014 GB of tensor 10 us against 46, 0.016 GB 17 / 49,
 // 0.15 GB 45 / 59, 0.26 GB 73 / 79, 0.55 GB 131 / 135, 0.76 GB 153 / 147, 0.81 GB
 // 175 / 155, 2.7 GB 0.467 / 0.452 ms.
 // Profiling events, all relative to ev[0]: ev[1] windows done, ev[2] far

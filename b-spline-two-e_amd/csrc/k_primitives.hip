@@ -33,6 +33,7 @@
 namespace bs2e {
 
 constexpr int kPThreads = 256;
+constexpr int kFewCells = 384;   // diagonal-cell workgroups
 
 static inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
@@ -112,7 +113,7 @@ static size_t window_lds_bytes(int64_t ks, int64_t kgl, int64_t cols, int64_t kc
 // the splines of its k intervals again for that.  The local pair (ta, tc), ta <= tc, of interval c + 1 - tc is
 // the pair (c - tc + ta, c) there, so a column takes every local pair once; the
 // pair (c, a) has the same numbers.
-template <int KS>
+template <int KS, int T>
 __device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int K, int kgl,
                                                const double* __restrict__ t, const double* __restrict__ bp,
                                                const double* __restrict__ x, const double* __restrict__ w, double* lds)
@@ -134,7 +135,7 @@ __device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int 
     double* sP = sInv + npt * nk;            // [nc][U][nk]
     double* sQ = sP + nc * U * nk;           // [nc][U][nk]
     const int tid = threadIdx.x;
-    for (int e = tid; e < npt; e += kPThreads) {
+    for (int e = tid; e < npt; e += T) {
         const int iv = iv0 + e / kgl, q = e - (iv - iv0) * kgl;
         const double lim1 = bp[iv - 1], lim2 = bp[iv];
         const double r = 0.5 * (lim2 - lim1) * x[q] + 0.5 * (lim2 + lim1);
@@ -142,14 +143,14 @@ __device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int 
         splines_at<KS>(t, KS - 1 + iv, r, sB + e * KS, 1);
     }
     __syncthreads();
-    for (int e = tid; e < npt * nk; e += kPThreads) {
+    for (int e = tid; e < npt * nk; e += T) {
         const int i = e / nk, k = k0 + e - i * nk;
         const double r = sR[i];
         sPow[e] = ipow_d(r, k);
         sInv[e] = 1.0 / ipow_d(r, k + 1);
     }
     __syncthreads();
-    for (int e = tid; e < nc * U * nk; e += kPThreads) {
+    for (int e = tid; e < nc * U * nk; e += T) {
         const int cu = e / nk, kk = e - cu * nk, c = c0 + cu / U, u = cu - (c - c0) * U;
         int ta, tc;
         local_pair(u, KS, ta, tc);
@@ -168,7 +169,7 @@ __device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int 
         sQ[e] = h * accq;
     }
     __syncthreads();
-    for (int e = tid; e < 2 * nc * KS * nk; e += kPThreads) {
+    for (int e = tid; e < 2 * nc * KS * nk; e += T) {
         int r = e / nk;
         const int kk = e - r * nk, i = r % KS;      // a = c - i
         r /= KS;
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(kPThreads) void kp_windows(WindowArgs A, int K, int
                                                         const double* __restrict__ w)
 {
     extern __shared__ double lds[];
-    window_columns<KS>((int)xcd_block(blockIdx.x, A.ws.n_wg), A, K, kgl, t, bp, x, w, lds);
+    window_columns<KS, kPThreads>((int)xcd_block(blockIdx.x, A.ws.n_wg), A, K, kgl, t, bp, x, w, lds);
 }
 
 template <int KSMAX>
@@ -299,8 +300,8 @@ __global__ __launch_bounds__(kPThreads) void kw_pair_windows(WindowArgs A, int K
 // or gather them.
 enum class With { kNothing, kMoments, kGather };
 
-template <int KS, bool SYM, int KC, With WITH>
-__global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells, WindowArgs A,
+template <int KS, bool SYM, int KC, int T, With WITH>
+__global__ __launch_bounds__(T) void kp_inner(int K, int kgl, int kc, int kchunks, int n_cells, WindowArgs A,
                                                       const double* __restrict__ t, const double* __restrict__ bp,
                                                       const double* __restrict__ x, const double* __restrict__ w,
                                                       double* __restrict__ D)
@@ -314,8 +315,8 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     extern __shared__ double lds[];
     if (WITH != With::kNothing && (int)blockIdx.x >= n_cells) {
         const int wg = (int)blockIdx.x - n_cells;
-        if constexpr (WITH == With::kMoments) window_columns<KS>(wg, A, K, kgl, t, bp, x, w, lds);
-        else window_gather<KS>((int64_t)wg * kPThreads + threadIdx.x, A, K, KS);
+        if constexpr (WITH == With::kMoments) window_columns<KS, T>(wg, A, K, kgl, t, bp, x, w, lds);
+        else window_gather<KS>((int64_t)wg * T + threadIdx.x, A, K, KS);
         return;
     }
     const int npt = kgl * (1 + kgl), QP = (kgl + 3) & ~3;
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
     const int i1 = KS - 1 + (v + 1);
 
 #pragma unroll 1
-    for (int e = tid; e < npt; e += kPThreads) {
+    for (int e = tid; e < npt; e += T) {
         const bool inner = e >= kgl;
         const int q = inner ? e / kgl - 1 : e, pp = inner ? e - (q + 1) * kgl : 0;
         const double rq = h * x[q] + c;
@@ -352,10 +353,10 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
             sXr[e - kgl] = ratio;
         }
     }
-    for (int e = kgl * U + tid; e < QP * U; e += kPThreads) sWB[e] = 0.0;
+    for (int e = kgl * U + tid; e < QP * U; e += T) sWB[e] = 0.0;
     __syncthreads();
 #pragma unroll 1
-    for (int e = tid; e < kgl * U; e += kPThreads) {
+    for (int e = tid; e < kgl * U; e += T) {
         const int q = e / U, u = e - q * U;
         int ta, tc;
         local_pair(u, KS, ta, tc);
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
 #pragma unroll 1
     for (int g = 0; g < nk; g += KC) {
 #pragma unroll 1
-        for (int e = tid; e < kgl * U; e += kPThreads) {
+        for (int e = tid; e < kgl * U; e += T) {
             const int q = e / U, u = e - q * U;
             int ta, tc;
             local_pair(u, KS, ta, tc);
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
             for (int kk = 0; kk < KC; ++kk) sJ[kk * kgl * U + e] = acc[kk];
         }
         __syncthreads();
-        for (int e = tid; e < kgl * kgl; e += kPThreads) {   // (read again after the next barrier)
+        for (int e = tid; e < kgl * kgl; e += T) {   // (read again after the next barrier)
             double xk = sX[e];
 #pragma unroll
             for (int kk = 0; kk < KC; ++kk) xk *= sXr[e];
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(kPThreads) void kp_inner(int K, int kgl, int kc, in
         }
         const int left = nk - g;             // multipoles from this group on
 #pragma unroll 1
-        for (int item = wave; item < NT * NP; item += kPThreads / 64) {
+        for (int item = wave; item < NT * NP; item += T / 64) {
             const int tile = item / NP, kk = 2 * (item - tile * NP);
             if (kk >= left) continue;
             const bool two = KC > 1 && kk + 1 < left;
@@ -531,7 +532,7 @@ int inner_kc_used(const Plan& p)
     return (int)std::min<int64_t>(kc, std::max(kmax, 1));
 }
 
-template <int KS, bool SYM, int KC, With WITH>
+template <int KS, bool SYM, int KC, int T, With WITH>
 static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
 {
     const int kc = inner_kc_used(p), kchunks = (int)((p.K + kc - 1) / kc);
@@ -543,20 +544,39 @@ static void launch_inner_kc(const Plan& p, const DevTables& d, hipStream_t s)
         lds = std::max(lds, window_lds_bytes(KS, p.k_gl, A.ws.cols, A.ws.kc));
         n_wg += (unsigned)A.ws.n_wg;
     }
-    if (WITH == With::kGather) n_wg += blocks_for(p.n_pairs * p.K, kPThreads);
-    const auto fn = kp_inner<KS, SYM, KC, WITH>;
+    if (WITH == With::kGather) n_wg += blocks_for(p.n_pairs * p.K, T);
+    const auto fn = kp_inner<KS, SYM, KC, T, WITH>;
     if (allow_lds((const void*)fn, lds) != hipSuccess) return;   // the error stays for hipGetLastError
-    hipLaunchKernelGGL(fn, dim3(n_wg), dim3(kPThreads), lds, s, (int)p.K, (int)p.k_gl, kc, kchunks, n_cells, A, d.t,
+    hipLaunchKernelGGL(fn, dim3(n_wg), dim3(T), lds, s, (int)p.K, (int)p.k_gl, kc, kchunks, n_cells, A, d.t,
                        d.bp, d.x, d.w, d.D);
 }
 
+template <int KS, bool SYM, int T, With WITH>
+static void launch_inner_threads(const Plan& p, const DevTables& d, hipStream_t s)
+{
+    const int KC = inner_group(p);
+    if (KC == 4) launch_inner_kc<KS, SYM, 4, T, WITH>(p, d, s);
+    else if (KC == 2) launch_inner_kc<KS, SYM, 2, T, WITH>(p, d, s);
+    else launch_inner_kc<KS, SYM, 1, T, WITH>(p, d, s);
+}
+
+// Small builds whose cells give a CU one workgroup or little more (kFewCells)
+// take them with twice the threads: nothing else covers a stage's latency there.
+// Whole builds, 512 threads against 256: order 8, 46 splines, 5 multipoles (120
+// workgroups) 17.0 / 19.7 us, order 16, 73, 3 (116) 74 / 95, order 9, 82, 16 (304)
+// 51.1 / 54.1, order 10, 114, 9 (321) 70-72 / 75, order 12, 85, 9 (370) 75.3 / 80.7;
+// but order 8, 160, 9 (465) 82.0 / 80.6 and order 5, 189, 12 (561) 52.0 / 50.3.
+// Beside the fill on a second stream they would take its wave slots: order 8, 200
+// splines 183 / 151 us.
 template <int KS, bool SYM, With WITH>
 static void launch_inner(const Plan& p, const DevTables& d, hipStream_t s)
 {
-    const int KC = inner_group(p);
-    if (KC == 4) launch_inner_kc<KS, SYM, 4, WITH>(p, d, s);
-    else if (KC == 2) launch_inner_kc<KS, SYM, 2, WITH>(p, d, s);
-    else launch_inner_kc<KS, SYM, 1, WITH>(p, d, s);
+    if constexpr (WITH != With::kNothing) {
+        const int64_t kc = inner_kc_used(p);
+        if (p.n_iv * ((p.K + kc - 1) / kc) <= kFewCells)
+            return launch_inner_threads<KS, SYM, 2 * kPThreads, WITH>(p, d, s);
+    }
+    launch_inner_threads<KS, SYM, kPThreads, WITH>(p, d, s);
 }
 
 template <int KS>
