@@ -40,6 +40,12 @@ __device__ __forceinline__ double ipow_d(double x, int m)
     return y;
 }
 
+// The point h x + c of an interval of half-width h and centre c, rounded once.
+// Next to r = 0 the two parts nearly cancel: with the product rounded first the
+// smallest of 16 points is off by 1e-14 relative, and its power -(k + 1) by k + 1
+// times that.
+__device__ __forceinline__ double gl_point(double h, double c, double x) { return fma(h, x, c); }
+
 // All KS splines non-zero on interval iv at x: out[ls] = B_{iv+ls}(x).
 // t is stored 0-based (t(n) == t[n-1]); i1 = k-1+iv is the left knot index.
 template <int KS>

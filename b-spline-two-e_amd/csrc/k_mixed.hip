@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kMxThreads) void kp_outer_mx(int K, int kgl, const 
     const double c = 0.5 * (lim2 + lim1);
     const int i1 = KS - 1 + (v + 1);
     for (int q = tid; q < kgl; q += kMxThreads) {
-        const double r = h * x[q] + c;
+        const double r = gl_point(h, c, x[q]);
         sR[q] = r;
         splines_at<KS>(t, i1, r, sB + q * KS, 1);
     }

@@ -138,7 +138,7 @@ __device__ __forceinline__ void window_columns(int wg, const WindowArgs& A, int 
     for (int e = tid; e < npt; e += T) {
         const int iv = iv0 + e / kgl, q = e - (iv - iv0) * kgl;
         const double lim1 = bp[iv - 1], lim2 = bp[iv];
-        const double r = 0.5 * (lim2 - lim1) * x[q] + 0.5 * (lim2 + lim1);
+        const double r = gl_point(0.5 * (lim2 - lim1), 0.5 * (lim2 + lim1), x[q]);
         sR[e] = r;
         splines_at<KS>(t, KS - 1 + iv, r, sB + e * KS, 1);
     }
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(T) void kp_inner(int K, int kgl, int kc, int kchunk
     for (int e = tid; e < npt; e += T) {
         const bool inner = e >= kgl;
         const int q = inner ? e / kgl - 1 : e, pp = inner ? e - (q + 1) * kgl : 0;
-        const double rq = h * x[q] + c;
+        const double rq = gl_point(h, c, x[q]);
         const double rho = inner ? 0.5 * (rq - lim1) * x[pp] + 0.5 * (rq + lim1) : rq;
         splines_at<KS>(t, i1, rho, sB + e * KS, 1);
         if (inner) {
