@@ -507,13 +507,18 @@ static void launch_far_shape(const Plan& p, const DevTables& d, double* R, int n
 {
     constexpr FarShape f = kFarShapes[V];
     const int64_t rowlen = p.n_pairs * p.K;
+    // The fill reads its factors two elements at a time.  A row of one element
+    // (one basis function, one multipole) has none that is rank-one: its pair
+    // overlaps itself.
+    const bool fill = rowlen > 1;
+    if (!fill && near < 0) return;
     const int64_t per = 2 * (int64_t)kThreads * f.iters;
     // (a shifted row's last elements lie up to 15 past its last chunk)
     const unsigned cols = (unsigned)((rowlen + (f.shift ? kFarLine - 1 : 0) + per - 1) / per);
     const unsigned x_cols = 2 * sizeof(double) * rowlen > kFarSliceBytes ? (cols + kXcds - 1) / kXcds : 0;
     const unsigned gx = x_cols ? kXcds * x_cols : cols;
     const unsigned near_y = near >= 0 ? (unsigned)((p.rows.size() + gx - 1) / gx) : 0;
-    const unsigned gy = (unsigned)((p.n_pairs + f.rows - 1) / f.rows) + near_y;
+    const unsigned gy = (fill ? (unsigned)((p.n_pairs + f.rows - 1) / f.rows) : 0) + near_y;
     const dim3 grid(gx, std::min(gy, kFarGridY), (gy + kFarGridY - 1) / kFarGridY);
     const FarArgs a{(int)p.n_pairs, (int)p.n_b, (int)p.K, (int)p.k_s, recip32(p.K), recip32(p.K + 1), (int)cols,
                     (int)x_cols, d.pairs, d.c_first, d.Ptot, d.Qtot, R};

@@ -90,3 +90,28 @@ def test_fill_shapes_at_edges(k, n_b, k_GL, max_k, oracle):
     assert (len(shapes) == 7) == (rk.n_pairs * rk.K % 2 == 0) and shapes
     rk.release()
     ctx.close()
+
+
+@pytest.mark.parametrize("max_k", [0, 1, 2])
+@pytest.mark.parametrize("k", [2, 3])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_one_basis_function(k, max_k, precision, oracle):
+    """Rows of one, two and three elements, none of them rank-one, by every shape that takes them and the default."""
+    t = _knots(k, 1)
+    assert len(t) - k - 2 == 1
+    ref = oracle.rk_dense(k, 1, max_k, oracle.slater_off_diag(k, t, 6, max_k), oracle.slater_diag(k, t, 6, max_k))
+    tol = 1e-12 if precision == "fp64" else 1e-10
+    ctx = bs2e.Context(0)
+    for shape in (None, *range(7)):
+        rk = bs2e.RkTensor.build(k, t, 6, max_k, ctx=ctx, compute=False, precision=precision)
+        try:
+            if shape is not None:
+                rk.set_tuning(shape, 1)
+        except bs2e.Bs2eError:
+            assert shape < 5 and rk.K % 2 == 1
+            continue
+        _fill_nan(rk)
+        rk.compute()
+        assert np.all(np.abs(rk.to_host() - ref) <= tol * np.abs(ref)), shape
+        rk.release()
+    ctx.close()
