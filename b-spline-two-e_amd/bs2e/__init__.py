@@ -56,6 +56,10 @@ class Context:
     def set_stream(self, stream_ptr: int | None):
         check(capi.lib().bs2e_set_stream(self.handle, C.c_void_p(stream_ptr) if stream_ptr else None), self.handle)
 
+    def trim(self):
+        """Gives the device memory kept from released handles back (bs2e_trim)."""
+        check(capi.lib().bs2e_trim(self.handle), self.handle)
+
     def close(self):
         if self.handle:
             capi.lib().bs2e_destroy(self.handle)

@@ -32,6 +32,7 @@ PREC_MIXED = 1
 SIGNATURES = [
     ("bs2e_create", i64, [P(vp), i64]),
     ("bs2e_destroy", i64, [vp]),
+    ("bs2e_trim", i64, [vp]),
     ("bs2e_last_error", C.c_char_p, [vp]),
     ("bs2e_set_stream", i64, [vp, vp]),
     ("bs2e_generate_grid", i64, [i64, i64, i64, dbl, dbl, P(dbl), i64]),

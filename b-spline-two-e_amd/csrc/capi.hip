@@ -86,6 +86,14 @@ int64_t bs2e_set_stream(bs2e_ctx* ctx, void* hip_stream)
     return BS2E_OK;
 }
 
+int64_t bs2e_trim(bs2e_ctx* ctx)
+{
+    if (!ctx) return fail(nullptr, BS2E_EINVAL, "bs2e_trim: ctx is NULL");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    ctx->pool.trim(0);
+    return BS2E_OK;
+}
+
 int64_t bs2e_generate_grid(int64_t k, int64_t m, int64_t Z, double h_max, double r_max, double* knots, int64_t cap)
 {
     if (k < 1 || m < 0 || m > 60 || Z < 1 || !(h_max > 0.0) || !(r_max > 0.0))
@@ -135,10 +143,10 @@ double bs2e_six_j(int64_t j1, int64_t j2, int64_t j3, int64_t j4, int64_t j5, in
 // ---------------------------------------------------------------------------
 // device arena
 // ---------------------------------------------------------------------------
-hipError_t bs2e::Arena::init(size_t bytes)
+hipError_t bs2e::Arena::init(size_t bytes, int device)
 {
     bytes = (bytes + 255) / 256 * 256;
-    hipError_t e = hipMalloc((void**)&base_, bytes);
+    hipError_t e = device_malloc(device, (void**)&base_, bytes);
     if (e != hipSuccess) {
         base_ = nullptr;
         return e;

@@ -22,7 +22,7 @@ namespace bs2e {
 // (hipFree waits for the whole device).  Host-side bookkeeping only.
 class Arena {
 public:
-    hipError_t init(size_t bytes);
+    hipError_t init(size_t bytes, int device);
     void destroy();
     void* alloc(size_t bytes);   // 256-byte aligned; nullptr when no free range fits
     void release(void* p);
@@ -42,16 +42,22 @@ private:
 // of about its size, because the driver clears what it hands out again (a
 // 0.76 GB tensor released and created: 25 ms, most of it the clearing).  At
 // most kMaxKept bytes and kMaxBlocks blocks are kept, the longest unused go
-// first; all of them go when an allocation fails and with the context.  A
-// release waits for the device, as hipFree does, once per QuietScope.
+// first; all of them go with the context, by bs2e_trim, and when an allocation
+// of the library on that device fails, whichever context or arena it is for.
+// A release waits for the device, as hipFree does, once per QuietScope.
 class DevicePool {
 public:
+    DevicePool();
+    ~DevicePool();
+    DevicePool(const DevicePool&) = delete;
     hipError_t alloc(void** out, size_t bytes);
     void release(void* p);
     void trim(size_t keep);
+    static void trim_device(int device);   // every pool of the device
     int device = 0;
 
 private:
+    DevicePool *prev_ = nullptr, *next_ = nullptr;   // the process's pools
     struct Kept {
         void* ptr;
         uint64_t stamp;
@@ -63,6 +69,10 @@ private:
     size_t kept_bytes_ = 0;
     uint64_t stamp_ = 0;
 };
+
+// hipMalloc on `device` (the current one); a failure for want of memory takes
+// what the device's pools keep and is tried once more.
+hipError_t device_malloc(int device, void** out, size_t bytes);
 
 // Releases of the calling thread inside one scope wait for the device once.
 struct QuietScope {

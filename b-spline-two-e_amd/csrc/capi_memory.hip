@@ -23,6 +23,44 @@ QuietScope::~QuietScope()
     if (--t_quiet_depth == 0) t_quiet = false;
 }
 
+namespace {
+std::mutex g_pools_mu;               // held before a pool's own
+DevicePool* g_pools = nullptr;
+}  // namespace
+
+DevicePool::DevicePool()
+{
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    next_ = g_pools;
+    if (next_) next_->prev_ = this;
+    g_pools = this;
+}
+
+DevicePool::~DevicePool()
+{
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    (prev_ ? prev_->next_ : g_pools) = next_;
+    if (next_) next_->prev_ = prev_;
+}
+
+void DevicePool::trim_device(int device)
+{
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    for (DevicePool* p = g_pools; p; p = p->next_)
+        if (p->device == device) p->trim(0);
+}
+
+hipError_t device_malloc(int device, void** out, size_t bytes)
+{
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        DevicePool::trim_device(device);
+        e = hipMalloc(out, bytes);
+    }
+    return e;
+}
+
 hipError_t DevicePool::alloc(void** out, size_t bytes)
 {
     *out = nullptr;
@@ -39,12 +77,7 @@ hipError_t DevicePool::alloc(void** out, size_t bytes)
             return hipSuccess;
         }
     }
-    hipError_t e = hipMalloc(out, need);
-    if (e == hipErrorOutOfMemory) {   // give everything back and try once more
-        (void)hipGetLastError();
-        trim(0);
-        e = hipMalloc(out, need);
-    }
+    const hipError_t e = device_malloc(device, out, need);
     if (e != hipSuccess) {
         *out = nullptr;
         return e;

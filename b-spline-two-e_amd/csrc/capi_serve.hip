@@ -463,7 +463,7 @@ int64_t bs2e_server_create(int64_t device, int64_t hbm_bytes, int64_t slots, bs2
         return rc;
     }
     (void)hipSetDevice(s->device);
-    hipError_t e = s->arena.init((size_t)hbm_bytes);
+    hipError_t e = s->arena.init((size_t)hbm_bytes, s->device);
     if (e != hipSuccess) {
         bs2e_destroy(s->err);
         delete s;

@@ -52,10 +52,16 @@ typedef struct bs2e_rk bs2e_rk;   /* one basis and its device-resident R^k tenso
  * stream.  (No reference counterpart: the reference runs on the host.) */
 int64_t bs2e_create(bs2e_ctx **ctx, int64_t device);
 /* A context keeps up to 4 GiB of the device memory its handles have released
- * for later ones, and up to 64 MiB of pinned host memory and eight threads for
- * copies of results to the host; bs2e_destroy gives all of it back, and an
- * allocation that fails the kept device memory. */
+ * for later ones (1.4 % of the card), and up to 64 MiB of pinned host memory and
+ * eight threads for copies of results to the host; bs2e_destroy gives all of it
+ * back.  The kept device memory also goes back by bs2e_trim, and when an
+ * allocation of this library on the same device fails, whichever context or
+ * service it is for (it is then tried again); another allocator in the process
+ * does not see it. */
 int64_t bs2e_destroy(bs2e_ctx *ctx);
+/* Gives the device memory that the context keeps, and no handle holds, back to
+ * the device.  (No reference counterpart.) */
+int64_t bs2e_trim(bs2e_ctx *ctx);
 const char *bs2e_last_error(const bs2e_ctx *ctx);
 /* Runs the context's device work on `hip_stream` (a hipStream_t) instead of
  * its own stream; NULL restores the context's stream. */

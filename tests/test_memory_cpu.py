@@ -1,0 +1,99 @@
+"""The library's device blocks and host copies without a device, over a stand-in
+for the HIP runtime (fake_hip.cpp): each scenario in a process of its own, as the
+stand-in has to be loaded before the library.
+"""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+K, K_GL, MAX_K = 4, 6, 2
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "fake_hip.cpp"), "-o", so,
+                    "-lpthread"], check=True)
+    return so
+
+
+# ------------------------------------------------------------- in the process
+def _load(so):
+    sys.path.insert(0, os.path.join(ROOT, "b-spline-two-e_amd"))
+    f = C.CDLL(so, mode=C.RTLD_GLOBAL)
+    for name, res, args in (("fake_capacity", None, [C.c_size_t]), ("fake_used", C.c_size_t, []),
+                            ("fake_mallocs", C.c_int64, []), ("fake_memcpys", C.c_int64, []),
+                            ("fake_fail_new", None, [C.c_int]), ("fake_stream", C.c_void_p, [C.c_int]),
+                            ("fake_block", None, [C.c_void_p, C.c_int]), ("fake_pinned", C.c_void_p, [C.c_size_t]),
+                            ("fake_holds", C.c_int, [C.c_void_p, C.c_size_t])):
+        getattr(f, name).restype = res
+        getattr(f, name).argtypes = args
+    import bs2e
+    bs2e.capi.lib()
+    return f, bs2e
+
+
+def _knots(bs2e, r_max):
+    return bs2e.generate_grid(K, 3, 2, 1.0, r_max)
+
+
+def scenario_other_contexts_give_back(f, bs2e):
+    """An allocation that fails takes what other contexts of the device keep."""
+    a, b = bs2e.Context(0), bs2e.Context(0)
+    t = _knots(bs2e, 40.0)
+    rk = bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=a, compute=False)
+    need = f.fake_used()
+    rk.release()
+    assert f.fake_used() == need          # kept
+    f.fake_capacity(need + need // 2)
+    bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=b, compute=False).release()
+    s = bs2e.Server(need + need // 4, 1)      # a service's arena is one allocation
+    s.close()
+
+
+def scenario_other_devices_keep(f, bs2e):
+    """Blocks kept on another device are left alone."""
+    a, b = bs2e.Context(0), bs2e.Context(1)
+    t = _knots(bs2e, 40.0)
+    bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=a, compute=False).release()
+    kept = f.fake_used()
+    f.fake_capacity(kept + kept // 2)
+    with pytest.raises(bs2e.Bs2eError):
+        bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=b, compute=False)
+    b.close()
+    assert f.fake_used() == kept
+
+
+def scenario_trim_gives_back(f, bs2e):
+    """Context.trim returns what no handle holds, and nothing else."""
+    ctx = bs2e.Context(0)
+    t = _knots(bs2e, 40.0)
+    held = bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=ctx, compute=False)
+    used = f.fake_used()
+    bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=ctx, compute=False).release()
+    assert f.fake_used() > used
+    ctx.trim()
+    assert f.fake_used() == used
+    held.release()
+    ctx.close()
+    assert f.fake_used() == 0
+
+
+SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
+
+
+@pytest.mark.parametrize("name", SCENARIOS)
+def test_scenario(name, fake):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake, name], stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-4000:]
+
+
+if __name__ == "__main__":
+    globals()["scenario_" + sys.argv[2]](*_load(sys.argv[1]))
