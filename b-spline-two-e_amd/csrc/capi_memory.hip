@@ -70,8 +70,12 @@ hipError_t DevicePool::alloc(void** out, size_t bytes)
         // the smallest kept block that holds it without wasting more than a quarter
         auto it = kept_.lower_bound(need);
         if (it != kept_.end() && it->first <= need + need / 4 + ((size_t)64 << 10)) {
+            try {
+                live_.emplace(it->second.ptr, it->first);
+            } catch (...) {
+                return hipErrorOutOfMemory;
+            }
             *out = it->second.ptr;
-            live_[*out] = it->first;
             kept_bytes_ -= it->first;
             kept_.erase(it);
             return hipSuccess;
@@ -82,8 +86,14 @@ hipError_t DevicePool::alloc(void** out, size_t bytes)
         *out = nullptr;
         return e;
     }
-    std::lock_guard<std::mutex> lk(mu_);
-    live_[*out] = need;
+    try {
+        std::lock_guard<std::mutex> lk(mu_);
+        live_.emplace(*out, need);
+    } catch (...) {
+        (void)hipFree(*out);
+        *out = nullptr;
+        return hipErrorOutOfMemory;
+    }
     return hipSuccess;
 }
 
@@ -107,9 +117,12 @@ void DevicePool::release(void* p)
             live_.erase(it);
         }
         if (idle && size > 0 && size <= kMaxKept) {
-            kept_.emplace(size, Kept{p, ++stamp_});
-            kept_bytes_ += size;
-            p = nullptr;
+            try {
+                kept_.emplace(size, Kept{p, ++stamp_});
+                kept_bytes_ += size;
+                p = nullptr;
+            } catch (...) {   // no memory for the entry: the block goes back
+            }
         }
     }
     if (p) (void)hipFree(p);

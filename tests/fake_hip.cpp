@@ -29,6 +29,13 @@ size_t capacity = (size_t)1 << 40, used = 0;
 int64_t n_malloc = 0, n_memcpy = 0;
 thread_local int fail_new_after = -1;   // allocations of this thread until one fails (< 0: none does)
 
+// the stand-in's own allocations do not count
+struct Own {
+    const int keep = fail_new_after;
+    Own() { fail_new_after = -1; }
+    ~Own() { fail_new_after = keep; }
+};
+
 constexpr int kOk = 0, kInvalid = 1, kNoMemory = 2, kNotReady = 600;
 
 bool lives(Stream* s)
@@ -82,6 +89,7 @@ int fake_holds(const void* p, size_t n)
 }
 void* fake_pinned(size_t n)
 {
+    Own own;
     std::lock_guard<std::mutex> lk(mu);
     void* p = std::calloc(n, 1);
     pinned[p] = n;
@@ -106,6 +114,7 @@ int hipDeviceSynchronize()
 }
 int hipMalloc(void** p, size_t n)
 {
+    Own own;
     std::lock_guard<std::mutex> lk(mu);
     *p = nullptr;
     if (used + n > capacity) return kNoMemory;
@@ -136,6 +145,7 @@ int hipHostFree(void* p)
 }
 int hipStreamCreateWithFlags(void** s, unsigned)
 {
+    Own own;
     std::lock_guard<std::mutex> lk(mu);
     streams.push_back(new Stream);
     *s = streams.back();
@@ -151,8 +161,12 @@ int hipStreamDestroy(void* s)
 int hipStreamSynchronize(void* s) { return wait_for((Stream*)s); }
 int hipStreamWaitEvent(void*, void*, unsigned) { return kOk; }
 int hipStreamIsCapturing(void*, int* st) { return *st = 0, kOk; }
-int hipEventCreate(void** e) { return *e = new Event, kOk; }
-int hipEventCreateWithFlags(void** e, unsigned) { return *e = new Event, kOk; }
+int hipEventCreate(void** e)
+{
+    Own own;
+    return *e = new Event, kOk;
+}
+int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
 int hipEventDestroy(void* e) { return delete (Event*)e, kOk; }
 int hipEventRecord(void* e, void* s) { return ((Event*)e)->on = (Stream*)s, kOk; }
 int hipEventSynchronize(void* e) { return wait_for(((Event*)e)->on); }

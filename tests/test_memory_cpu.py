@@ -85,6 +85,34 @@ def scenario_trim_gives_back(f, bs2e):
     assert f.fake_used() == 0
 
 
+def scenario_host_memory_runs_out(f, bs2e):
+    """Host allocations that fail in the middle of a call that only moves device
+    blocks end in an error code or in a block given back, never in an exception."""
+    ctx = bs2e.Context(0)
+    t = _knots(bs2e, 20.0)
+    rk = bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=ctx)
+    n_b = len(t) - K - 2
+    cfg = bs2e.count_configs(bs2e.sym(0), 1, n_b, K, n_b, n_b, 1)
+    L, n = (C.c_int64 * 1)(0), (C.c_int64 * 1)(len(cfg))
+    cfg = np.ascontiguousarray(cfg, np.int64)
+    lib, codes = bs2e.capi.lib(), set()
+    for fail_at in range(12):
+        h = C.c_void_p()
+        bs2e.capi.check(lib.bs2e_blockset_create(rk.handle, 1, L, n, cfg.ctypes.data_as(C.POINTER(C.c_int64)), 1,
+                                                 C.byref(h)), ctx.handle)
+        for size in (1000, 5000, 1000):     # (later rounds take kept blocks)
+            f.fake_fail_new(fail_at)
+            codes.add(lib.bs2e_blockset_reserve(h, size * (fail_at + 1), size * (fail_at + 1)))
+            f.fake_fail_new(-1)
+        f.fake_fail_new(fail_at)
+        codes.add(lib.bs2e_blockset_release(h))
+        f.fake_fail_new(-1)
+    assert codes == {0, bs2e.capi.BS2E_ENOMEM}, codes
+    rk.release()
+    ctx.close()
+    assert f.fake_used() == 0
+
+
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
 
 
