@@ -2,6 +2,7 @@
 #pragma once
 
 #include <array>
+#include <atomic>
 #include <condition_variable>
 #include <deque>
 #include <initializer_list>
@@ -99,8 +100,12 @@ struct Piece {
 // 90 splines (130 and 907 KB) 189 against 290; a tensor of 1.3 MB 125 against
 // 150.  With results up to 4 MiB direct, S and H of 7 l and 190 splines (0.6 and
 // 4.0 MB) take 515 us against 465.
+// A transfer has a ring of its own while it runs, of at most max_rings (a
+// service's slots share one copier and may be read by a thread each: none waits
+// for another's stream or transfer); the threads are shared, and only copy.
 class HostCopier {
 public:
+    explicit HostCopier(int max_rings) : max_rings_(max_rings) {}
     ~HostCopier();
     // to_host: returns when every piece is in place; otherwise when the
     // pieces have been read and their copies enqueued on s.
@@ -111,27 +116,39 @@ private:
     static constexpr int kBufs = 8;
     static constexpr size_t kMinBuf = (size_t)64 << 10, kMaxBuf = (size_t)8 << 20, kSlice = (size_t)256 << 10;
     static constexpr size_t kDirectToDevice = (size_t)64 << 10, kDirectToHost = (size_t)2 << 20;
+    struct Ring {
+        char* pin = nullptr;
+        size_t buf = 0;                // bytes of a buffer
+        hipEvent_t ev[kBufs] = {};     // behind the copies of a buffer
+        bool in_flight[kBufs] = {};
+        int pending[kBufs] = {};       // slices not copied yet (mu_)
+        bool taken = false;            // (rings_mu_)
+        bool prepare(size_t total);
+        void drop();
+        bool idle();
+    };
     struct Slice {
         void* dst;
         const void* src;
         size_t bytes;
-        int buf;
+        int* pending;
     };
-    bool prepare(size_t total);
-    void drop_ring();
+    Ring* take();
+    void give(Ring* r);
+    void start_threads(size_t total);
     void run();
-    void spread(void* dst, const void* src, size_t bytes, int buf);
-    void wait_slices(int buf);
-    std::mutex call_mu_, mu_;
-    std::condition_variable work_, done_;
+    void spread(void* dst, const void* src, size_t bytes, int* pending);
+    void wait_slices(const int* pending);
+    hipError_t through(Ring& r, const Piece* pieces, size_t n, bool to_host, hipStream_t s);
+    const int max_rings_;
+    std::mutex rings_mu_, mu_;
+    std::condition_variable rings_cv_, work_, done_;
+    std::vector<std::unique_ptr<Ring>> rings_;
     std::deque<Slice> queue_;
-    int pending_[kBufs] = {};
     bool stop_ = false;
+    std::once_flag threads_once_;
+    std::atomic<bool> has_threads_{false};
     std::vector<std::thread> threads_;
-    char* pin_ = nullptr;
-    size_t buf_ = 0;
-    hipEvent_t ev_[kBufs] = {};
-    bool in_flight_[kBufs] = {};
 };
 
 }  // namespace bs2e

@@ -159,47 +159,104 @@ HostCopier::~HostCopier()
     }
     work_.notify_all();
     for (std::thread& t : threads_) t.join();
-    drop_ring();
+    for (auto& r : rings_) r->drop();
 }
 
-void HostCopier::drop_ring()
+void HostCopier::Ring::drop()
 {
     for (int b = 0; b < kBufs; ++b) {
-        if (ev_[b]) {
-            if (in_flight_[b]) (void)hipEventSynchronize(ev_[b]);
-            (void)hipEventDestroy(ev_[b]);
+        if (ev[b]) {
+            if (in_flight[b]) (void)hipEventSynchronize(ev[b]);
+            (void)hipEventDestroy(ev[b]);
         }
-        ev_[b] = nullptr;
-        in_flight_[b] = false;
+        ev[b] = nullptr;
+        in_flight[b] = false;
     }
-    if (pin_) (void)hipHostFree(pin_);
-    pin_ = nullptr;
-    buf_ = 0;
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    buf = 0;
 }
 
-// kBufs pinned buffers, an eighth of the copy each (64 KiB to 8 MiB), and for
-// copies of some size the threads.
-bool HostCopier::prepare(size_t total)
+// Whether all its copies have run.
+bool HostCopier::Ring::idle()
+{
+    for (int b = 0; b < kBufs; ++b) {
+        if (in_flight[b] && hipEventQuery(ev[b]) != hipSuccess) return false;
+        in_flight[b] = false;
+    }
+    return true;
+}
+
+// kBufs pinned buffers, an eighth of the copy each (64 KiB to 8 MiB).
+bool HostCopier::Ring::prepare(size_t total)
 {
     size_t want = kMinBuf;
     while (want < kMaxBuf && want * kBufs < total) want *= 2;
-    if (want > buf_) {
-        drop_ring();
-        if (hipHostMalloc((void**)&pin_, want * kBufs, hipHostMallocDefault) != hipSuccess) {
+    if (want <= buf) return true;
+    drop();
+    if (hipHostMalloc((void**)&pin, want * kBufs, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        pin = nullptr;
+        return false;
+    }
+    buf = want;
+    for (int b = 0; b < kBufs; ++b)
+        if (hipEventCreateWithFlags(&ev[b], hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
-            pin_ = nullptr;
+            ev[b] = nullptr;
+            drop();
             return false;
         }
-        buf_ = want;
-        for (int b = 0; b < kBufs; ++b)
-            if (hipEventCreateWithFlags(&ev_[b], hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                ev_[b] = nullptr;
-                drop_ring();
-                return false;
+    return true;
+}
+
+// A ring for one transfer: one whose copies have all run, else a new one, else
+// one that still uploads behind its stream's work, else the next given back;
+// nullptr where there is no memory for the first.
+HostCopier::Ring* HostCopier::take()
+{
+    std::unique_lock<std::mutex> lk(rings_mu_);
+    for (;;) {
+        Ring* busy = nullptr;
+        for (auto& r : rings_) {
+            if (r->taken) continue;
+            if (r->idle()) {
+                r->taken = true;
+                return r.get();
             }
+            busy = r.get();
+        }
+        if ((int)rings_.size() < max_rings_) {
+            try {
+                rings_.push_back(std::make_unique<Ring>());
+                rings_.back()->taken = true;
+                return rings_.back().get();
+            } catch (...) {
+                if (rings_.empty()) return nullptr;
+            }
+        }
+        if (busy) {
+            busy->taken = true;
+            return busy;
+        }
+        rings_cv_.wait(lk);
     }
-    if (threads_.empty() && total > kSlice) {
+}
+
+void HostCopier::give(Ring* r)
+{
+    {
+        std::lock_guard<std::mutex> lk(rings_mu_);
+        r->taken = false;
+    }
+    rings_cv_.notify_one();
+}
+
+// For copies of some size, once.
+void HostCopier::start_threads(size_t total)
+{
+    if (total <= kSlice || has_threads_) return;
+    std::call_once(threads_once_, [this] {
         cpu_set_t set;
         int n = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) / 2 : 1;
         n = std::min(8, n);
@@ -207,8 +264,8 @@ bool HostCopier::prepare(size_t total)
             for (int i = 0; i < n; ++i) threads_.emplace_back([this] { run(); });
         } catch (...) {   // fewer threads, or none: the caller copies
         }
-    }
-    return true;
+        has_threads_ = !threads_.empty();
+    });
 }
 
 void HostCopier::run()
@@ -222,15 +279,15 @@ void HostCopier::run()
         lk.unlock();
         std::memcpy(s.dst, s.src, s.bytes);
         lk.lock();
-        if (--pending_[s.buf] == 0) done_.notify_all();
+        if (--*s.pending == 0) done_.notify_all();
     }
 }
 
-// Copies src to dst in slices on the threads (counted for buffer buf), or here
+// Copies src to dst in slices on the threads (counted in *pending), or here
 // when it is short or there are none.
-void HostCopier::spread(void* dst, const void* src, size_t bytes, int buf)
+void HostCopier::spread(void* dst, const void* src, size_t bytes, int* pending)
 {
-    if (threads_.empty() || bytes <= kSlice / 2) {
+    if (!has_threads_ || bytes <= kSlice / 2) {
         std::memcpy(dst, src, bytes);
         return;
     }
@@ -238,51 +295,60 @@ void HostCopier::spread(void* dst, const void* src, size_t bytes, int buf)
         std::unique_lock<std::mutex> lk(mu_);
         for (size_t o = 0; o < bytes; o += kSlice) {
             try {
-                queue_.push_back(Slice{(char*)dst + o, (const char*)src + o, std::min(kSlice, bytes - o), buf});
+                queue_.push_back(Slice{(char*)dst + o, (const char*)src + o, std::min(kSlice, bytes - o), pending});
             } catch (...) {   // no memory for the entry: the rest here
                 lk.unlock();
                 std::memcpy((char*)dst + o, (const char*)src + o, bytes - o);
                 break;
             }
-            ++pending_[buf];
+            ++*pending;
         }
     }
     work_.notify_all();
 }
 
-void HostCopier::wait_slices(int buf)
+void HostCopier::wait_slices(const int* pending)
 {
     std::unique_lock<std::mutex> lk(mu_);
-    done_.wait(lk, [this, buf] { return pending_[buf] == 0; });
+    done_.wait(lk, [pending] { return *pending == 0; });
 }
 
 void HostCopier::copy(void* dst, const void* src, size_t bytes)
 {
-    std::lock_guard<std::mutex> call(call_mu_);
-    if (!prepare(bytes)) {
-        std::memcpy(dst, src, bytes);
-        return;
-    }
-    spread(dst, src, bytes, 0);
-    wait_slices(0);
+    start_threads(bytes);
+    int pending = 0;
+    spread(dst, src, bytes, &pending);
+    wait_slices(&pending);
 }
 
 hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hipStream_t s)
 {
-    std::lock_guard<std::mutex> call(call_mu_);
     size_t total = 0;
     for (size_t i = 0; i < n; ++i) total += pieces[i].bytes;
     if (total == 0) return to_host ? hipStreamSynchronize(s) : hipSuccess;
-    const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
-    if (total <= (to_host ? kDirectToHost : kDirectToDevice) || !prepare(total)) {
-        for (size_t i = 0; i < n; ++i)
-            if (pieces[i].bytes > 0) {
-                const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes, kind, s);
-                if (e != hipSuccess) return e;
-            }
-        // (the runtime has read a pageable source when it returns)
-        return to_host ? hipStreamSynchronize(s) : hipSuccess;
+    if (Ring* r = total > (to_host ? kDirectToHost : kDirectToDevice) ? take() : nullptr) {
+        const bool ready = r->prepare(total);
+        hipError_t e = hipSuccess;
+        if (ready) {
+            start_threads(total);
+            e = through(*r, pieces, n, to_host, s);
+        }
+        give(r);
+        if (ready) return e;
     }
+    for (size_t i = 0; i < n; ++i)
+        if (pieces[i].bytes > 0) {
+            const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes,
+                                                to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
+            if (e != hipSuccess) return e;
+        }
+    // (the runtime has read a pageable source when it returns)
+    return to_host ? hipStreamSynchronize(s) : hipSuccess;
+}
+
+hipError_t HostCopier::through(Ring& r, const Piece* pieces, size_t n, bool to_host, hipStream_t s)
+{
+    const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
     struct Part {
         void* dst;
         const void* src;
@@ -297,17 +363,17 @@ hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hip
     while (e == hipSuccess && (pi < n || tail < head)) {
         if (pi < n && head - tail < kBufs) {
             const int b = (int)(head % kBufs);
-            wait_slices(b);
-            if (in_flight_[b]) {
-                e = hipEventSynchronize(ev_[b]);
-                in_flight_[b] = false;
+            wait_slices(&r.pending[b]);
+            if (r.in_flight[b]) {
+                e = hipEventSynchronize(r.ev[b]);
+                r.in_flight[b] = false;
             }
-            char* const base = pin_ + (size_t)b * buf_;
+            char* const base = r.pin + (size_t)b * r.buf;
             size_t used = 0;
             n_parts[b] = 0;
-            while (pi < n && used < buf_ && n_parts[b] < kParts) {
+            while (pi < n && used < r.buf && n_parts[b] < kParts) {
                 const Piece& p = pieces[pi];
-                const size_t m = std::min(p.bytes - po, buf_ - used);
+                const size_t m = std::min(p.bytes - po, r.buf - used);
                 if (m > 0) {
                     char* const mine = base + used;
                     char* const dst = (char*)p.dst + po;
@@ -315,7 +381,7 @@ hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hip
                     if (to_host) {
                         if (e == hipSuccess) e = hipMemcpyAsync(mine, src, m, kind, s);
                     } else {
-                        spread(mine, src, m, b);
+                        spread(mine, src, m, &r.pending[b]);
                     }
                     parts[b][n_parts[b]++] = Part{dst, mine, m};
                     used += (m + 255) / 256 * 256;
@@ -327,26 +393,26 @@ hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hip
                 }
             }
             if (!to_host) {
-                wait_slices(b);
+                wait_slices(&r.pending[b]);
                 for (int i = 0; i < n_parts[b] && e == hipSuccess; ++i)
                     e = hipMemcpyAsync(parts[b][i].dst, parts[b][i].src, parts[b][i].bytes, kind, s);
             }
-            if (e == hipSuccess) e = hipEventRecord(ev_[b], s);
-            in_flight_[b] = e == hipSuccess;
+            if (e == hipSuccess) e = hipEventRecord(r.ev[b], s);
+            r.in_flight[b] = e == hipSuccess;
             ++head;
             if (!to_host) tail = head;   // (the buffer is free once its event has passed)
             continue;
         }
         const int b = (int)(tail % kBufs);
-        e = hipEventSynchronize(ev_[b]);
-        in_flight_[b] = false;
+        e = hipEventSynchronize(r.ev[b]);
+        r.in_flight[b] = false;
         if (e == hipSuccess)
-            for (int i = 0; i < n_parts[b]; ++i) spread(parts[b][i].dst, parts[b][i].src, parts[b][i].bytes, b);
+            for (int i = 0; i < n_parts[b]; ++i) spread(parts[b][i].dst, parts[b][i].src, parts[b][i].bytes, &r.pending[b]);
         ++tail;
     }
     if (e != hipSuccess) (void)hipStreamSynchronize(s);   // nothing reads or writes the buffers any more
     if (to_host)
-        for (int b = 0; b < kBufs; ++b) wait_slices(b);
+        for (int b = 0; b < kBufs; ++b) wait_slices(&r.pending[b]);
     return e;
 }
 
@@ -355,7 +421,7 @@ HostCopier* ctx_copier(bs2e_ctx* c)
     std::lock_guard<std::mutex> lk(c->up_mu);
     if (!c->copier) {
         try {
-            c->copier = std::make_shared<HostCopier>();
+            c->copier = std::make_shared<HostCopier>(1);
         } catch (...) {
             return nullptr;
         }

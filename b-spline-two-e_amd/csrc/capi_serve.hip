@@ -470,13 +470,17 @@ int64_t bs2e_server_create(int64_t device, int64_t hbm_bytes, int64_t slots, bs2
         return fail(nullptr, e == hipErrorOutOfMemory ? BS2E_ENOMEM : BS2E_EDEVICE,
                     std::string("bs2e_server_create: ") + hipGetErrorString(e));
     }
+    std::shared_ptr<HostCopier> copier;   // one set of copy threads, a ring for each slot that is read
+    try {
+        copier = std::make_shared<HostCopier>((int)slots);
+    } catch (...) {   // (the slots make their own)
+    }
     for (int64_t i = 0; i < slots; ++i) {
         bs2e_ctx* c = nullptr;
         rc = bs2e_create(&c, device);
         if (rc) break;
         c->arena = &s->arena;
-        if (!s->slots.empty()) c->copier = s->slots.front()->copier;   // one set of copy threads and buffers
-        else (void)ctx_copier(c);
+        c->copier = copier;
         s->slots.push_back(c);
         s->slot_job.push_back(-1);
     }

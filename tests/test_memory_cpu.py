@@ -6,6 +6,8 @@ import ctypes as C
 import os
 import subprocess
 import sys
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -111,6 +113,104 @@ def scenario_host_memory_runs_out(f, bs2e):
     rk.release()
     ctx.close()
     assert f.fake_used() == 0
+
+
+def _write(rk, values):
+    p, n = rk.device_ptr()
+    assert n == values.size
+    C.memmove(p, values.ctypes.data, values.nbytes)
+
+
+def scenario_service_reads_overlap(f, bs2e):
+    """A job's results are read while another slot's stream is busy, and while a
+    thread waits for that slot's: long reads, middle ones and the copy out of the mirror."""
+    s = bs2e.Server(1 << 30, 2)
+    slot0 = f.fake_stream(2)              # streams: two of the service's own context, two of each slot
+    t = _knots(bs2e, 80.0)
+    f.fake_block(slot0, 1)
+    a = s.submit(K, t, K_GL, MAX_K)
+    b = s.submit(K, t, K_GL, MAX_K)
+    s.wait(b)
+    f.fake_block(slot0, 0)
+    s.wait(a)
+    ra, rb = s.tensor(a), s.tensor(b)
+    va, vb = (np.random.default_rng(i).random(ra.device_ptr()[1]) for i in (0, 1))
+    assert va.nbytes > 4 << 20
+    _write(ra, va)
+    _write(rb, vb)
+    f.fake_block(slot0, 1)
+    got = {}
+
+    def read(name, rk):
+        got[name] = rk.to_host().ravel()
+
+    def middle(name, rk):
+        out = np.empty((20, rk.n_pairs, rk.K))
+        assert 16 << 10 < out.nbytes < 2 << 20
+        bs2e.capi.check(bs2e.capi.lib().bs2e_rk_copy_rows(rk.handle, 0, 20, out.ctypes.data_as(C.POINTER(C.c_double))))
+        got[name] = out.ravel()
+
+    first = threading.Thread(target=read, args=("a", ra), daemon=True)
+    first.start()
+    time.sleep(0.3)                       # (it waits for its slot's stream)
+    others = [threading.Thread(target=w, args=(n, rb), daemon=True) for w, n in ((middle, "m"), (read, "b"))]
+    for th in others:
+        th.start()
+        th.join(20)
+        assert not th.is_alive()
+    assert first.is_alive()
+    assert np.array_equal(got["b"], vb) and np.array_equal(got["m"], vb[:got["m"].size])
+    f.fake_block(slot0, 0)
+    first.join(20)
+    assert np.array_equal(got["a"], va)
+    s.close()
+
+
+def scenario_many_threads_read_one_context(f, bs2e):
+    """Reads of several tensors of one context from a thread each arrive whole."""
+    ctx = bs2e.Context(0)
+    rks = [bs2e.RkTensor.build(K, _knots(bs2e, r), K_GL, MAX_K, ctx=ctx) for r in (80.0, 90.0, 60.0, 30.0)]
+    vals = [np.random.default_rng(i).random(rk.device_ptr()[1]) for i, rk in enumerate(rks)]
+    for rk, v in zip(rks, vals):
+        _write(rk, v)
+    bad = []
+
+    def read(rk, v):
+        for _ in range(5):
+            rk.compute()                  # (drops the mirror)
+            if not np.array_equal(rk.to_host().ravel(), v):
+                bad.append(v.size)
+
+    threads = [threading.Thread(target=read, args=p) for p in zip(rks, vals)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+    for rk in rks:
+        rk.release()
+    ctx.close()
+
+
+def scenario_uploads_longer_than_the_ring(f, bs2e):
+    """Containers of more than eight buffers of 8 MiB reach the device byte for byte."""
+    ctx = bs2e.Context(0)
+    k, max_k = 8, 9
+    t = bs2e.generate_grid(k, 3, 2, 0.5, 60.0)
+    spl = bs2e.b_spline(k, t)
+    r_k, r_m_k, r_d_k = (x().init(max_k, spl) for x in (bs2e.sparse_4d, bs2e.sparse_4d, bs2e.sparse_6d))
+    rng = np.random.default_rng(5)
+    for x in (r_k, r_m_k, r_d_k):
+        x.data = np.asfortranarray(rng.random(x.data.shape))
+    r_d_k.i_p = rng.integers(0, 1 << 40, r_d_k.nnz)
+    assert r_d_k.data.nbytes + 40 * r_d_k.nnz > 64 << 20
+    R = bs2e.Nd_DOK()
+    bs2e.compute_R_K_map(r_d_k, r_k, r_m_k, spl, max_k, R, ctx=ctx)
+    for x in (r_k, r_m_k, r_d_k):         # (the blocks are kept, with what was uploaded)
+        flat = x.data.ravel(order="F")
+        assert f.fake_holds(flat.ctypes.data, flat.nbytes)
+    cols = np.concatenate([r_d_k.iv, r_d_k.i, r_d_k.i_p, r_d_k.j, r_d_k.j_p])
+    assert f.fake_holds(cols.ctypes.data, cols.nbytes)
 
 
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
