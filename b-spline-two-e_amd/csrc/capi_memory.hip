@@ -321,27 +321,56 @@ void HostCopier::copy(void* dst, const void* src, size_t bytes)
     wait_slices(&pending);
 }
 
+// Whether the runtime knows the array (pinned, or memory of a device): it
+// copies straight to and from it.
+static bool known_memory(const void* p, size_t bytes)
+{
+    for (const char* at : {(const char*)p, (const char*)p + (bytes - 1)}) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, at) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (a.type == hipMemoryTypeUnregistered) return false;
+    }
+    return true;
+}
+
 hipError_t HostCopier::transfer(const Piece* pieces, size_t n, bool to_host, hipStream_t s)
 {
+    const size_t line = to_host ? kDirectToHost : kDirectToDevice;
     size_t total = 0;
     for (size_t i = 0; i < n; ++i) total += pieces[i].bytes;
-    if (total == 0) return to_host ? hipStreamSynchronize(s) : hipSuccess;
-    if (Ring* r = total > (to_host ? kDirectToHost : kDirectToDevice) ? take() : nullptr) {
-        const bool ready = r->prepare(total);
+    auto direct = [&](const Piece& p) {
+        return hipMemcpyAsync(p.dst, p.src, p.bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
+    };
+    // what takes the ring: of a long transfer, the pageable pieces
+    std::array<Piece, kMaxPieces> ringed;
+    size_t nr = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const Piece& p = pieces[i];
+        if (p.bytes == 0) continue;
+        if (total > line && nr < kMaxPieces && !known_memory(to_host ? p.dst : p.src, p.bytes)) {
+            ringed[nr++] = p;
+        } else {
+            const hipError_t e = direct(p);
+            if (e != hipSuccess) return e;
+        }
+    }
+    if (nr > 0) {
+        Ring* r = take();
+        const bool ready = r && r->prepare(total);
         hipError_t e = hipSuccess;
         if (ready) {
             start_threads(total);
-            e = through(*r, pieces, n, to_host, s);
+            e = through(*r, ringed.data(), nr, to_host, s);
+        } else {
+            for (size_t i = 0; i < nr && e == hipSuccess; ++i) e = direct(ringed[i]);
         }
-        give(r);
-        if (ready) return e;
+        if (r) give(r);
+        if (e != hipSuccess) return e;
+        if (ready && nr == n) return hipSuccess;   // (all in place)
     }
-    for (size_t i = 0; i < n; ++i)
-        if (pieces[i].bytes > 0) {
-            const hipError_t e = hipMemcpyAsync(pieces[i].dst, pieces[i].src, pieces[i].bytes,
-                                                to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, s);
-            if (e != hipSuccess) return e;
-        }
     // (the runtime has read a pageable source when it returns)
     return to_host ? hipStreamSynchronize(s) : hipSuccess;
 }

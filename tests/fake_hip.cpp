@@ -187,6 +187,21 @@ int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)
     return kOk;
 }
 int hipMemcpy(void* d, const void* s, size_t n, int) { return std::memmove(d, s, n), kOk; }
+struct Attributes {
+    int type, device;
+    void *on_device, *on_host;
+    int managed;
+    unsigned flags;
+};
+int hipPointerGetAttributes(Attributes* a, const void* p)
+{
+    std::lock_guard<std::mutex> lk(mu);
+    *a = Attributes{};
+    for (const auto* m : {&blocks, &pinned})
+        for (const auto& b : *m)
+            if (p >= b.first && p < (const char*)b.first + b.second) a->type = m == &pinned ? 1 : 2;
+    return kOk;
+}
 int hipFuncSetAttribute(const void*, int, int) { return kOk; }
 struct dim3v {
     unsigned x, y, z;

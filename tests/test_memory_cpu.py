@@ -213,6 +213,27 @@ def scenario_uploads_longer_than_the_ring(f, bs2e):
     assert f.fake_holds(cols.ctypes.data, cols.nbytes)
 
 
+def scenario_pinned_arrays_are_copied_straight(f, bs2e):
+    """A long result for a pinned array is one copy into it; a pageable one takes the ring and arrives whole."""
+    ctx = bs2e.Context(0)
+    rk = bs2e.RkTensor.build(K, _knots(bs2e, 80.0), K_GL, MAX_K, ctx=ctx)
+    v = np.random.default_rng(3).random(rk.device_ptr()[1])
+    assert v.nbytes > 4 << 20
+    _write(rk, v)
+    P = C.POINTER(C.c_double)
+
+    def copies(address):
+        n = f.fake_memcpys()
+        bs2e.capi.check(bs2e.capi.lib().bs2e_rk_copy_rows(rk.handle, 0, rk.n_pairs, C.cast(address, P)))
+        return f.fake_memcpys() - n
+
+    pinned, page = f.fake_pinned(v.nbytes), np.zeros(v.size)
+    assert copies(pinned) == 1
+    assert copies(page.ctypes.data) > 1
+    got = np.ctypeslib.as_array(C.cast(pinned, P), (v.size,))
+    assert np.array_equal(got, v) and np.array_equal(page, v)
+
+
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
 
 
