@@ -64,7 +64,7 @@ struct Plan {
     std::vector<int32_t> c_first;       // first pair index with column c (1-based c, size n_b+2)
     std::vector<DiagEntry> diag;        // sparse_6d order (built on demand)
     int far_variant = -1;               // rank-one fill shape (index into the far variants; -1: default)
-    int inner_kc = 0;                   // multipoles per diagonal-cell workgroup (0: the largest that fits)
+    int inner_kc = 0;                   // multipoles per diagonal-cell workgroup (0: by the rule of inner_kc_used)
     std::vector<int32_t> rows;          // near-kernel rows: pairs (a, c) with a <= c (built with the tensor)
     int64_t near_elems = -1;            // tensor elements whose pairs share a support interval (-1: not counted)
 };

@@ -798,7 +798,7 @@ int64_t bs2e_rk_autotune(bs2e_rk* rk, int64_t force)
     best = 1e30f;
     int best_kc = 0;
     const int kmax = inner_kc(p.k_s, p.k_gl, p.K);
-    std::vector<int> kcs;
+    std::vector<int> kcs{0};   // what an untuned build takes (inner_kc_used), kept where nothing is faster
     for (int kc : {1, 2, 4, 8, kmax})
         if (kc >= 1 && kc <= kmax && std::find(kcs.begin(), kcs.end(), kc) == kcs.end()) kcs.push_back(kc);
     for (int kc : kcs) {

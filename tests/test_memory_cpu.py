@@ -1,4 +1,4 @@
-"""The library's device blocks and host copies without a device, over a stand-in
+"""The library's device blocks, host copies and tuning without a device, over a stand-in
 for the HIP runtime (fake_hip.cpp): each scenario in a process of its own, as the
 stand-in has to be loaded before the library.
 """
@@ -232,6 +232,21 @@ def scenario_pinned_arrays_are_copied_straight(f, bs2e):
     assert copies(page.ctypes.data) > 1
     got = np.ctypeslib.as_array(C.cast(pinned, P), (v.size,))
     assert np.array_equal(got, v) and np.array_equal(page, v)
+
+
+def scenario_tuning_keeps_the_default(f, bs2e):
+    """Where every candidate takes the same time (as all do here), the autotuner leaves the
+    multipole chunk of an untuned build, also one that is no power of two and not the largest."""
+    ctx = bs2e.Context(0)
+    t = bs2e.generate_grid(6, 3, 2, 1.0, 280.0)
+    rk = bs2e.RkTensor.build(6, t, 8, 16, ctx=ctx, compute=False)
+    untuned = rk.tuning()[1]
+    assert untuned == 12
+    rk.autotune(force=True)
+    assert rk.tuning()[1] == untuned
+    other = bs2e.RkTensor.build(6, t, 8, 16, ctx=ctx, compute=False)
+    other.autotune()                      # (taken from what the process has timed)
+    assert other.tuning()[1] == untuned
 
 
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
