@@ -83,6 +83,7 @@ int64_t bs2e_set_stream(bs2e_ctx* ctx, void* hip_stream)
 {
     if (!ctx) return fail(nullptr, BS2E_EINVAL, "bs2e_set_stream: ctx is NULL");
     ctx->stream = hip_stream ? (hipStream_t)hip_stream : ctx->own;
+    ctx->foreign = ctx->foreign || hip_stream;
     return BS2E_OK;
 }
 
@@ -501,9 +502,10 @@ int64_t bs2e_slater_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const 
     struct Guard {
         bs2e_rk* h;
         std::vector<void*> extra;
+        bool waited = false;
         ~Guard()
         {
-            QuietScope quiet;
+            QuietScope quiet(waited);
             free_tables(h);
             for (void* e : extra) ctx_free(h->ctx, e);
         }
@@ -541,6 +543,7 @@ int64_t bs2e_slater_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const 
                                     {j4, d_i4 + 2 * nnz4, b4}, {rdk, d_rdk, b6 * K}, {iv6, d_i6, b6},
                                     {i6, d_i6 + nnz6, b6}, {ip6, d_i6 + 2 * nnz6, b6}, {j6, d_i6 + 3 * nnz6, b6},
                                     {jp6, d_i6 + 4 * nnz6, b6}}));
+    guard.waited = true;
     return BS2E_OK;
 }
 
@@ -621,12 +624,12 @@ int64_t bs2e_rk_from_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const
     const Plan& p = rk->plan;
     const int64_t K = p.K;
     std::vector<void*> tmp;
-    auto cleanup = [&]() {
-        QuietScope quiet;
+    auto cleanup = [&](bool waited) {
+        QuietScope quiet(waited);
         for (void*& e : tmp) ctx_free(ctx, e);
     };
     auto bail = [&](int64_t code) {
-        cleanup();
+        cleanup(false);
         free_tables(rk);
         rk_delete(rk);
         return code;
@@ -677,7 +680,7 @@ int64_t bs2e_rk_from_primitives(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const
     STEP(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, s));
     STEP(hipStreamSynchronize(s));
 #undef STEP
-    cleanup();
+    cleanup(true);
     if (bad != 0) {
         free_tables(rk);
         rk_delete(rk);

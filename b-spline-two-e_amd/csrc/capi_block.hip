@@ -178,7 +178,7 @@ static void set_drop_graph(bs2e_blockset* b)
 }
 
 // A set's device memory comes from its tensor's context: the context's arena
-// when it has one (a build service's slot), else hipMalloc.
+// when it has one (a build service's slot), else its pool.
 static void set_drop_outputs(bs2e_blockset* b)
 {
     QuietScope quiet;
@@ -197,8 +197,8 @@ static void set_drop_outputs(bs2e_blockset* b)
 
 static void set_free(bs2e_blockset* b)
 {
-    QuietScope quiet;
     bs2e_ctx* c = b->rk->ctx;
+    QuietScope quiet(ctx_waited(c));
     set_drop_outputs(b);
     ctx_free(c, b->d_cfg);
     ctx_free(c, b->d_cfg_chan);
@@ -488,7 +488,10 @@ int64_t bs2e::set_count_finish(bs2e_blockset* b)
     HIP_TRY(ctx, hipEventSynchronize(b->count_ev[2]));
     b->count_pending = false;
     HIP_TRY(ctx, hipEventElapsedTime(&b->ms_count, b->count_ev[0], b->count_ev[1]));
-    ctx_free(ctx, b->d_count_tmp);
+    {
+        QuietScope quiet(true);   // (its last use lies before the event)
+        ctx_free(ctx, b->d_count_tmp);
+    }
     const int64_t N = b->n_rows;
     const int64_t* cnt = (const int64_t*)ctx->pin;
     b->prefH.resize((size_t)N + 1);

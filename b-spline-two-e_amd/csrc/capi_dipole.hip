@@ -34,7 +34,7 @@ struct bs2e_dip {
 
 static void dip_free(bs2e_dip* b)
 {
-    QuietScope quiet;
+    QuietScope quiet(ctx_waited(b->ctx));
     ctx_free(b->ctx, b->d_cfg1);
     ctx_free(b->ctx, b->d_cfg_chan1);
     ctx_free(b->ctx, b->d_chan2);
@@ -124,8 +124,8 @@ int64_t bs2e_setup_radial_dip(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const d
     const size_t tab = (size_t)p.n_iv * p.k_gl * p.k_s;
     DevTables d;
     double *B = nullptr, *B1 = nullptr, *rw = nullptr, *dM1 = nullptr, *dM2 = nullptr;
-    auto cleanup = [&]() {
-        QuietScope quiet;
+    auto cleanup = [&](bool waited) {
+        QuietScope quiet(waited);
         ctx_free(ctx, d.t);
         ctx_free(ctx, d.bp);
         ctx_free(ctx, d.x);
@@ -156,7 +156,7 @@ int64_t bs2e_setup_radial_dip(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const d
         return BS2E_OK;
     };
     const int64_t rc = run();
-    cleanup();
+    cleanup(rc == BS2E_OK);   // (its results are on the host)
     return rc;
 }
 
@@ -287,8 +287,8 @@ int64_t bs2e_dip_block_fill(bs2e_dip* b, int64_t gauge, const double* S, const d
     const size_t nn = (size_t)b->n_b * b->n_b;
     double *dS = nullptr, *dR1 = nullptr, *dR2 = nullptr, *dd = nullptr, *dT = nullptr;
     int64_t* dix = nullptr;
-    auto cleanup = [&]() {
-        QuietScope quiet;
+    auto cleanup = [&](bool waited) {
+        QuietScope quiet(waited);
         ctx_free(ctx, dT);
         ctx_free(ctx, dS);
         ctx_free(ctx, dR1);
@@ -334,7 +334,7 @@ int64_t bs2e_dip_block_fill(bs2e_dip* b, int64_t gauge, const double* S, const d
         return BS2E_OK;
     };
     const int64_t rc = run();
-    cleanup();
+    cleanup(rc == BS2E_OK);   // (its results are on the host)
     return rc;
 }
 

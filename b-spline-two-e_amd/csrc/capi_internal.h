@@ -63,23 +63,30 @@ private:
         void* ptr;
         uint64_t stamp;
     };
-    static constexpr size_t kMaxKept = (size_t)4 << 30, kMaxBlocks = 256;
+    bool wait_idle();
+    static constexpr size_t kMaxKept = (size_t)4 << 30, kMaxBlocks = 256, kToken = 256;
     std::mutex mu_;
     std::map<void*, size_t> live_;
     std::multimap<size_t, Kept> kept_;   // by size
     size_t kept_bytes_ = 0;
     uint64_t stamp_ = 0;
+    void* token_ = nullptr;              // a block to free (wait_idle)
 };
 
 // hipMalloc on `device` (the current one); a failure for want of memory takes
 // what the device's pools keep and is tried once more.
 hipError_t device_malloc(int device, void** out, size_t bytes);
 
-// Releases of the calling thread inside one scope wait for the device once.
+// Releases of the calling thread inside one scope wait for the device once; not
+// at all where the caller has `waited` for every use of what it releases
+// (temporaries of a call that has waited for its stream; a wait costs 20 to 40 us).
 struct QuietScope {
-    QuietScope();
+    explicit QuietScope(bool waited = false);
     ~QuietScope();
     QuietScope(const QuietScope&) = delete;
+
+private:
+    const bool waited_, outer_;
 };
 
 // One part of a copy between device memory and a caller's array.
@@ -163,6 +170,7 @@ struct bs2e_ctx {
     bs2e::Arena* arena = nullptr;   // when set, the tensors of this context live in it
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;   // the build's stream (own, or the caller's)
+    bool foreign = false;           // has run on a caller's stream
     hipStream_t side = nullptr;     // diagonal cells + near ranges, concurrent with the rank-one fill
     std::string err;
     bs2e::DevicePool pool;          // the context's device blocks (without an arena)
@@ -252,6 +260,9 @@ inline void ctx_free(bs2e_ctx* c, T*& p)
 // copy_to_host returns when they are done.
 hipError_t copy_to_host(bs2e_ctx* c, std::initializer_list<Piece> pieces);
 hipError_t copy_to_device(bs2e_ctx* c, std::initializer_list<Piece> pieces);
+// Waits for the context's stream; whether that covers every use of blocks that
+// only this stream's work reaches (not a tensor's, which callers read too).
+bool ctx_waited(bs2e_ctx* c);
 HostCopier* ctx_copier(bs2e_ctx* c);   // nullptr: no memory for one
 
 // Device bytes a tensor build of this plan allocates (tables and tensor,

@@ -14,13 +14,18 @@ namespace bs2e {
 // ---------------------------------------------------------------------------
 namespace {
 thread_local int t_quiet_depth = 0;
-thread_local bool t_quiet = false;   // the device was idle since the outermost scope began
+thread_local bool t_quiet = false;   // nothing uses what this scope releases any more
 }  // namespace
 
-QuietScope::QuietScope() { ++t_quiet_depth; }
+QuietScope::QuietScope(bool waited) : waited_(waited), outer_(t_quiet)
+{
+    ++t_quiet_depth;
+    if (waited) t_quiet = true;
+}
 QuietScope::~QuietScope()
 {
     if (--t_quiet_depth == 0) t_quiet = false;
+    else if (waited_) t_quiet = outer_;   // (said of this scope's blocks only)
 }
 
 namespace {
@@ -38,6 +43,7 @@ DevicePool::DevicePool()
 
 DevicePool::~DevicePool()
 {
+    if (token_) (void)hipFree(token_);
     std::lock_guard<std::mutex> lk(g_pools_mu);
     (prev_ ? prev_->next_ : g_pools) = next_;
     if (next_) next_->prev_ = prev_;
@@ -88,6 +94,10 @@ hipError_t DevicePool::alloc(void** out, size_t bytes)
     }
     try {
         std::lock_guard<std::mutex> lk(mu_);
+        if (!token_ && hipMalloc(&token_, kToken) != hipSuccess) {
+            (void)hipGetLastError();
+            token_ = nullptr;
+        }
         live_.emplace(*out, need);
     } catch (...) {
         (void)hipFree(*out);
@@ -97,6 +107,28 @@ hipError_t DevicePool::alloc(void** out, size_t bytes)
     return hipSuccess;
 }
 
+// Waits for the device by hipFree of a block held for that.  (Waiting for the
+// device as such ends every stream capture under way in the process, other
+// threads' and relaxed ones among them; hipFree does not.)
+bool DevicePool::wait_idle()
+{
+    void* t;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        t = token_;
+        token_ = nullptr;
+    }
+    if (!t) return false;
+    const bool idle = hipFree(t) == hipSuccess;
+    if (idle && hipMalloc(&t, kToken) != hipSuccess) {   // (the next allocation tries again)
+        (void)hipGetLastError();
+        t = nullptr;
+    }
+    std::lock_guard<std::mutex> lk(mu_);
+    if (t && !token_) token_ = t;
+    return idle;
+}
+
 void DevicePool::release(void* p)
 {
     if (!p) return;
@@ -104,10 +136,7 @@ void DevicePool::release(void* p)
     // caller's own among them, may still read the block.
     (void)hipSetDevice(device);
     bool idle = t_quiet;
-    if (!idle) {
-        idle = hipDeviceSynchronize() == hipSuccess;
-        if (t_quiet_depth > 0) t_quiet = idle;
-    }
+    if (!idle) idle = wait_idle();
     size_t size = 0;
     {
         std::lock_guard<std::mutex> lk(mu_);
@@ -125,7 +154,8 @@ void DevicePool::release(void* p)
             }
         }
     }
-    if (p) (void)hipFree(p);
+    if (p && hipFree(p) == hipSuccess) idle = true;
+    if (t_quiet_depth > 0) t_quiet = idle;
     trim(kMaxKept);
 }
 
@@ -443,6 +473,11 @@ hipError_t HostCopier::through(Ring& r, const Piece* pieces, size_t n, bool to_h
     if (to_host)
         for (int b = 0; b < kBufs; ++b) wait_slices(&r.pending[b]);
     return e;
+}
+
+bool ctx_waited(bs2e_ctx* c)
+{
+    return !c->arena && !c->foreign && hipStreamSynchronize(c->stream) == hipSuccess;
 }
 
 HostCopier* ctx_copier(bs2e_ctx* c)

@@ -26,8 +26,8 @@ static int64_t one_body(bs2e_ctx* ctx, const char* who, int64_t k, int64_t n_kno
     const size_t tab = (size_t)p.n_iv * p.k_gl * p.k_s;
     DevTables d;
     double *B = nullptr, *B2 = nullptr, *rw = nullptr, *dS = nullptr, *dH = nullptr;
-    auto cleanup = [&]() {
-        QuietScope quiet;
+    auto cleanup = [&](bool waited) {
+        QuietScope quiet(waited);
         ctx_free(ctx, d.t);
         ctx_free(ctx, d.bp);
         ctx_free(ctx, d.x);
@@ -61,7 +61,7 @@ static int64_t one_body(bs2e_ctx* ctx, const char* who, int64_t k, int64_t n_kno
         return BS2E_OK;
     };
     const int64_t rc = run();
-    cleanup();
+    cleanup(rc == BS2E_OK);   // (its results are on the host)
     return rc;
 }
 
@@ -82,8 +82,8 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
     const size_t tab = (size_t)p.n_iv * p.k_gl * p.k_s;
     DevTables d;
     double *B = nullptr, *rw = nullptr, *dout = nullptr;
-    auto cleanup = [&]() {
-        QuietScope quiet;
+    auto cleanup = [&](bool waited) {
+        QuietScope quiet(waited);
         ctx_free(ctx, d.t);
         ctx_free(ctx, d.bp);
         ctx_free(ctx, d.x);
@@ -110,7 +110,7 @@ static int64_t rk_int(bs2e_ctx* ctx, int64_t k, int64_t n_knots, const double* k
         return BS2E_OK;
     };
     const int64_t rc = run();
-    cleanup();
+    cleanup(rc == BS2E_OK);   // (its results are on the host)
     return rc;
 }
 

@@ -36,7 +36,8 @@ struct Own {
     ~Own() { fail_new_after = keep; }
 };
 
-constexpr int kOk = 0, kInvalid = 1, kNoMemory = 2, kNotReady = 600;
+constexpr int kOk = 0, kInvalid = 1, kNoMemory = 2, kNotReady = 600, kCaptureUnsupported = 900;
+bool capturing = false, captures_ended = false;   // a stream capture under way elsewhere, and whether a call ended it
 
 bool lives(Stream* s)
 {
@@ -48,6 +49,16 @@ int wait_for(Stream* s)
 {
     std::unique_lock<std::mutex> lk(mu);
     cv.wait(lk, [s] { return !s || !lives(s) || !s->blocked; });
+    return kOk;
+}
+int wait_for_all()
+{
+    std::unique_lock<std::mutex> lk(mu);
+    cv.wait(lk, [] {
+        for (Stream* s : streams)
+            if (s->blocked) return false;
+        return true;
+    });
     return kOk;
 }
 }  // namespace
@@ -79,6 +90,8 @@ void fake_block(void* s, int on)
     }
     cv.notify_all();
 }
+void fake_capture(int on) { capturing = on != 0; }
+int fake_captures_ended() { return captures_ended; }
 // whether a device block starts with these bytes
 int fake_holds(const void* p, size_t n)
 {
@@ -104,13 +117,8 @@ int hipGetLastError() { return kOk; }
 const char* hipGetErrorString(int e) { return e == kNoMemory ? "out of memory" : "error"; }
 int hipDeviceSynchronize()
 {
-    std::unique_lock<std::mutex> lk(mu);
-    cv.wait(lk, [] {
-        for (Stream* s : streams)
-            if (s->blocked) return false;
-        return true;
-    });
-    return kOk;
+    if (capturing) return captures_ended = true, kCaptureUnsupported;
+    return wait_for_all();
 }
 int hipMalloc(void** p, size_t n)
 {
@@ -127,6 +135,7 @@ int hipMalloc(void** p, size_t n)
 }
 int hipFree(void* p)
 {
+    wait_for_all();
     std::lock_guard<std::mutex> lk(mu);
     auto it = blocks.find(p);
     if (it == blocks.end()) return kInvalid;

@@ -33,6 +33,7 @@ def _load(so):
                             ("fake_mallocs", C.c_int64, []), ("fake_memcpys", C.c_int64, []),
                             ("fake_fail_new", None, [C.c_int]), ("fake_stream", C.c_void_p, [C.c_int]),
                             ("fake_block", None, [C.c_void_p, C.c_int]), ("fake_pinned", C.c_void_p, [C.c_size_t]),
+                            ("fake_capture", None, [C.c_int]), ("fake_captures_ended", C.c_int, []),
                             ("fake_holds", C.c_int, [C.c_void_p, C.c_size_t])):
         getattr(f, name).restype = res
         getattr(f, name).argtypes = args
@@ -247,6 +248,35 @@ def scenario_tuning_keeps_the_default(f, bs2e):
     other = bs2e.RkTensor.build(6, t, 8, 16, ctx=ctx, compute=False)
     other.autotune()                      # (taken from what the process has timed)
     assert other.tuning()[1] == untuned
+
+
+def scenario_releases_spare_captures(f, bs2e):
+    """Handles made and released, and the calls that do so inside, leave stream captures of the
+    process alone; the device is waited for all the same before a block is taken again."""
+    ctx = bs2e.Context(0)
+    t = _knots(bs2e, 40.0)
+    spl = bs2e.b_spline(K, t)
+    f.fake_capture(1)
+    rk = bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=ctx)
+    rk.to_host()
+    rk.release()
+    kept = f.fake_mallocs()
+    bs2e.setup_S(spl, K_GL, ctx=ctx)
+    bs2e.setup_H_one_particle(2, (2, 10.0, 0.0), range(3), spl, K_GL, ctx=ctx)
+    rk = bs2e.RkTensor.build(K, t, K_GL, MAX_K, ctx=ctx)
+    assert not f.fake_captures_ended()
+    f.fake_capture(0)
+    other = f.fake_stream(1)                     # (not the stream that the context builds on)
+    f.fake_block(other, 1)
+    th = threading.Thread(target=rk.release, daemon=True)
+    th.start()
+    th.join(0.5)
+    assert th.is_alive()
+    f.fake_block(other, 0)
+    th.join(20)
+    assert not th.is_alive() and f.fake_mallocs() < kept + 20
+    ctx.close()
+    assert f.fake_used() == 0
 
 
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
