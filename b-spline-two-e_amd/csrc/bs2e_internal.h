@@ -268,11 +268,10 @@ int far_variant_count();
 // Zeros over n16 16-byte elements at dst, one store per thread (the store
 // ceiling the rank-one fill is measured against).
 hipError_t launch_store_fill(void* dst, int64_t n16, bool nt, hipStream_t s);
-bool far_variant_valid(const Plan& p, int v);      // 16-byte variants need rows of even length
+bool far_variant_valid(const Plan& p, int v);      // unshifted rows need an even length
 int far_variant_default(const Plan& p);
 // overlapping pairs (symmetric: the moments of (a, c) and (c, a) are the same numbers)
 hipError_t launch_tensor_near(const Plan& p, const DevTables& d, double* R, bool symmetric, hipStream_t s);
-size_t outer_lds_bytes(int64_t ks, int64_t kgl, int64_t K);
 size_t inner_lds_bytes(int64_t ks, int64_t kgl, int64_t kc);
 int inner_kc(int64_t ks, int64_t kgl, int64_t K);   // largest multipole chunk of a diagonal-cell workgroup (0: unsupported)
 int inner_kc_used(const Plan& p);                   // the chunk the next build takes

@@ -371,7 +371,7 @@ static int64_t alloc_tables(bs2e_ctx* ctx, bs2e_rk* rk, bool with_tensor)
 int64_t bs2e::check_plan_limits(bs2e_ctx* ctx, const Plan& p, bool needs_primitives)
 {
     if (needs_primitives &&
-        (p.k_s > 16 || inner_kc(p.k_s, p.k_gl, p.K) == 0 || outer_lds_bytes(p.k_s, p.k_gl, p.K) > kLdsPerWorkgroup))
+        (p.k_s > 16 || inner_kc(p.k_s, p.k_gl, p.K) == 0))
         return fail(ctx, BS2E_EINVAL,
                     "the per-interval primitive kernels support spline orders <= 16 whose tables fit 160 KiB of LDS "
                     "(about k_GL^2 * k + k_GL * k^2 doubles; e.g. k = 16 with k_GL <= 26)");

@@ -43,14 +43,12 @@ hipError_t allow_lds(const void* fn, size_t bytes)
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-size_t outer_lds_bytes(int64_t ks, int64_t kgl, int64_t K)
-{
-    return sizeof(double) * (size_t)(kgl * ks + kgl + 2 * kgl * K);
-}
-
-// The multipoles that one diagonal-cell workgroup may be given (what a caller
-// can pin): 16, up to order 9 and 16 GL points as many as tables of all of
-// them in LDS would allow, 4 elsewhere.
+// Which bases are accepted and which multipole chunks a caller can pin, as
+// earlier layouts of the diagonal cells in LDS allowed: tables of every multipole
+// of a chunk, at most 16 of them up to order 9 and 16 GL points, 4 elsewhere.
+// The kernels' own tables (diag_lds_bytes, window_lds_bytes of window_shape) fit
+// for every order, GL order and multipole count that this lets through; it stays
+// as the line because callers meet it as a refusal.
 size_t inner_lds_bytes(int64_t ks, int64_t kgl, int64_t kc)
 {
     const int64_t U = ks * (ks + 1) / 2;

@@ -385,7 +385,9 @@ int64_t bs2e_dip_block_release(bs2e_dip *d);
  * order, smaller jobs passing one that does not fit yet), so builds of
  * several jobs overlap on the device.  Each job's tensor is computed by the
  * same kernels as bs2e_rk_compute, so its values do not depend on what else
- * runs.  Calls on one service must come from one thread at a time. */
+ * runs.  Calls on one service must come from one thread at a time; the results
+ * of different slots' jobs may be read by a thread each, with up to 64 MiB of
+ * pinned host memory for each such read and the copy threads shared. */
 typedef struct bs2e_server bs2e_server;
 int64_t bs2e_server_create(int64_t device, int64_t hbm_bytes, int64_t slots, bs2e_server **out);
 int64_t bs2e_server_destroy(bs2e_server *srv);
