@@ -170,7 +170,7 @@ private:
 
 struct bs2e_ctx {
     int device = 0;
-    int refs = 0;                   // live tensor handles created on this context
+    std::atomic<int> refs{0};       // live tensor handles created on this context
     bool closing = false;           // bs2e_destroy was called; freed with the last tensor
     bs2e::Arena* arena = nullptr;   // when set, the tensors of this context live in it
     hipStream_t own = nullptr;

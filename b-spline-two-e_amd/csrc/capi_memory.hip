@@ -124,8 +124,11 @@ bool DevicePool::wait_idle()
         (void)hipGetLastError();
         t = nullptr;
     }
-    std::lock_guard<std::mutex> lk(mu_);
-    if (t && !token_) token_ = t;
+    if (t) {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (!token_) std::swap(t, token_);
+    }
+    if (t) (void)hipFree(t);   // (an allocation of another thread has made one meanwhile)
     return idle;
 }
 

@@ -279,6 +279,24 @@ def scenario_releases_spare_captures(f, bs2e):
     assert f.fake_used() == 0
 
 
+def scenario_threads_share_a_context(f, bs2e):
+    """Handles made and released by several threads on one context leave nothing behind."""
+    ctx = bs2e.Context(0)
+
+    def work(i):
+        for j in range(60):
+            rk = bs2e.RkTensor.build(K, _knots(bs2e, 8.0 + i + j % 7), K_GL, MAX_K, ctx=ctx, compute=False)
+            rk.release()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    ctx.close()
+    assert f.fake_used() == 0
+
+
 SCENARIOS = [n[len("scenario_"):] for n in list(globals()) if n.startswith("scenario_")]
 
 
